@@ -15,12 +15,13 @@
 // solved by right-preconditioned BiCGStab (:959-1151); the reference's
 // preconditioner is a symmetric Gauss-Seidel sweep, which is sequential over
 // all unknowns, so here each colatitude ring is solved exactly instead (a
-// periodic tridiagonal solve of the ring's longitude coupling, one thread per
-// ring). Dot products are two-pass block reductions in a fixed order; the
-// iterates therefore differ from the reference's by rounding, and the
-// converged potential agrees with it to the solve's tolerance. Both
-// hemispheres run in the same launches (blockIdx.y).
-#include <hip/hip_cooperative_groups.h>
+// periodic tridiagonal solve of the ring's longitude coupling). Dot products
+// are reductions in a fixed order; the iterates therefore differ from the
+// reference's by rounding, and the converged potential agrees with it to the
+// solve's tolerance. Both hemispheres run in the same launches. The solves
+// keep their vectors in registers, one wavefront per ring (k_ring_cg,
+// k_ring_bicgstab); where their workgroups cannot all be resident, one
+// workgroup per hemisphere solves instead (k_mi_cg, k_mi_bicgstab).
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
@@ -91,8 +92,10 @@ struct MiState {
   // potential plus the network's answer for the current residual
   unet::Net *net = nullptr;
   double *warm_scale = nullptr;  // [2] residual-current RMS, [2] step lengths
-  double *coop_slots = nullptr;  // partial sums of the cooperative solve
-  int *coop_flags = nullptr;     // its per-hemisphere liveness exchange
+  // exchange buffers of the register-resident solve (null: one workgroup
+  // per hemisphere solves instead) and its workgroups per hemisphere
+  unsigned long long *ring_words = nullptr;
+  int ring_groups = 0;
 };
 
 namespace {
@@ -333,9 +336,14 @@ GCS_DEV TensorRow tensor_row(double sp, double hall, int i, double dt, double dp
 // Right-hand side (:428-448, weighted by sin theta), initial guess from the
 // previous potential (:449-464), and the diagonal (Pedersen, :322-344) or the
 // five-point tensor stencil (:777-833).
-__global__ void k_mi_setup(MiK c, int tensor, double hall) {
+// The exchange words of the register-resident solve are cleared here too.
+__global__ void k_mi_setup(MiK c, int tensor, double hall, unsigned long long *words,
+                           long n_words) {
   const int h = blockIdx.y;
   const long q = gtid();
+  for (long t = q + h * (long)gridDim.x * blockDim.x; t < n_words;
+       t += 2L * gridDim.x * blockDim.x)
+    words[t] = 0ull;
   if (q >= c.n) return;
   const int np = c.np;
   const double dt = c.max_colat / (double)(c.nt - 1);
@@ -497,6 +505,10 @@ MiK make_mik(Problem &P) {
 }
 
 // ---- fused solves: one workgroup per hemisphere runs the whole Krylov loop -------
+//
+// The solves of devices or grids that cannot hold the register-resident
+// kernels' workgroups at once (more than 768 rings on 256 compute units), or
+// with GCS_MI_COOPERATIVE=0.
 //
 // The same iterations as the reference's solvers (CG: :516-600, BiCGStab:
 // :1029-1131, with the ring preconditioner above), but every scalar stays on
@@ -938,216 +950,797 @@ __global__ void __launch_bounds__(kSolveThreads) k_mi_bicgstab(MiK c, double rel
   store_result(c, h, res, first);
 }
 
-// Cooperative BiCGStab: each hemisphere's solve spread over kCoopBlocks
-// workgroups (the same iterations as k_mi_bicgstab, with grid-wide barriers
-// where one workgroup's barrier sufficed there). Dot products sum the
-// workgroups' partial sums in workgroup order from two alternating slot
-// banks (a bank is rewritten only after every workgroup passed the barrier
-// that follows its last read), so every workgroup of a hemisphere computes
-// the same sums and takes the same branches.
-constexpr int kCoopBlocks = 16;
+// ---- register-resident solves: one wavefront per colatitude ring ------------------
+//
+// The iterations of k_mi_cg and k_mi_bicgstab with every solver vector held
+// in registers: a wavefront owns one ring, a lane kRingPoints = ceil(np / 64)
+// consecutive points of it, and a workgroup kRingOwn rings plus a ghost copy
+// of the ring on each side. Neighbour rings inside a workgroup meet in LDS.
+// A ghost wavefront runs the same vector updates as the ring's owner (so its
+// values are the owner's, bit for bit) and receives from it only the product
+// A p that it cannot form itself. Workgroups exchange two things, both as
+// self-validating words (32 bits of a double and a 32-bit sequence number
+// in one 64-bit atomic): the partial sums of the dot products, and those
+// boundary rings, which are sent before a reduction and read after it, so
+// that their way is hidden behind the reduction's. A reduction is therefore
+// the only wait: one per CG iteration, two per BiCGStab iteration, where a
+// grid barrier per dot product and per vector took ten. What bounds an
+// iteration is the latency of these reductions and of the ring solve's two
+// wavefront-wide prefixes; nothing in it is limited by bandwidth or issue.
+// Measured on 2 x 128 x 256 points: BiCGStab 9.4 us an iteration and 4.6 ms a
+// solve (two grid barriers of cooperative groups per step of the method, all
+// vectors in memory: 115 us, 48 ms), CG 4.0 us and 4.0 ms (one workgroup per
+// hemisphere: 88 us, 83 ms); on 2 x 33 x 57, 7.5 us and 0.9 ms (75 us, 8.9
+// ms). Putting a hemisphere's workgroups on one XCD changed nothing (3 %).
+//
+// The hemispheres are independent groups of workgroups. Every workgroup of a
+// hemisphere sums the same words in the same order and so takes the same
+// branches. All workgroups must be resident (a cooperative launch); a wait
+// ends after kSpinLimit polls at the latest, and a workgroup that gave up
+// leaves with the solve marked as failed, after which its neighbours' waits
+// end the same way.
 
-// Both hemispheres in one cooperative launch: workgroups [0, kCoopBlocks)
-// solve the north, [kCoopBlocks, 2 kCoopBlocks) the south, concurrently. The
-// grid barriers are shared, so every workgroup must pass the same sequence
-// of barriers whatever its hemisphere does: each iteration runs a fixed
-// schedule of ten barrier-carrying steps, and a hemisphere that has
-// converged, broken down or needs no true-residual check this iteration
-// skips the work of a step but not its barrier. No branch contains a
-// barrier, the loop bound and its exit test are grid-uniform (the exit reads
-// both hemispheres' flags after a barrier), so every workgroup leaves after
-// the same number of barriers, at the latest after maximum_iterations.
-// Per hemisphere the arithmetic is k_mi_bicgstab's.
-__global__ void __launch_bounds__(kSolveThreads) k_mi_bicgstab_pair(MiK c, double rel_tol,
-                                                                    int maxit, double *slots,
-                                                                    int *flags) {
-  namespace cg = cooperative_groups;
-  cg::grid_group grid = cg::this_grid();
-  __shared__ double red[kSolveThreads / 64];
-  const int h = blockIdx.x / kCoopBlocks, lb = blockIdx.x % kCoopBlocks;
-  const long n = c.n;
-  const long t0 = lb * (long)blockDim.x + threadIdx.x;
-  const long st = (long)kCoopBlocks * blockDim.x;
-  const bool pole_wave = lb == 0 && threadIdx.x < 64;
-  int bank = 0;
-  // sums of up to two values over this hemisphere's workgroups
-  auto gsum2 = [&](double v, double w, double &sv, double &sw) {
-    const double bv = block_sum(v, red);
-    const double bw = block_sum(w, red);
-    double *sl = slots + bank * (4 * kCoopBlocks) + h * (2 * kCoopBlocks);
-    if (threadIdx.x == 0) {
-      sl[lb] = bv;
-      sl[kCoopBlocks + lb] = bw;
-    }
-    bank ^= 1;
-    grid.sync();
-    sv = 0.0;
-    sw = 0.0;
-    for (int i = 0; i < kCoopBlocks; ++i) {
-      sv += sl[i];
-      sw += sl[kCoopBlocks + i];
-    }
-  };
-  auto gsum = [&](double v) {
-    double sv, sw;
-    gsum2(v, 0.0, sv, sw);
-    return sv;
-  };
-  const double dt = c.max_colat / (double)(c.nt - 1);
-  const double half = 0.5 * dt;
-  const double pe = sin(half) * c.pedersen / (incl2(half) * dt * dt);
-  const double ps = (double)c.np * pe;
-  double *x = c.vec(h, V_X), *r = c.vec(h, V_R), *p = c.vec(h, V_P), *ap = c.vec(h, V_AP),
-         *sh = c.vec(h, V_SH), *pp = c.vec(h, V_PP), *s = c.vec(h, V_S), *psv = c.vec(h, V_PS),
-         *as = c.vec(h, V_AS);
-  const double *rhs = c.vec(h, V_RHS);
-  const int lane = threadIdx.x & 63;
-  auto precondition = [&](bool work, const double *in, double *out) {
-    grid.sync();  // `in` complete
-    if (work) {
-      if (t0 == 0) out[0] = in[0] / c.vec(h, V_DIAG)[0];
-      for (long ring = t0 >> 6; ring < c.nt - 2; ring += st >> 6)
-        ring_apply(c, h, in, out, (int)ring, lane);
-    }
-    grid.sync();  // `out` complete
-  };
-  for (long ring = t0; ring < c.nt - 2; ring += st) ring_factor(c, h, (int)ring);
-  double a = 0.0, b = 0.0;
-  {
-    const double pole = pole_wave ? pole_row(c, h, true, x, pe) : 0.0;
-    for (long q = t0; q < n; q += st) {
-      r[q] = rhs[q] - (q == 0 ? pole : apply_at(c, h, true, x, q, nullptr, pe));
-      sh[q] = r[q];
-      p[q] = 0.0;
-      ap[q] = 0.0;
-      a += orig_term(c, r[q], q, ps, dt);
-      b += q == 0 ? 0.0 : orig_term(c, rhs[q], q, ps, dt);
+typedef unsigned long long ll_word;
+
+constexpr int kRingWaves = 8;
+constexpr int kRingOwn = kRingWaves - 2;
+constexpr int kRingThreads = 64 * kRingWaves;
+constexpr int kRingSums = 7;         // most values of one reduction
+constexpr int kSpinLimit = 1 << 20;  // polls of a wait, about a second
+
+// Device buffers of the exchange, zeroed before each solve (the sequence
+// numbers of a solve start at 1): red [2 banks][2 hemispheres][groups]
+// [kRingSums][2 words], halo [2 banks][2 hemispheres][groups][2 sides]
+// [points][2 halves][64 lanes]. A bank is used again two messages later; by
+// then a reduction has passed, which its reader entered after reading it.
+struct RingComm {
+  ll_word *red, *halo;
+  int groups, points;
+  static size_t red_words(int groups) { return 2UL * 2 * groups * kRingSums * 2; }
+  static size_t halo_words(int groups, int points) {
+    return 2UL * 2 * groups * 2 * points * 2 * 64;
+  }
+};
+
+GCS_DEV void ll_put(ll_word *hi, ll_word *lo, double v, unsigned seq) {
+  const ll_word b = (ll_word)__double_as_longlong(v);
+  __hip_atomic_store(hi, (b & 0xffffffff00000000ull) | seq, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(lo, (b << 32) | seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+GCS_DEV ll_word ll_load(const ll_word *w) {
+  return __hip_atomic_load(const_cast<ll_word *>(w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+GCS_DEV double ll_value(ll_word hi, ll_word lo) {
+  return __longlong_as_double((long long)((hi & 0xffffffff00000000ull) | (lo >> 32)));
+}
+
+// Lane moves by DPP (a few cycles; a shuffle through LDS takes over a hundred):
+// v of the lane the control names, `old` where there is none.
+enum Dpp {
+  DPP_ROW_SHL = 0x100, DPP_ROW_SHR = 0x110,  // + n: within rows of 16 lanes
+  DPP_WAVE_SHL1 = 0x130, DPP_WAVE_SHR1 = 0x138, DPP_BCAST15 = 0x142, DPP_BCAST31 = 0x143
+};
+template <int Ctrl, int RowMask = 0xf>
+GCS_DEV double dpp_move(double old, double v) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), Ctrl,
+                                             RowMask, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), Ctrl,
+                                             RowMask, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+GCS_DEV double read_lane(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// Sum over the wavefront, in every lane.
+GCS_DEV double wave_sum(double v) {
+  v += dpp_move<DPP_ROW_SHR + 1>(0.0, v);
+  v += dpp_move<DPP_ROW_SHR + 2>(0.0, v);
+  v += dpp_move<DPP_ROW_SHR + 4>(0.0, v);
+  v += dpp_move<DPP_ROW_SHR + 8>(0.0, v);
+  v += dpp_move<DPP_BCAST15, 0xa>(0.0, v);
+  v += dpp_move<DPP_BCAST31, 0xc>(0.0, v);
+  return read_lane(v, 63);
+}
+
+// One step of a prefix (N lanes to the left) or suffix of affine maps
+// x -> a + b x; a lane without such a neighbour composes with the identity.
+template <int Ctrl>
+GCS_DEV void affine_step(double &a, double &b) {
+  const double ao = dpp_move<Ctrl>(0.0, a), bo = dpp_move<Ctrl>(1.0, b);
+  a = a + b * ao;
+  b = b * bo;
+}
+
+// What a wavefront knows of its place in the solve.
+template <int KP>
+struct RingWave {
+  int h, g, groups;      // hemisphere, workgroup of it, workgroups of it
+  int w, lane, nown;     // wavefront, lane, rings this workgroup owns
+  int ring;              // colatitude index of the wavefront's ring
+  bool own, ghost;       // owner or ghost copy of `ring` (neither: idle)
+  int j0, cnt;           // this lane's points j0 .. j0 + cnt - 1
+  int last_lane, last_t; // where the ring's last point is
+  unsigned seq, hseq;    // sequence numbers of the last reduction and message
+  bool dead;             // a wait was given up
+  RingComm comm;
+  double (*rows)[64 * KP];         // LDS [kRingWaves][points, t-major]
+  double (*part)[kRingWaves];      // LDS [kRingSums][kRingWaves]
+  double *total;                   // LDS [kRingSums + 1]
+  int *gave_up;                    // LDS
+
+  GCS_DEV void init(const MiK &c, const RingComm &cm, double (*r)[64 * KP],
+                    double (*p)[kRingWaves], double *t, int *gu) {
+    comm = cm;
+    groups = cm.groups;
+    h = blockIdx.x / groups;
+    g = blockIdx.x % groups;
+    w = threadIdx.x >> 6;
+    lane = threadIdx.x & 63;
+    nown = min(kRingOwn, c.nt - 2 - g * kRingOwn);
+    ring = g * kRingOwn + w;
+    own = w >= 1 && w <= nown;
+    ghost = (w == 0 && g > 0) || (w == nown + 1 && ring <= c.nt - 2);
+    j0 = min(c.np, lane * KP);
+    cnt = min(c.np, j0 + KP) - j0;
+    last_lane = (c.np - 1) / KP;
+    last_t = (c.np - 1) - last_lane * KP;
+    seq = hseq = 0;
+    dead = false;
+    rows = r;
+    part = p;
+    total = t;
+    gave_up = gu;
+    if (threadIdx.x == 0) *gave_up = 0;
+    __syncthreads();
+  }
+
+  GCS_DEV ll_word *halo_slot(int group, int side) const {
+    return comm.halo + ((((hseq & 1) * 2 + h) * (long)groups + group) * 2 + side) *
+                           (KP * 2 * 64);
+  }
+
+  // Start sending the boundary rings of v to the neighbour workgroups.
+  GCS_DEV void send(const double v[KP]) {
+    ++hseq;
+    for (int side = 0; side < 2; ++side) {
+      // side 0: my first ring is the upper ghost of workgroup g - 1
+      const bool mine = own && (side == 0 ? w == 1 && g > 0 : w == nown && g + 1 < groups);
+      if (!mine) continue;
+      ll_word *s = halo_slot(side == 0 ? g - 1 : g + 1, side == 0 ? 1 : 0);
+#pragma unroll
+      for (int t = 0; t < KP; ++t)
+        if (t < cnt) ll_put(s + (2 * t) * 64 + lane, s + (2 * t + 1) * 64 + lane, v[t], hseq);
     }
   }
-  double n0, b0;
-  gsum2(a, b, n0, b0);  // also orders the ring factors before their first use
-  double norm = sqrt(fmax(0.0, n0));
-  const double first = norm;
-  const double target = rel_tol * fmax(sqrt(fmax(0.0, b0)), 1.0);
-  SolveResult res{0, norm <= target, norm};
-  bool live = !res.ok;  // this hemisphere still iterates
-  double rho_prev = 1.0, alpha = 1.0, omega = 1.0;
-  bool other_live = true;
-  for (int it = 1; it <= maxit && (live || other_live); ++it) {
-    // 1: rho
-    a = 0.0;
-    if (live)
-      for (long q = t0; q < n; q += st) a += sh[q] * r[q];
-    const double rho = gsum(a);
-    if (live && (!isfinite(rho) || fabs(rho) <= DBL_MIN || !isfinite(omega) ||
-                 fabs(omega) <= DBL_MIN))
-      live = false;
-    // 2, 3: p and its preconditioned image
-    if (live) {
-      const double beta = (rho / rho_prev) * (alpha / omega);
-      for (long q = t0; q < n; q += st) p[q] = r[q] + beta * (p[q] - omega * ap[q]);
-    }
-    precondition(live, p, pp);
-    // 4: A pp and den
-    a = 0.0;
-    {
-      const double pole = (live && pole_wave) ? pole_row(c, h, true, pp, pe) : 0.0;
-      if (live)
-        for (long q = t0; q < n; q += st) {
-          ap[q] = q == 0 ? pole : apply_at(c, h, true, pp, q, nullptr, pe);
-          a += sh[q] * ap[q];
+
+  // Ghost wavefronts: v of the ghost ring, sent by its owner.
+  GCS_DEV void receive(double v[KP]) {
+    if (!ghost) return;
+    const ll_word *s = halo_slot(g, w == 0 ? 0 : 1);
+    for (int spin = 0; spin < kSpinLimit; ++spin) {
+      ll_word a[KP], b[KP];
+      bool ok = true;
+#pragma unroll
+      for (int t = 0; t < KP; ++t)
+        if (t < cnt) {
+          a[t] = ll_load(s + (2 * t) * 64 + lane);
+          b[t] = ll_load(s + (2 * t + 1) * 64 + lane);
         }
-    }
-    const double den = gsum(a);
-    // 5: s and its norm
-    a = 0.0;
-    if (live) {
-      alpha = rho / den;
-      for (long q = t0; q < n; q += st) {
-        s[q] = r[q] - alpha * ap[q];
-        a += orig_term(c, s[q], q, ps, dt);
+#pragma unroll
+      for (int t = 0; t < KP; ++t)
+        if (t < cnt) ok = ok && (unsigned)a[t] == hseq && (unsigned)b[t] == hseq;
+      if (__all(ok)) {
+#pragma unroll
+        for (int t = 0; t < KP; ++t)
+          if (t < cnt) v[t] = ll_value(a[t], b[t]);
+        return;
       }
     }
-    const double snorm = sqrt(fmax(0.0, gsum(a)));
-    if (live && (!isfinite(den) || fabs(den) <= DBL_MIN)) live = false;
-    if (live && snorm <= target) {
+    *gave_up = 1;
+  }
+
+  // Sums of NV values over the hemisphere (ghosts and idle wavefronts give
+  // zero), the same in every thread of it.
+  template <int NV>
+  GCS_DEV void sum(double (&v)[NV]) {
+    ++seq;
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      const double s = wave_sum(own ? v[n] : 0.0);
+      if (lane == 0) part[n][w] = s;
+    }
+    __syncthreads();
+    if (w == 0) {
+      ll_word *bank = comm.red + (((seq & 1) * 2 + h) * (long)groups) * (kRingSums * 2);
+      if (lane < NV) {
+        double s = 0.0;
+        for (int q = 0; q < kRingWaves; ++q) s += part[lane][q];
+        ll_word *mine = bank + (g * kRingSums + lane) * 2;
+        ll_put(mine, mine + 1, s, seq);
+      }
+      double acc[NV];
+#pragma unroll
+      for (int n = 0; n < NV; ++n) acc[n] = 0.0;
+      bool got = true;
+      for (int q = lane; q < (groups + 63) / 64 * 64; q += 64) {
+        const ll_word *slot = bank + (long)min(q, groups - 1) * (kRingSums * 2);
+        int spin = 0;
+        for (; spin < kSpinLimit; ++spin) {
+          ll_word a[NV], b[NV];
+          bool ok = true;
+#pragma unroll
+          for (int n = 0; n < NV; ++n) {
+            a[n] = ll_load(slot + 2 * n);
+            b[n] = ll_load(slot + 2 * n + 1);
+          }
+#pragma unroll
+          for (int n = 0; n < NV; ++n)
+            ok = ok && (unsigned)a[n] == seq && (unsigned)b[n] == seq;
+          if (__all(ok)) {
+#pragma unroll
+            for (int n = 0; n < NV; ++n)
+              if (q < groups) acc[n] += ll_value(a[n], b[n]);
+            break;
+          }
+        }
+        got = got && spin < kSpinLimit;
+      }
+#pragma unroll
+      for (int n = 0; n < NV; ++n) {
+        const double s = wave_sum(acc[n]);
+        if (lane == 0) total[n] = s;
+      }
+      if (lane == 0) {
+        if (!got) *gave_up = 1;
+        // one thread's reading, so that the workgroup leaves together
+        total[kRingSums] = *(volatile int *)gave_up != 0 ? 1.0 : 0.0;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NV; ++n) v[n] = total[n];
+    dead = dead || total[kRingSums] != 0.0;
+  }
+
+  // Put v into this wavefront's LDS row, for the neighbour rings.
+  GCS_DEV void publish(const double v[KP]) {
+    if (own || ghost)
+#pragma unroll
+      for (int t = 0; t < KP; ++t) rows[w][t * 64 + lane] = v[t];
+    __syncthreads();
+  }
+
+  // v at j - 1 of this lane's first point and at j + 1 of its last one.
+  GCS_DEV void ends(const double v[KP], double &left, double &right) const {
+    const double lv = v[KP - 1];
+    double mine_last = v[0];
+#pragma unroll
+    for (int t = 0; t < KP; ++t)
+      if (t == last_t) mine_last = v[t];
+    // the lane reads stand outside the selections: under a branch, the value
+    // read would be computed for the branch's own lanes only
+    const double before = dpp_move<DPP_WAVE_SHR1>(0.0, lv), end = read_lane(mine_last, last_lane);
+    const double after = dpp_move<DPP_WAVE_SHL1>(0.0, v[0]), start = read_lane(v[0], 0);
+    left = lane == 0 ? end : before;
+    right = lane == last_lane ? start : after;
+  }
+};
+
+// The ring's row of the operator (uniform along the ring) and the pole's.
+struct RingRow {
+  double diag, lo, hi, llo, lhi;  // tensor: coefficients as k_mi_setup stores them
+  double w, plo, phi, plon;       // Pedersen: k_mi_apply's factors
+  double pe, pole_diag;
+};
+
+// out = A v on own rings (v published), and the pole row in the wavefront
+// of ring 1; k_mi_apply's arithmetic.
+template <int KP, bool Tensor>
+GCS_DEV void ring_product(const MiK &c, const RingWave<KP> &s, const RingRow &row,
+                          const double v[KP], double v_pole, double out[KP], double &out_pole) {
+  if (!s.own) return;
+  double left, right;
+  s.ends(v, left, right);
+  const bool first = s.ring == 1, last = s.ring == c.nt - 2;
+  double below[KP], above[KP];
+#pragma unroll
+  for (int t = 0; t < KP; ++t) {
+    below[t] = first ? v_pole : s.rows[s.w - 1][t * 64 + s.lane];
+    above[t] = last ? 0.0 : s.rows[s.w + 1][t * 64 + s.lane];
+  }
+  double ring = 0.0;
+#pragma unroll
+  for (int t = 0; t < KP; ++t) {
+    const double vm = t == 0 ? left : v[t - 1];
+    const double vp = (t == KP - 1 || t == s.cnt - 1) ? right : v[t < KP - 1 ? t + 1 : t];
+    if (Tensor)
+      out[t] = row.diag * v[t] + row.lo * below[t] + row.hi * above[t] + row.llo * vm +
+               row.lhi * vp;
+    else
+      out[t] = row.w * (row.plo * (v[t] - below[t]) + row.phi * (v[t] - above[t]) +
+                        row.plon * (2.0 * v[t] - vm - vp));
+    if (t < s.cnt) ring += v[t];
+    if (t >= s.cnt) out[t] = 0.0;
+  }
+  if (first) {
+    ring = wave_sum(ring);
+    out_pole = Tensor ? row.pole_diag * v_pole - row.pe * ring
+                      : row.pe * ((double)c.np * v_pole - ring);
+  }
+}
+
+template <int KP>
+GCS_DEV double ring_dot(const double a[KP], const double b[KP]) {
+  double s = 0.0;
+#pragma unroll
+  for (int t = 0; t < KP; ++t) s += a[t] * b[t];
+  return s;
+}
+
+// Constants of the wavefront's ring; rings of the tensor system also need
+// the sums' weight of the unweighted residual (orig_term).
+template <int KP, bool Tensor>
+GCS_DEV RingRow ring_row(const MiK &c, const RingWave<KP> &s, double &inv_sin2, double &ps) {
+  RingRow r = {};
+  const double dt = c.max_colat / (double)(c.nt - 1);
+  const double dp = 2.0 * kPi / (double)c.np;
+  const double half = 0.5 * dt;
+  r.pe = sin(half) * c.pedersen / (incl2(half) * dt * dt);
+  ps = (double)c.np * r.pe;
+  r.pole_diag = c.vec(s.h, V_DIAG)[0];
+  inv_sin2 = 0.0;
+  if (!s.own && !s.ghost) return r;
+  const int base = red_at(c.np, s.ring, 0);
+  const double th = (double)s.ring * dt;
+  r.diag = c.vec(s.h, V_DIAG)[base];
+  if (Tensor) {
+    r.lo = c.vec(s.h, V_LO)[base];
+    r.hi = c.vec(s.h, V_HI)[base];
+    r.llo = c.vec(s.h, V_LLO)[base];
+    r.lhi = c.vec(s.h, V_LHI)[base];
+  } else {
+    r.w = sin(th);
+    r.plo = theta_coeff(c.pedersen, th - 0.5 * dt, th, dt);
+    r.phi = theta_coeff(c.pedersen, th + 0.5 * dt, th, dt);
+    r.plon = c.pedersen / (sin(th) * sin(th) * dp * dp);
+  }
+  inv_sin2 = 1.0 / (sin(th) * sin(th));
+  return r;
+}
+
+template <int KP>
+GCS_DEV void ring_load(const RingWave<KP> &s, const MiK &c, const double *vec, double out[KP]) {
+  const int base = red_at(c.np, max(s.ring, 1), 0);
+#pragma unroll
+  for (int t = 0; t < KP; ++t)
+    out[t] = (s.own || s.ghost) && t < s.cnt ? vec[base + s.j0 + t] : 0.0;
+}
+
+// The solved potential to the polar grid: pole row, rings, zero outer row.
+template <int KP>
+GCS_DEV void ring_store(const RingWave<KP> &s, const MiK &c, const double x[KP], double x_pole) {
+  double *pot = c.potential + (long)s.h * c.nt * c.np;
+  if (!s.own) return;
+#pragma unroll
+  for (int t = 0; t < KP; ++t)
+    if (t < s.cnt) {
+      const int j = s.j0 + t;
+      pot[(long)s.ring * c.np + j] = x[t];
+      if (s.ring == 1) pot[j] = x_pole;
+      if (s.ring == c.nt - 2) pot[(long)(c.nt - 1) * c.np + j] = 0.0;
+    }
+}
+
+// Jacobi-preconditioned CG on the reduced Pedersen system (:516-600), with
+// its two dot products and the residual norm in one reduction: A p follows
+// from A z by the recurrence of p, and p . A p from z . A z (Chronopoulos and
+// Gear, J. Comput. Appl. Math. 25, 1989). The iterates are CG's up to
+// rounding; convergence is decided on the true residual, as before.
+template <int KP>
+__global__ void __launch_bounds__(kRingThreads) k_ring_cg(MiK c, RingComm comm, double rel_tol,
+                                                          int maxit) {
+  __shared__ double rows[kRingWaves][64 * KP], part[kRingSums][kRingWaves], total[kRingSums + 1];
+  __shared__ int gave_up;
+  RingWave<KP> s;
+  s.init(c, comm, rows, part, total, &gave_up);
+  double is2, ps;
+  const RingRow row = ring_row<KP, false>(c, s, is2, ps);
+  const bool pole = s.own && s.ring == 1;     // carries the pole unknown
+  const bool pole_lane = pole && s.lane == 0; // adds it to the sums
+  const double inv_diag = (s.own || s.ghost) ? 1.0 / row.diag : 0.0;
+  const double inv_pole = 1.0 / row.pole_diag;
+  // u = z of the current residual, w = A u, p and s = A p
+  double x[KP], r[KP], u[KP], w[KP], p[KP], sv[KP];
+  double x0, r0, u0 = 0.0, w0 = 0.0, p0 = 0.0, s0 = 0.0;
+  // r = rhs - A x, sent to the ghosts; b2 = this wavefront's part of |rhs|^2
+  auto residual = [&](double &b2) {
+    double rhs[KP];
+    ring_load<KP>(s, c, c.vec(s.h, V_RHS), rhs);
+    s.publish(x);
+    ring_product<KP, false>(c, s, row, x, x0, w, w0);
+    if (s.own)
+#pragma unroll
+      for (int t = 0; t < KP; ++t) r[t] = rhs[t] - w[t];
+    r0 = c.vec(s.h, V_RHS)[0] - w0;
+    b2 = ring_dot<KP>(rhs, rhs) * is2;
+    s.send(r);
+  };
+  // |r|^2 of the unweighted equations
+  auto norm_part = [&]() {
+    return ring_dot<KP>(r, r) * is2 + (pole_lane ? (double)c.np * (r0 / ps) * (r0 / ps) : 0.0);
+  };
+#pragma unroll
+  for (int t = 0; t < KP; ++t) r[t] = u[t] = w[t] = p[t] = sv[t] = 0.0;
+  ring_load<KP>(s, c, c.vec(s.h, V_X), x);
+  x0 = c.vec(s.h, V_X)[0];
+  double v2[2];
+  residual(v2[1]);
+  v2[0] = norm_part();
+  s.sum(v2);
+  s.receive(r);
+  double norm = sqrt(fmax(0.0, v2[0]));
+  const double first = norm;
+  const double target = rel_tol * fmax(sqrt(fmax(0.0, v2[1])), 1.0);
+  SolveResult res{0, norm <= target, norm};
+  bool restart = true;
+  double alpha = 0.0, gamma_prev = 1.0;
+  for (int it = 0; it <= maxit && !res.ok && !s.dead; ++it) {
+    // r is the residual after `it` iterations
+#pragma unroll
+    for (int t = 0; t < KP; ++t) u[t] = r[t] * inv_diag;
+    u0 = r0 * inv_pole;
+    s.publish(u);
+    ring_product<KP, false>(c, s, row, u, u0, w, w0);
+    s.send(w);
+    double v3[3] = {ring_dot<KP>(r, u) + (pole_lane ? r0 * u0 : 0.0),
+                    ring_dot<KP>(w, u) + (pole_lane ? w0 * u0 : 0.0), norm_part()};
+    s.sum(v3);
+    s.receive(w);
+    const double gamma = v3[0], delta = v3[1];
+    norm = sqrt(fmax(0.0, v3[2]));
+    res.iters = it;
+    res.last = norm;
+    if (!restart && (norm <= target || it % 1024 == 0)) {
+      residual(v2[1]);
+      v2[0] = norm_part();
+      s.sum(v2);
+      s.receive(r);
+      norm = sqrt(fmax(0.0, v2[0]));
+      res.last = norm;
+      if (norm <= target) res.ok = true;
+      restart = true;
+      --it;  // the same iteration again, from the true residual
+      continue;
+    }
+    if (it == maxit) break;
+    const double beta = restart ? 0.0 : gamma / gamma_prev;
+    // p . A p = u . A u - beta^2 p_prev . A p_prev, with the latter
+    // gamma_prev / alpha
+    const double pap = restart ? delta : delta - beta * gamma / alpha;
+    if (!isfinite(gamma) || gamma <= DBL_MIN || !isfinite(pap) || pap <= DBL_MIN) break;
+    alpha = gamma / pap;
+    gamma_prev = gamma;
+#pragma unroll
+    for (int t = 0; t < KP; ++t) {
+      p[t] = u[t] + (restart ? 0.0 : beta * p[t]);
+      sv[t] = w[t] + (restart ? 0.0 : beta * sv[t]);
+      x[t] += alpha * p[t];
+      r[t] -= alpha * sv[t];
+    }
+    p0 = u0 + (restart ? 0.0 : beta * p0);
+    s0 = w0 + (restart ? 0.0 : beta * s0);
+    x0 += alpha * p0;
+    r0 -= alpha * s0;
+    restart = false;
+  }
+  res.ok = res.ok && !s.dead;
+  ring_store<KP>(s, c, x, x0);
+  if (s.g == 0) store_result(c, s.h, res, first);
+}
+
+// Factors of the ring preconditioner (ring_factor) that a lane applies.
+template <int KP>
+struct RingFactors {
+  double ib[KP], gd[KP], zz[KP], a, corner, inv_den;
+};
+
+template <int KP>
+GCS_DEV RingFactors<KP> ring_factors(const RingWave<KP> &s, const MiK &c, const RingRow &row) {
+  RingFactors<KP> f = {};
+  if (!s.own && !s.ghost) return f;
+  const int base = red_at(c.np, s.ring, 0);
+  const double *g = c.vec(s.h, V_SCR) + base, *z = c.vec(s.h, V_SCR2) + base,
+               *ib = c.vec(s.h, V_IB) + base;
+#pragma unroll
+  for (int t = 0; t < KP; ++t) {
+    const int j = s.j0 + t;
+    const bool in = t < s.cnt;
+    f.ib[t] = in ? ib[j] : 0.0;
+    f.gd[t] = in && j < c.np - 1 ? -g[j + 1] : 0.0;
+    f.zz[t] = in ? z[j] : 0.0;
+  }
+  f.a = row.llo;
+  f.corner = row.llo / -row.diag;  // the periodic corner's weight, a / gamma
+  f.inv_den = 1.0 / c.vec(s.h, V_RDEN)[base];
+  return f;
+}
+
+// out = M^-1 in on the wavefront's ring: ring_apply with its operands in
+// registers.
+template <int KP>
+GCS_DEV void ring_solve(const RingWave<KP> &s, const RingFactors<KP> &f, const double in[KP],
+                        double out[KP]) {
+  const int lane = s.lane;
+  double fa[KP], fb[KP];
+  double A = 0.0, B = 1.0;
+#pragma unroll
+  for (int t = 0; t < KP; ++t) {
+    fa[t] = f.ib[t] * in[t];
+    fb[t] = (t == 0 && lane == 0) ? 0.0 : -f.a * f.ib[t];
+    if (t < s.cnt) {
+      A = fa[t] + fb[t] * A;
+      B = fb[t] * B;
+    }
+  }
+  // rows of 16 lanes, then the value at the end of the rows before
+  affine_step<DPP_ROW_SHR + 1>(A, B);
+  affine_step<DPP_ROW_SHR + 2>(A, B);
+  affine_step<DPP_ROW_SHR + 4>(A, B);
+  affine_step<DPP_ROW_SHR + 8>(A, B);
+  const double p1 = read_lane(A, 15);
+  const double p2 = read_lane(A, 31) + read_lane(B, 31) * p1;
+  const double p3 = read_lane(A, 47) + read_lane(B, 47) * p2;
+  const int rowid = lane >> 4;
+  A = A + B * (rowid == 0 ? 0.0 : rowid == 1 ? p1 : rowid == 2 ? p2 : p3);
+  double w = dpp_move<DPP_WAVE_SHR1>(0.0, A);
+  double v[KP];
+#pragma unroll
+  for (int t = 0; t < KP; ++t) {
+    v[t] = 0.0;
+    if (t < s.cnt) {
+      w = fa[t] + fb[t] * w;
+      v[t] = w;
+    }
+  }
+  double C = 0.0, D = 1.0;
+#pragma unroll
+  for (int t = KP - 1; t >= 0; --t)
+    if (t < s.cnt) {
+      C = v[t] + f.gd[t] * C;
+      D = f.gd[t] * D;
+    }
+  affine_step<DPP_ROW_SHL + 1>(C, D);
+  affine_step<DPP_ROW_SHL + 2>(C, D);
+  affine_step<DPP_ROW_SHL + 4>(C, D);
+  affine_step<DPP_ROW_SHL + 8>(C, D);
+  const double q2 = read_lane(C, 48);
+  const double q1 = read_lane(C, 32) + read_lane(D, 32) * q2;
+  const double q0 = read_lane(C, 16) + read_lane(D, 16) * q1;
+  C = C + D * (rowid == 3 ? 0.0 : rowid == 2 ? q2 : rowid == 1 ? q1 : q0);
+  w = dpp_move<DPP_WAVE_SHL1>(0.0, C);
+#pragma unroll
+  for (int t = KP - 1; t >= 0; --t)
+    if (t < s.cnt) {
+      w = v[t] + f.gd[t] * w;
+      v[t] = w;
+    }
+  const double y0 = read_lane(v[0], 0);
+  double mine_last = v[0];
+#pragma unroll
+  for (int t = 0; t < KP; ++t)
+    if (t == s.last_t) mine_last = v[t];
+  const double yl = read_lane(mine_last, s.last_lane);
+  const double fact = (y0 + f.corner * yl) * f.inv_den;
+#pragma unroll
+  for (int t = 0; t < KP; ++t) out[t] = t < s.cnt ? v[t] - fact * f.zz[t] : 0.0;
+}
+
+// ring_factor with the ring's coefficients read once (they are uniform along
+// it) and the serial recurrences in LDS: one workgroup per ring, spread over
+// the chip, whose first lane factors and whose lanes store.
+__global__ void __launch_bounds__(64) k_ring_factor(MiK c) {
+  __shared__ double g[64 * kRingChunk], z[64 * kRingChunk], ib[64 * kRingChunk];
+  const int h = blockIdx.y, np = c.np, base = red_at(np, 1 + blockIdx.x, 0);
+  if (threadIdx.x == 0) {
+    const double a = c.vec(h, V_LLO)[base], b = c.vec(h, V_DIAG)[base],
+                 cc = c.vec(h, V_LHI)[base];
+    const double gam = -b, tail = b - cc * a / gam;
+    double inv = 1.0 / (b - gam), zp = gam * inv;
+    ib[0] = inv;
+    g[0] = 0.0;
+    z[0] = zp;
+    for (int j = 1; j < np; ++j) {
+      const bool last = j == np - 1;
+      const double gj = cc * inv;
+      g[j] = gj;
+      inv = 1.0 / ((last ? tail : b) - a * gj);
+      ib[j] = inv;
+      zp = ((last ? cc : 0.0) - a * zp) * inv;
+      z[j] = zp;
+    }
+    const double zl = zp;
+    for (int j = np - 2; j >= 0; --j) {
+      zp = z[j] - g[j + 1] * zp;
+      z[j] = zp;
+    }
+    c.vec(h, V_RDEN)[base] = 1.0 + zp + a * zl / gam;
+  }
+  __syncthreads();
+  for (int j = threadIdx.x; j < np; j += 64) {
+    c.vec(h, V_SCR)[base + j] = g[j];
+    c.vec(h, V_SCR2)[base + j] = z[j];
+    c.vec(h, V_IB)[base + j] = ib[j];
+  }
+}
+
+// Right-preconditioned BiCGStab on the tensor system (:1029-1131). The norm
+// of the new residual s - omega A s and its product with the shadow vector
+// are formed from the sums that omega needs anyway, so that an iteration has
+// two reductions; the norm decides only when the true residual is computed.
+template <int KP>
+__global__ void __launch_bounds__(kRingThreads) k_ring_bicgstab(MiK c, RingComm comm,
+                                                                double rel_tol, int maxit) {
+  __shared__ double rows[kRingWaves][64 * KP], part[kRingSums][kRingWaves], total[kRingSums + 1];
+  __shared__ int gave_up;
+  RingWave<KP> s;
+  s.init(c, comm, rows, part, total, &gave_up);
+  double is2, ps;
+  const RingRow row = ring_row<KP, true>(c, s, is2, ps);
+  const RingFactors<KP> fac = ring_factors<KP>(s, c, row);
+  const bool pole = s.own && s.ring == 1;
+  const bool pole_lane = pole && s.lane == 0;
+  double x[KP], r[KP], p[KP], ap[KP], sh[KP], pp[KP], sv[KP], psv[KP], as[KP];
+  double x0, r0, p0 = 0.0, ap0 = 0.0, sh0, pp0 = 0.0, s0 = 0.0, ps0 = 0.0, as0 = 0.0;
+  // one vector's part of the squared norm of the unweighted equations
+  auto norm_part = [&](const double v[KP], double v0) {
+    double q = ring_dot<KP>(v, v) * is2;
+    if (pole_lane) q += (double)c.np * (v0 / ps) * (v0 / ps);
+    return q;
+  };
+  auto residual = [&](double &b2) {
+    double rhs[KP];
+    ring_load<KP>(s, c, c.vec(s.h, V_RHS), rhs);
+    s.publish(x);
+    double t0 = 0.0;
+    ring_product<KP, true>(c, s, row, x, x0, as, t0);
+    if (s.own)
+#pragma unroll
+      for (int t = 0; t < KP; ++t) r[t] = rhs[t] - as[t];
+    r0 = c.vec(s.h, V_RHS)[0] - t0;
+    b2 = ring_dot<KP>(rhs, rhs) * is2;
+    s.send(r);
+  };
+#pragma unroll
+  for (int t = 0; t < KP; ++t) r[t] = p[t] = ap[t] = pp[t] = sv[t] = psv[t] = as[t] = 0.0;
+  ring_load<KP>(s, c, c.vec(s.h, V_X), x);
+  x0 = c.vec(s.h, V_X)[0];
+  double v3[3];
+  residual(v3[2]);
+  v3[0] = norm_part(r, r0);
+  v3[1] = ring_dot<KP>(r, r) + (pole_lane ? r0 * r0 : 0.0);
+  s.sum(v3);
+  s.receive(r);
+  double norm = sqrt(fmax(0.0, v3[0])), rho = v3[1];
+  const double first = norm;
+  const double target = rel_tol * fmax(sqrt(fmax(0.0, v3[2])), 1.0);
+  SolveResult res{0, norm <= target, norm};
+#pragma unroll
+  for (int t = 0; t < KP; ++t) sh[t] = r[t];
+  sh0 = r0;
+  double rho_prev = 1.0, alpha = 1.0, omega = 1.0;
+  for (int it = 1; it <= maxit && !res.ok && !s.dead; ++it) {
+    if (!isfinite(rho) || fabs(rho) <= DBL_MIN || !isfinite(omega) || fabs(omega) <= DBL_MIN)
+      break;
+    const double beta = (rho / rho_prev) * (alpha / omega);
+#pragma unroll
+    for (int t = 0; t < KP; ++t) p[t] = r[t] + beta * (p[t] - omega * ap[t]);
+    p0 = r0 + beta * (p0 - omega * ap0);
+    ring_solve<KP>(s, fac, p, pp);
+    pp0 = p0 / row.pole_diag;
+    s.publish(pp);
+    ring_product<KP, true>(c, s, row, pp, pp0, ap, ap0);
+    s.send(ap);
+    double v1[1] = {ring_dot<KP>(sh, ap) + (pole_lane ? sh0 * ap0 : 0.0)};
+    s.sum(v1);
+    s.receive(ap);
+    const double den = v1[0];
+    if (!isfinite(den) || fabs(den) <= DBL_MIN) break;
+    alpha = rho / den;
+#pragma unroll
+    for (int t = 0; t < KP; ++t) sv[t] = r[t] - alpha * ap[t];
+    s0 = r0 - alpha * ap0;
+    ring_solve<KP>(s, fac, sv, psv);
+    ps0 = s0 / row.pole_diag;
+    s.publish(psv);
+    ring_product<KP, true>(c, s, row, psv, ps0, as, as0);
+    s.send(as);
+    double v7[7] = {ring_dot<KP>(as, as), ring_dot<KP>(as, sv), ring_dot<KP>(sh, sv),
+                    ring_dot<KP>(sh, as), 0.0, 0.0, norm_part(sv, s0)};
+    v7[4] = v7[0] * is2;
+    v7[5] = v7[1] * is2;
+    if (pole_lane) {
+      v7[0] += as0 * as0;
+      v7[1] += as0 * s0;
+      v7[2] += sh0 * s0;
+      v7[3] += sh0 * as0;
+      v7[4] += (double)c.np * (as0 / ps) * (as0 / ps);
+      v7[5] += (double)c.np * (as0 / ps) * (s0 / ps);
+    }
+    s.sum(v7);
+    s.receive(as);
+    const double wden = v7[0], wnum = v7[1], snorm = sqrt(fmax(0.0, v7[6]));
+    if (snorm <= target) {
       res.last = snorm;
       res.iters = it;
       res.ok = true;
-      live = false;
-      for (long q = t0; q < n; q += st) x[q] += alpha * pp[q];
+#pragma unroll
+      for (int t = 0; t < KP; ++t) x[t] += alpha * pp[t];
+      x0 += alpha * pp0;
+      break;
     }
-    // 6, 7: preconditioned s
-    precondition(live, s, psv);
-    // 8: A ps and omega
-    a = 0.0;
-    b = 0.0;
-    {
-      const double pole = (live && pole_wave) ? pole_row(c, h, true, psv, pe) : 0.0;
-      if (live)
-        for (long q = t0; q < n; q += st) {
-          as[q] = q == 0 ? pole : apply_at(c, h, true, psv, q, nullptr, pe);
-          a += as[q] * as[q];
-          b += as[q] * s[q];
-        }
+    omega = wnum / wden;
+    if (!isfinite(wden) || wden <= DBL_MIN || !isfinite(omega) || fabs(omega) <= DBL_MIN) break;
+#pragma unroll
+    for (int t = 0; t < KP; ++t) {
+      x[t] += alpha * pp[t] + omega * psv[t];
+      r[t] = sv[t] - omega * as[t];
     }
-    double wden, wnum;
-    gsum2(a, b, wden, wnum);
-    if (live) {
-      omega = wnum / wden;
-      if (!isfinite(wden) || wden <= DBL_MIN || !isfinite(omega) || fabs(omega) <= DBL_MIN)
-        live = false;
-    }
-    // 9: x, r and the recursive residual norm
-    a = 0.0;
-    if (live)
-      for (long q = t0; q < n; q += st) {
-        x[q] += alpha * pp[q] + omega * psv[q];
-        r[q] = s[q] - omega * as[q];
-        a += orig_term(c, r[q], q, ps, dt);
-      }
-    const double rn = gsum(a);
-    bool verify = false;
-    if (live) {
-      norm = sqrt(fmax(0.0, rn));
-      res.iters = it;
+    x0 += alpha * pp0 + omega * ps0;
+    r0 = s0 - omega * as0;
+    // |r|^2 and shadow . r of r = s - omega A s, from the sums above
+    double v2[2] = {v7[6] - omega * (2.0 * v7[5] - omega * v7[4]), v7[2] - omega * v7[3]};
+    norm = sqrt(fmax(0.0, v2[0]));
+    res.iters = it;
+    res.last = norm;
+    if (norm <= target || it % 256 == 0) {
+      residual(v3[2]);
+      v2[0] = norm_part(r, r0);
+      v2[1] = ring_dot<KP>(r, r) + (pole_lane ? r0 * r0 : 0.0);
+      s.sum(v2);
+      s.receive(r);
+      norm = sqrt(fmax(0.0, v2[0]));
       res.last = norm;
-      verify = norm <= target || it % 256 == 0;
-    }
-    // 10: true residual when checked; the exit flags of both hemispheres
-    a = 0.0;
-    if (verify) {
-      const double pole = pole_wave ? pole_row(c, h, true, x, pe) : 0.0;
-      for (long q = t0; q < n; q += st) {
-        r[q] = rhs[q] - (q == 0 ? pole : apply_at(c, h, true, x, q, nullptr, pe));
-        sh[q] = r[q];
-        a += orig_term(c, r[q], q, ps, dt);
+      if (norm <= target) res.ok = true;
+#pragma unroll
+      for (int t = 0; t < KP; ++t) {
+        sh[t] = r[t];
+        p[t] = ap[t] = 0.0;
       }
+      sh0 = r0;
+      p0 = ap0 = 0.0;
+      rho = v2[1];
+      rho_prev = alpha = omega = 1.0;
+      continue;
     }
-    const double tn = gsum(a);
-    if (verify) {
-      norm = sqrt(fmax(0.0, tn));
-      res.last = norm;
-      if (norm <= target) {
-        res.ok = true;
-        live = false;
-      } else {
-        for (long q = t0; q < n; q += st) {
-          p[q] = 0.0;
-          ap[q] = 0.0;
-        }
-        rho_prev = alpha = omega = 1.0;
-      }
-    } else if (live) {
-      rho_prev = rho;
-    }
-    // exchange liveness: written now, read after the next iteration's first
-    // barrier; one more round trip than needed only delays the exit
-    if (lb == 0 && threadIdx.x == 0) flags[(it & 1) * 2 + h] = live ? 1 : 0;
-    grid.sync();
-    other_live = flags[(it & 1) * 2 + (1 - h)] != 0;
+    rho_prev = rho;
+    rho = v2[1];
   }
-  if (lb == 0) store_result(c, h, res, first);
+  res.ok = res.ok && !s.dead;
+  ring_store<KP>(s, c, x, x0);
+  if (s.g == 0) store_result(c, s.h, res, first);
+}
+
+// The kernels by points per lane, 1 .. kRingChunk.
+typedef void (*RingKernel)(MiK, RingComm, double, int);
+template <int KP>
+RingKernel ring_kernel_of(bool tensor) {
+  return tensor ? k_ring_bicgstab<KP> : k_ring_cg<KP>;
+}
+RingKernel ring_kernel(int points, bool tensor) {
+  static_assert(kRingChunk == 8, "one case per points per lane");
+  switch (points) {
+    case 1: return ring_kernel_of<1>(tensor);
+    case 2: return ring_kernel_of<2>(tensor);
+    case 3: return ring_kernel_of<3>(tensor);
+    case 4: return ring_kernel_of<4>(tensor);
+    case 5: return ring_kernel_of<5>(tensor);
+    case 6: return ring_kernel_of<6>(tensor);
+    case 7: return ring_kernel_of<7>(tensor);
+    default: return ring_kernel_of<8>(tensor);
+  }
 }
 
 // ---- learned warm start ----------------------------------------------------------
@@ -1350,34 +1943,35 @@ int solve(Problem &P, bool tensor) {
   MiK c = make_mik(P);
   hipStream_t s = P.stream;
   const auto t0 = std::chrono::steady_clock::now();
-  const int act[2] = {1, 1};
-  GCS_HIP(hipMemcpyAsync(m.active, act, sizeof(act), hipMemcpyHostToDevice, s));
   const dim3 g2(blocks_of(m.n), 2);
-  k_mi_setup<<<g2, kT, 0, s>>>(c, tensor ? 1 : 0, m.hall);
+  const int points = (m.np + 63) / 64;
+  RingComm comm{m.ring_words, nullptr, m.ring_groups, points};
+  const long red = (long)RingComm::red_words(m.ring_groups);
+  const long words =
+      comm.red != nullptr ? red + (long)RingComm::halo_words(m.ring_groups, points) : 0;
+  comm.halo = comm.red + red;
+  k_mi_setup<<<g2, kT, 0, s>>>(c, tensor ? 1 : 0, m.hall, m.ring_words, words);
   if (m.net != nullptr && warm_start(P, c, tensor) != 0) return -1;
-  const double rel = m.cfg.relative_tolerance;
-  const int maxit = m.cfg.maximum_iterations;
-  if (tensor) {
-    // cooperative form (both hemispheres, 2 kCoopBlocks workgroups) when the
-    // device can hold its workgroups at once; one workgroup per hemisphere
-    // otherwise
-    bool coop = m.coop_slots != nullptr;
-    if (coop) {
-      double relv = rel;
-      int maxv = maxit;
-      double *slots = m.coop_slots;
-      int *flags = m.coop_flags;
-      void *args[] = {&c, &relv, &maxv, &slots, &flags};
-      if (hipLaunchCooperativeKernel((const void *)k_mi_bicgstab_pair, dim3(2 * kCoopBlocks),
-                                     dim3(kSolveThreads), args, 0, s) != hipSuccess) {
-        (void)hipGetLastError();
-        coop = false;
-      }
+  double rel = m.cfg.relative_tolerance;
+  int maxit = m.cfg.maximum_iterations;
+  bool resident = comm.red != nullptr;
+  if (resident) {
+    if (tensor) k_ring_factor<<<dim3(m.nt - 2, 2), 64, 0, s>>>(c);
+    void *args[] = {&c, &comm, &rel, &maxit};
+    if (hipLaunchCooperativeKernel((const void *)ring_kernel(points, tensor),
+                                   dim3(2 * m.ring_groups), dim3(kRingThreads), args, 0, s) !=
+        hipSuccess) {
+      (void)hipGetLastError();
+      resident = false;
     }
-    if (!coop) k_mi_bicgstab<<<2, kSolveThreads, 0, s>>>(c, rel, maxit);
-  } else
-    k_mi_cg<<<2, kSolveThreads, 4 * (size_t)m.nt * sizeof(double), s>>>(c, rel, maxit);
-  k_mi_vec<<<dim3(blocks_of((long)m.np * m.nt), 2), kT, 0, s>>>(c, OP_EXPAND, 0.0, m.active);
+  }
+  if (!resident) {
+    if (tensor)
+      k_mi_bicgstab<<<2, kSolveThreads, 0, s>>>(c, rel, maxit);
+    else
+      k_mi_cg<<<2, kSolveThreads, 4 * (size_t)m.nt * sizeof(double), s>>>(c, rel, maxit);
+    k_mi_vec<<<dim3(blocks_of((long)m.np * m.nt), 2), kT, 0, s>>>(c, OP_EXPAND, 0.0, m.active);
+  }
   GCS_HIP(hipGetLastError());
   GCS_HIP(hipMemcpyAsync(m.host_scal, m.scal, 2 * SL_COUNT * sizeof(double),
                          hipMemcpyDeviceToHost, s));
@@ -1553,27 +2147,33 @@ int mi_create(Problem &P) {
   GCS_HIP(hipMalloc(&m.drift, 18L * L.ghost * L.NJ * L.NK * sizeof(double)));
   GCS_HIP(hipMalloc(&m.work, 2L * kVectors * m.n * sizeof(double)));
   {
-    // the cooperative BiCGStab needs all 2 kCoopBlocks workgroups resident;
-    // GCS_MI_COOPERATIVE=0 selects the single-workgroup solve instead (for
-    // tools that cannot follow a cooperative launch, such as the kernel
+    // the register-resident solves need all their workgroups resident at
+    // once; GCS_MI_COOPERATIVE=0 selects the single-workgroup solves instead
+    // (for tools that cannot follow a cooperative launch, such as the kernel
     // tracer of rocprofv3 7.2, which faults at exit after one)
     const char *env = std::getenv("GCS_MI_COOPERATIVE");
     const bool allowed = env == nullptr || std::strcmp(env, "0") != 0;
+    const int points = (m.np + 63) / 64, groups = (m.nt - 2 + kRingOwn - 1) / kRingOwn;
     int dev = 0, coop = 0, per_cu = 0, cus = 0;
     if (allowed && hipGetDevice(&dev) == hipSuccess &&
         hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) == hipSuccess &&
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_mi_bicgstab_pair, kSolveThreads,
-                                                     0) == hipSuccess &&
-        coop != 0 && per_cu * cus >= 2 * kCoopBlocks) {
-      GCS_HIP(hipMalloc(&m.coop_slots, 8 * kCoopBlocks * sizeof(double)));
-      GCS_HIP(hipMalloc(&m.coop_flags, 4 * sizeof(int)));
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &per_cu, (const void *)ring_kernel(points, m.hall > 0.0), kRingThreads, 0) ==
+            hipSuccess &&
+        coop != 0 && (long)per_cu * cus >= 2L * groups) {
+      m.ring_groups = groups;
+      GCS_HIP(hipMalloc(&m.ring_words, (RingComm::red_words(groups) +
+                                        RingComm::halo_words(groups, points)) *
+                                           sizeof(ll_word)));
     }
     (void)hipGetLastError();
   }
   GCS_HIP(hipMalloc(&m.scal, 2 * SL_COUNT * sizeof(double)));
   GCS_HIP(hipHostMalloc(&m.host_scal, 2 * SL_COUNT * sizeof(double)));
   GCS_HIP(hipMalloc(&m.active, 2 * sizeof(int)));
+  const int act[2] = {1, 1};
+  GCS_HIP(hipMemcpy(m.active, act, sizeof(act), hipMemcpyHostToDevice));
   GCS_HIP(hipMemset(m.shell_fac, 0, 6L * S * S * sizeof(double)));
   GCS_HIP(hipMemset(m.fac, 0, polar * sizeof(double)));
   GCS_HIP(hipMemset(m.potential, 0, polar * sizeof(double)));
@@ -1612,8 +2212,7 @@ void mi_destroy(Problem &P) {
   (void)hipFree(m->active);
   if (m->host_scal) (void)hipHostFree(m->host_scal);
   (void)hipFree(m->warm_scale);
-  (void)hipFree(m->coop_slots);
-  (void)hipFree(m->coop_flags);
+  (void)hipFree(m->ring_words);
   delete m;
   P.mi = nullptr;
 }

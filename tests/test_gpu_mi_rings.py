@@ -1,0 +1,52 @@
+"""The register-resident polar solves (one wavefront per colatitude ring) at
+the sizes where their layout can go wrong: one ring and one point per lane up
+to eight, rings that end inside a lane, exactly full workgroups (six rings)
+and one ring more.
+
+The current of a generated potential (gcs_problem_mi_make_pairs) is solved
+from zero and must give that potential back. Tolerance: the solve stops at a
+residual of 1e-12 of the right-hand side, and the error is at most the
+operator's condition times that; the smallest eigenvalue of the polar
+operator is of order one of its colatitude coupling, and the largest, the
+longitude coupling of the ring next to the pole, exceeds it by less than 1e3
+(the residual norm weighs that ring up by the same sine), so 1e-9 of the
+largest potential is the bound. The single-workgroup solve of the same
+problem (GCS_MI_COOPERATIVE=0, read when a problem is made) must agree to
+twice that."""
+import importlib
+
+import numpy as np
+import pytest
+
+from conftest import gcs_config
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-9
+
+
+@pytest.mark.parametrize("hall", [0.0, 5.0])
+@pytest.mark.parametrize("nt,np_", [(3, 8), (4, 64), (8, 65), (9, 57), (14, 130), (20, 200),
+                                    (15, 256), (26, 321), (13, 385), (10, 449), (33, 512)])
+def test_ring_solves_return_the_generated_potential(gpu, monkeypatch, nt, np_, hall):
+    ws = importlib.import_module("gamera-cube_amd.warm_start")
+    cfg = gcs_config.earth_problem(16, 12, mi=True, hall_siemens=hall, mi_azimuth=np_,
+                                   mi_colatitude=nt)
+    cfg.mi.relative_tolerance = 1e-12
+    print(f"ring solve {nt} x {np_} hall {hall}", flush=True)
+    p = gpu.GpuProblem(cfg)
+    cur, pot = ws.make_pairs(p, seed=nt + np_, count=2, pedersen=cfg.mi.pedersen_siemens,
+                             hall=hall)
+    scale = np.abs(pot).max()
+    got, cold, _ = ws.solve_current(p, cur, np.zeros_like(pot), use_network=False)
+    print(f"  iterations {cold}, error {np.abs(got - pot).max() / scale:.1e}", flush=True)
+    assert np.abs(got - pot).max() <= TOL * scale
+    # from the solution itself: no more iterations than from zero (a BiCGStab
+    # solve may have stopped on its recursive residual, with the true one a
+    # little above the bound, so a few can be left), the same potential
+    again, warm, _ = ws.solve_current(p, cur, got, use_network=False)
+    assert sum(warm) <= sum(cold) and np.abs(again - got).max() <= TOL * scale
+    monkeypatch.setenv("GCS_MI_COOPERATIVE", "0")
+    q = gpu.GpuProblem(cfg)
+    single, _, _ = ws.solve_current(q, cur, np.zeros_like(pot), use_network=False)
+    assert np.abs(single - got).max() <= 2 * TOL * scale
