@@ -371,7 +371,9 @@ int upload_wind(Problem &P, int count, const double *time, const double *state);
 // array (at most 16,777,216 active cells; calls overlapping on one GPU race).
 int pressure_control_noalloc(Problem &P, const double args[7], unsigned long long counts[2],
                              double maxima[2]);
-int enqueue_phase(Problem &P, Phase phase);
+// With `driver` the first phase also runs the dt rule and the last one
+// advances the clock (enqueue_step of a driver step).
+int enqueue_phase(Problem &P, Phase phase, bool driver = false);
 // Constants derived from uploaded geometry and background: recovery
 // pivots, edge-B solve, B0 normal and edge-tangential components.
 int derive_constants(Problem &P);

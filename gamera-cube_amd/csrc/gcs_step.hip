@@ -197,10 +197,6 @@ GCS_DEV void cfl_fold(double v, unsigned long long *slots) {
   if ((threadIdx.x & 63) == 0) atomicMin(&slots[(tid() >> 6) % kCflSlots], bits);
 }
 
-__global__ void k_cfl_reset(unsigned long long *slots) {
-  slots[threadIdx.x] = __double_as_longlong(DBL_MAX);
-}
-
 // The CFL dt of every active cell from the current level, min-reduced to
 // one partial per block: the first step after creation or an upload (later
 // steps take the minimum the previous step's update folded into the slots).
@@ -234,10 +230,9 @@ __global__ void __launch_bounds__(kCflThreads) k_cfl(K c, unsigned long long *pa
 }
 
 // Driver dt rule (test_cubedsphere_dipole_background.c:593-616, :669-670),
-// after the min over the CFL kernel's per-block partials (one block).
-__global__ void __launch_bounds__(kCflThreads) k_dt(K c, double fraction,
-                                                    const unsigned long long *partial,
-                                                    int nblock) {
+// after the min over the CFL kernel's per-block partials or the update's
+// slots (one block of kCflThreads).
+GCS_DEV void dt_rule(const K &c, double fraction, const unsigned long long *partial, int nblock) {
   unsigned long long m = __double_as_longlong(DBL_MAX);
   for (int b = threadIdx.x; b < nblock; b += kCflThreads) m = partial[b] < m ? partial[b] : m;
   __shared__ unsigned long long red[kCflThreads];
@@ -266,7 +261,7 @@ __global__ void __launch_bounds__(kCflThreads) k_dt(K c, double fraction,
   s->wall_dt = s->dt;
 }
 
-__global__ void k_clock(K c) {
+GCS_DEV void advance_clock(const K &c) {
   StepScalars *s = c.sc;
   s->time += s->dt;
   s->previous_dt = s->dt;
@@ -276,8 +271,7 @@ __global__ void k_clock(K c) {
 // ---- seams -----------------------------------------------------------------
 
 // cubedsphere_interface.c:7-81 for the face flux of the given levels.
-__global__ void k_sync_phi(K c, const SeamPair *pairs, int n, int both) {
-  const long t = tid();
+GCS_DEV void sync_phi(const K &c, const SeamPair *pairs, int n, int both, long t) {
   if (t >= n) return;
   const SeamPair sp = pairs[t];
   for (int lv = 0; lv < (both ? 2 : 1); ++lv) {
@@ -314,8 +308,7 @@ GCS_DEV float *maxwell_plane<float>(const K &c, int d, int m) {
 
 // Same reconciliation of the fluid (5) and Maxwell (3) face fluxes.
 template <typename T>
-__global__ void k_sync_flux(K c, const SeamPair *pairs, int n) {
-  const long t = tid();
+GCS_DEV void sync_flux(const K &c, const SeamPair *pairs, int n, long t) {
   if (t >= n) return;
   const SeamPair sp = pairs[t];
   for (int q = 0; q < 8; ++q) {
@@ -331,9 +324,17 @@ __global__ void k_sync_flux(K c, const SeamPair *pairs, int n) {
 }
 
 // cubedsphere_interface.c:217-242: signed mean over each coincident group.
+// The block after the groups' ones clears the CFL slots that the update
+// folds into (null: no driver step).
 __global__ void k_sync_edges(K c, const int *groups, const EdgeMember *m,
-                             int n) {
+                             int n, unsigned long long *cfl) {
   const long g = tid();
+  if (blockIdx.x == gridDim.x - 1) {
+    if (cfl != nullptr)
+      for (int q = threadIdx.x; q < kCflSlots; q += blockDim.x)
+        cfl[q] = __double_as_longlong(DBL_MAX);
+    return;
+  }
   if (g >= n) return;
   const int a = groups[g], b = groups[g + 1];
   double common = 0.0;
@@ -373,8 +374,7 @@ GCS_DEV double block_sum(const double *plane, int donor, int sk,
 // cell B of a ghost cell (the predictor recovers B* from face fluxes, halo
 // donors and the MI shell are active cells), so without `with_b` (the
 // problem API's fidelity 0) only U is filled.
-__global__ void k_halo_cells(K c, const HaloCell *e, int n, int with_b) {
-  const long t = tid();
+GCS_DEV void halo_cell(const K &c, const HaloCell *e, int n, int with_b, long t) {
   if (t >= n) return;
   const HaloCell h = e[t];
   const int sk = c.L.SK;
@@ -407,8 +407,7 @@ __global__ void k_halo_cells(K c, const HaloCell *e, int n, int with_b) {
 // the current level, are still exact once that step's ghost phase left the
 // active B alone: with `both` = 0 (fidelity 0, Problem::old_halo_current)
 // only the current level is filled.
-__global__ void k_halo_faces(K c, const HaloFace *e, int n, int both) {
-  const long t = tid();
+GCS_DEV void halo_face(const K &c, const HaloFace *e, int n, int both, long t) {
   if (t >= n) return;
   const HaloFace h = e[t];
   const int sk = c.L.SK;
@@ -421,6 +420,50 @@ __global__ void k_halo_faces(K c, const HaloFace *e, int n, int both) {
   }
   c.p(plane_phi(c.cur, h.dir))[h.target] = cf;
   if (both) c.p(plane_phi(c.old, h.dir))[h.target] = of;
+}
+
+// The first work of a step in one launch: the dt rule (one block, driver
+// steps), the seam averages of the face flux, the tangential halo cells and
+// the ghost faces. None reads what another writes: the cells and ghost faces
+// take active cells' U and B, the averages change active faces only, and the
+// times and ratio that the dt rule sets are read from the next launch on.
+// On small grids a launch costs its latency, several us, whatever it does
+// (16 x 12^2: a step's 33 launches took 236 us; see enqueue_phase).
+struct GhostWork {
+  const SeamPair *seams;
+  const HaloCell *cells;
+  const HaloFace *faces;
+  int n_seams, n_cells, n_faces;
+  int with_b, both;
+  // dt rule: null partial for steps with a given dt
+  const unsigned long long *partial;
+  int n_partial;
+  double fraction;
+  unsigned seam_blocks, cell_blocks;
+};
+constexpr int kGhostThreads = 256;
+
+__global__ void __launch_bounds__(kGhostThreads) k_ghost_fill(K c, GhostWork g) {
+  static_assert(kGhostThreads == kCflThreads, "the dt rule's block");
+  unsigned b = blockIdx.x;
+  if (g.partial != nullptr) {
+    if (b == 0) {
+      dt_rule(c, g.fraction, g.partial, g.n_partial);
+      return;
+    }
+    --b;
+  }
+  if (b < g.cell_blocks) {
+    halo_cell(c, g.cells, g.n_cells, g.with_b, b * (long)kGhostThreads + threadIdx.x);
+    return;
+  }
+  b -= g.cell_blocks;
+  if (b < g.seam_blocks) {
+    sync_phi(c, g.seams, g.n_seams, 1, b * (long)kGhostThreads + threadIdx.x);
+    return;
+  }
+  b -= g.seam_blocks;
+  halo_face(c, g.faces, g.n_faces, g.both, b * (long)kGhostThreads + threadIdx.x);
 }
 
 // cubedsphere_halo.c:217-245 (plain problems without the Earth boundary).
@@ -635,12 +678,12 @@ __global__ void k_mi_point(MiView m, int what, double x0, double x1, double x2, 
 // ---- Earth radial boundary -------------------------------------------------
 
 // cubedsphere_earth_boundary.c:27-112: radial ghost cells of both levels.
-__global__ void k_earth_cells(K c, WindSeries w) {
+GCS_DEV void earth_cell(const K &c, const WindSeries &w, long tq) {
   const Layout &L = c.L;
   const int lo[3] = {0, 0, 0};
   const int hi[3] = {2 * L.ghost, L.NJ, L.NK};
   int f, r, j, k;
-  if (!box(tid(), lo, hi, f, r, j, k)) return;
+  if (!box(tq, lo, hi, f, r, j, k)) return;
   const bool inner = r < L.ghost;
   const int outer = L.ghost + L.nr;
   const int i = inner ? r : outer + (r - L.ghost);
@@ -713,14 +756,14 @@ __global__ void k_earth_cells(K c, WindSeries w) {
 // cubedsphere_earth_boundary.c:114-176: radial ghost faces, both levels.
 // Thread box: radial slot r < ghost is inner face r; otherwise faces beyond
 // the outer wall (r - ghost of them).
-__global__ void k_earth_faces(K c, int d, WindSeries w) {
+GCS_DEV void earth_face(const K &c, int d, const WindSeries &w, long tq) {
   const Layout &L = c.L;
   const int outer = L.ghost + L.nr;
   const int n_out = (L.NI + (d == 0)) - (outer + (d == 0));
   const int lo[3] = {0, 0, 0};
   const int hi[3] = {L.ghost + n_out, L.NJ + (d == 1), L.NK + (d == 2)};
   int f, r, j, k;
-  if (!box(tid(), lo, hi, f, r, j, k)) return;
+  if (!box(tq, lo, hi, f, r, j, k)) return;
   const bool inner = r < L.ghost;
   const int i = inner ? r : outer + (d == 0) + (r - L.ghost);
   const long t = L.at(f, i, j, k);
@@ -751,6 +794,23 @@ __global__ void k_earth_faces(K c, int d, WindSeries w) {
       flux[t] = wt * wf + (1.0 - wt) * flux[s];
     }
   }
+}
+
+// The radial ghost cells and the ghost faces of the three directions in one
+// launch: each reads elements that none of them writes.
+struct EarthWork {
+  unsigned face_blocks[3];  // blocks of the faces of each direction, then the cells
+};
+__global__ void __launch_bounds__(256) k_earth_ghosts(K c, WindSeries w, EarthWork g) {
+  unsigned b = blockIdx.x;
+  for (int d = 0; d < 3; ++d) {
+    if (b < g.face_blocks[d]) {
+      earth_face(c, d, w, b * 256L + threadIdx.x);
+      return;
+    }
+    b -= g.face_blocks[d];
+  }
+  earth_cell(c, w, b * 256L + threadIdx.x);
 }
 
 // ---- recovery ----------------------------------------------------------------
@@ -804,10 +864,10 @@ __global__ void k_recover(K c, int phi_plane, int b_plane, int inner_copy,
 }
 
 // k_recover over the cells outside the active box only.
-__global__ void k_recover_ghosts(K c, int phi_plane, int b_plane, int inner_copy) {
+GCS_DEV void recover_ghost(const K &c, int phi_plane, int b_plane, int inner_copy, long t) {
   const Layout &L = c.L;
   int f, i, j, k;
-  if (!ghost_cell(tid(), L, f, i, j, k)) return;
+  if (!ghost_cell(t, L, f, i, j, k)) return;
   const long at = L.at(f, i, j, k);
   double b[3];
   if (!recover_at(c, at, phi_plane, b)) {
@@ -819,6 +879,12 @@ __global__ void k_recover_ghosts(K c, int phi_plane, int b_plane, int inner_copy
     return;
   }
   for (int d = 0; d < 3; ++d) c.p(b_plane + d)[at] = b[d];
+}
+
+// The ghost cells of both levels (blockIdx.y: current, old).
+__global__ void k_recover_ghosts(K c, int inner_copy) {
+  const int level = blockIdx.y == 0 ? c.cur : c.old;
+  recover_ghost(c, plane_phi(level, 0), plane_b(level, 0), inner_copy, tid());
 }
 
 // Static data of the seam cells' recovery and CFL dt, gathered once per
@@ -854,9 +920,15 @@ __global__ void k_seam_geometry(K c, const int *cells, int n, double *geom) {
 // the gathered arrays (from the planes when geom is null: the plain-kernel
 // switch, which tests hold the two to). With `cfl`, the cells are the
 // current level's seam cells after the final seam sync, and their CFL dt is
-// folded into the CFL slots.
+// folded into the CFL slots. Blocks from `ghost_from` on recover the ghost
+// cells instead (fidelity).
 __global__ void k_recover_list(K c, const int *cells, const double *geom, int n, int phi_plane,
-                               int b_plane, unsigned long long *cfl) {
+                               int b_plane, unsigned long long *cfl, unsigned ghost_from) {
+  if (blockIdx.x >= ghost_from) {
+    recover_ghost(c, phi_plane, b_plane, 0,
+                  (blockIdx.x - ghost_from) * (long)blockDim.x + threadIdx.x);
+    return;
+  }
   const long t = tid();
   double dt_cell = DBL_MAX;
   if (t < n) {
@@ -1551,12 +1623,12 @@ __global__ void __launch_bounds__(256) k_edge_emf_tiled(K c) {
 
 // nonorthogonal_step.c:35-71 on the inner wall face.
 template <typename T>
-__global__ void k_inner_trap(K c) {
+GCS_DEV void inner_trap(const K &c, long t) {
   const Layout &L = c.L;
   const int lo[3] = {L.ghost, L.ghost, L.ghost};
   const int hi[3] = {L.ghost + 1, L.ghost + L.n, L.ghost + L.n};
   int f, i, j, k;
-  if (!box(tid(), lo, hi, f, i, j, k)) return;
+  if (!box(t, lo, hi, f, i, j, k)) return;
   const long at = L.at(f, i, j, k);
   T *m = fluid_plane<T>(c, 0, 0) + at;
   T *e = fluid_plane<T>(c, 0, 4) + at;
@@ -1564,6 +1636,16 @@ __global__ void k_inner_trap(K c) {
     *m = T(0);
     if (*e > T(0)) *e = T(0);
   }
+}
+
+// The seam averages of the face fluxes (j- and k-faces) and the inner wall's
+// trap (i-faces, blocks from trap_from on) in one launch.
+template <typename T>
+__global__ void k_finish_flux(K c, const SeamPair *pairs, int n, unsigned trap_from) {
+  if (blockIdx.x < trap_from)
+    sync_flux<T>(c, pairs, n, tid());
+  else
+    inner_trap<T>(c, (blockIdx.x - trap_from) * (long)blockDim.x + threadIdx.x);
 }
 
 // ---- edge EMF --------------------------------------------------------------------
@@ -2026,103 +2108,95 @@ __global__ void __launch_bounds__(128) k_edge_emf_fp32(K c, int e) {
   c.p(P_EMF + e)[at] = (double)emf;
 }
 
-// cubedsphere_earth_boundary.c:445-489: outer shells blend toward the wind
-// line integral -(V x B) . l.
-__global__ void k_earth_emf_outer(K c, int d, WindSeries w) {
+// The Earth boundary's three EMF stages, one thread per edge position (i, j,
+// k) of the shells they touch, for its edges of the three directions in the
+// stages' order: each edge is changed by its own position's thread only, so
+// the stages need no launch of their own. Radial slots 0-3 are the shells
+// outer - 3 .. outer, slot 4 the inner wall where it is none of them.
+//  * cubedsphere_earth_boundary.c:445-489: outer shells blend toward the wind
+//    line integral -(V x B) . l;
+//  * :362-443: diffusive wind EMF on the outer wall;
+//  * :429-440: E_t = 0 on the inner wall shell, or with the ionosphere ready,
+//    -(potential difference) / potential norm along each wall edge
+//    (cubedsphere_mi_dipole.c:478-503).
+__global__ void __launch_bounds__(256) k_earth_emf(K c, WindSeries w) {
   const Layout &L = c.L;
   const int outer = L.ghost + L.nr;
-  const int lo[3] = {outer - 3, 0, 0};
-  const int hi[3] = {min(outer + 1, L.NI + (d != 0)), L.NJ + (d != 1), L.NK + (d != 2)};
-  int f, i, j, k;
-  if (!box(tid(), lo, hi, f, i, j, k)) return;
+  const int lo[3] = {0, 0, 0}, hi[3] = {5, L.NJ + 1, L.NK + 1};
+  int f, slot, j, k;
+  if (!box(tid(), lo, hi, f, slot, j, k)) return;
+  if (slot == 4 && L.ghost >= outer - 3) return;
+  const int i = slot == 4 ? L.ghost : outer - 3 + slot;
   const long at = L.at(f, i, j, k);
-  if (!c.b(Q_VALID + d)[at]) return;
-  const long up = at + (d == 0 ? L.di() : d == 1 ? (long)L.SK : 1);
-  double x[3];
-  for (int m = 0; m < 3; ++m) x[m] = 0.5 * (c.p(P_VERT + m)[at] + c.p(P_VERT + m)[up]);
-  double sw[8], wt;
-  if (!sample_wind(w, x, c.sc->wall_time + 0.5 * c.sc->wall_dt, sw, wt)) {
-    c.fail(61, at);
-    return;
+  const long step[3] = {L.di(), (long)L.SK, 1};
+  bool ok[3];
+  for (int d = 0; d < 3; ++d)
+    ok[d] = i < L.NI + (d != 0) && j < L.NJ + (d != 1) && k < L.NK + (d != 2) &&
+            c.b(Q_VALID + d)[at];
+  double sw[3][8], wt[3];
+  if (i >= outer - 3) {
+    for (int d = 0; d < 3; ++d) {
+      if (!ok[d]) continue;
+      double x[3];
+      for (int m = 0; m < 3; ++m)
+        x[m] = 0.5 * (c.p(P_VERT + m)[at] + c.p(P_VERT + m)[at + step[d]]);
+      if (!sample_wind(w, x, c.sc->wall_time + 0.5 * c.sc->wall_dt, sw[d], wt[d])) {
+        c.fail(61, at);
+        return;
+      }
+      double weight = wt[d];
+      if (i < outer) weight /= 1.0 + (double)(outer - i);
+      const double *vv = sw[d] + 2, *bb = sw[d] + 5;
+      const double el[3] = {-(vv[1] * bb[2] - vv[2] * bb[1]), -(vv[2] * bb[0] - vv[0] * bb[2]),
+                            -(vv[0] * bb[1] - vv[1] * bb[0])};
+      const int eb = P_EDGE + EDGE_PLANES * d;
+      const double len = c.p(eb + EO_LEN)[at];
+      double line = 0.0;
+      for (int m = 0; m < 3; ++m) line += el[m] * c.p(eb + EO_N + m)[at] * len;
+      double *emf = c.p(P_EMF + d) + at;
+      *emf = (1.0 - weight) * *emf + weight * line;
+    }
   }
-  if (i < outer) wt /= 1.0 + (double)(outer - i);
-  const double *vv = sw + 2, *bb = sw + 5;
-  const double el[3] = {-(vv[1] * bb[2] - vv[2] * bb[1]), -(vv[2] * bb[0] - vv[0] * bb[2]),
-                        -(vv[0] * bb[1] - vv[1] * bb[0])};
-  const int eb = P_EDGE + EDGE_PLANES * d;
-  const double len = c.p(eb + EO_LEN)[at];
-  double line = 0.0;
-  for (int m = 0; m < 3; ++m) line += el[m] * c.p(eb + EO_N + m)[at] * len;
-  double *emf = c.p(P_EMF + d) + at;
-  *emf = (1.0 - wt) * *emf + wt * line;
-}
-
-// cubedsphere_earth_boundary.c:362-443: diffusive wind EMF on the outer wall.
-__global__ void k_earth_emf_diffusive(K c, WindSeries w) {
-  const Layout &L = c.L;
-  const int i = L.ghost + L.nr;
-  const int lo[3] = {i, L.ghost, L.ghost};
-  const int hi[3] = {i + 1, L.ghost + L.n + 1, L.ghost + L.n + 1};
-  int f, ii, j, k;
-  if (!box(tid(), lo, hi, f, ii, j, k)) return;
-  // Edge extents: J (NI+1, NJ, NK+1), K (NI+1, NJ+1, NK).
-  if (j == 0 || k == 0 || j >= L.NJ || k >= L.NK) return;
-  const long at = L.at(f, i, j, k);
-  if (!c.b(Q_VALID + 1)[at] || !c.b(Q_VALID + 2)[at]) return;
-  const long si = L.di(), sj = L.SK;
-  auto dens = [&](int dir, long fa, double &out) {
-    const double area = c.p(P_FACE + FACE_PLANES * dir + FO_AREA)[fa];
-    if (!(area > 0.0)) return false;
-    const double cf = c.p(plane_phi(c.cur, dir))[fa], of = c.p(plane_phi(c.old, dir))[fa];
-    out = (cf + c.sc->ratio * (cf - of)) / area;  // the predictor's Phi*
-    return (bool)isfinite(out);
-  };
-  double bikp, bikm, bkip, bkim, bjip, bjim, bijp, bijm;
-  if (!dens(0, at, bikp) || !dens(0, at - 1, bikm) || !dens(2, at, bkip) ||
-      !dens(2, at - si, bkim) || !dens(1, at, bjip) || !dens(1, at - si, bjim) ||
-      !dens(0, at, bijp) || !dens(0, at - sj, bijm)) {
-    c.fail(62, at);
-    return;
+  // Edge extents: J (NI+1, NJ, NK+1), K (NI+1, NJ+1, NK). The wind samples of
+  // the two edges are those of the blend above.
+  if (i == outer && j >= L.ghost && j <= L.ghost + L.n && k >= L.ghost && k <= L.ghost + L.n &&
+      ok[1] && ok[2]) {
+    const long si = step[0], sj = step[1];
+    auto dens = [&](int dir, long fa, double &out) {
+      const double area = c.p(P_FACE + FACE_PLANES * dir + FO_AREA)[fa];
+      if (!(area > 0.0)) return false;
+      const double cf = c.p(plane_phi(c.cur, dir))[fa], of = c.p(plane_phi(c.old, dir))[fa];
+      out = (cf + c.sc->ratio * (cf - of)) / area;  // the predictor's Phi*
+      return (bool)isfinite(out);
+    };
+    double bikp, bikm, bkip, bkim, bjip, bjim, bijp, bijm;
+    if (!dens(0, at, bikp) || !dens(0, at - 1, bikm) || !dens(2, at, bkip) ||
+        !dens(2, at - si, bkim) || !dens(1, at, bjip) || !dens(1, at - si, bjim) ||
+        !dens(0, at, bijp) || !dens(0, at - sj, bijm)) {
+      c.fail(62, at);
+      return;
+    }
+    const double cj = (bikp - bikm) - (bkip - bkim);
+    const double ck = (bjip - bjim) - (bijp - bijm);
+    const double dl = sqrt(c.p(P_EDGE + EDGE_PLANES * 1 + EO_LEN)[at] *
+                           c.p(P_EDGE + EDGE_PLANES * 2 + EO_LEN)[at]);
+    if (!(dl > 0.0)) {
+      c.fail(63, at);
+      return;
+    }
+    const double c2 = w.by * w.by + w.bz * w.bz;
+    const double front = fmax(fabs(sw[1][2]), fabs(sw[2][2])) / sqrt(1.0 + c2);
+    const double speed = fmin(front, c.o.wall_cfl * dl / c.sc->wall_dt);
+    c.p(P_EMF + 1)[at] += wt[1] * speed * cj * dl;
+    c.p(P_EMF + 2)[at] += wt[2] * speed * ck * dl;
   }
-  const double cj = (bikp - bikm) - (bkip - bkim);
-  const double ck = (bjip - bjim) - (bijp - bijm);
-  const double dl = sqrt(c.p(P_EDGE + EDGE_PLANES * 1 + EO_LEN)[at] *
-                         c.p(P_EDGE + EDGE_PLANES * 2 + EO_LEN)[at]);
-  double xj[3], xk[3];
-  for (int m = 0; m < 3; ++m) {
-    xj[m] = 0.5 * (c.p(P_VERT + m)[at] + c.p(P_VERT + m)[at + sj]);
-    xk[m] = 0.5 * (c.p(P_VERT + m)[at] + c.p(P_VERT + m)[at + 1]);
-  }
-  const double t = c.sc->wall_time + 0.5 * c.sc->wall_dt;
-  double wj[8], wk[8], gj, gk;
-  if (!(dl > 0.0) || !sample_wind(w, xj, t, wj, gj) || !sample_wind(w, xk, t, wk, gk)) {
-    c.fail(63, at);
-    return;
-  }
-  const double c2 = w.by * w.by + w.bz * w.bz;
-  const double front = fmax(fabs(wj[2]), fabs(wk[2])) / sqrt(1.0 + c2);
-  const double speed = fmin(front, c.o.wall_cfl * dl / c.sc->wall_dt);
-  c.p(P_EMF + 1)[at] += gj * speed * cj * dl;
-  c.p(P_EMF + 2)[at] += gk * speed * ck * dl;
-}
-
-// cubedsphere_earth_boundary.c:429-440: E_t = 0 on the inner wall shell, or
-// with the ionosphere ready, -(potential difference) / potential norm along
-// each wall edge (cubedsphere_mi_dipole.c:478-503).
-__global__ void k_earth_emf_inner(K c) {
-  const Layout &L = c.L;
-  const int lo[3] = {L.ghost, 0, 0};
-  const int hi[3] = {L.ghost + 1, L.NJ + 1, L.NK + 1};
-  int f, i, j, k;
-  if (!box(tid(), lo, hi, f, i, j, k)) return;
-  const long at = L.at(f, i, j, k);
+  if (i != L.ghost) return;
   // J edges span (NI+1, NJ, NK+1), K edges (NI+1, NJ+1, NK).
   for (int d = 1; d <= 2; ++d) {
-    if ((d == 1 && j >= L.NJ) || (d == 2 && k >= L.NK) || !c.b(Q_VALID + d)[at])
-      continue;
+    if (!ok[d]) continue;
     double emf = 0.0;
     if (c.mi.potential != nullptr) {
-      const long end = at + (d == 1 ? (long)L.SK : 1L);
+      const long end = at + step[d];
       const double a[3] = {c.p(P_VERT)[at], c.p(P_VERT + 1)[at], c.p(P_VERT + 2)[at]};
       const double b[3] = {c.p(P_VERT)[end], c.p(P_VERT + 1)[end], c.p(P_VERT + 2)[end]};
       double pa, pb;
@@ -2272,12 +2346,12 @@ __global__ void __launch_bounds__(128) k_update(K c, unsigned long long *cfl) {
 // Ghost values of the new level as the reference leaves them in storage:
 // ghost U and ghost face fluxes keep the step's start values (the reference
 // copies current into old before updating only active elements).
-__global__ void k_keep_ghosts(K c) {
+GCS_DEV void keep_ghosts(const K &c, long t) {
   const Layout &L = c.L;
   const int lo[3] = {0, 0, 0};
   const int hi[3] = {L.NI + 1, L.NJ + 1, L.NK + 1};
   int f, i, j, k;
-  if (!box(tid(), lo, hi, f, i, j, k)) return;
+  if (!box(t, lo, hi, f, i, j, k)) return;
   const long at = L.at(f, i, j, k);
   const int g = L.ghost;
   const bool ai = i >= g && i < g + L.nr, aj = j >= g && j < g + L.n,
@@ -2296,6 +2370,24 @@ __global__ void k_keep_ghosts(K c) {
                         i < L.NI && j < L.NJ && k <= L.NK && !(ai && aj && fk)};
   for (int d = 0; d < 3; ++d)
     if (face[d]) c.p(plane_phi(c.old, d))[at] = c.p(plane_phi(c.cur, d))[at];
+}
+
+// After the update, in one launch: the final seam average of the new face
+// flux (blocks below keep_from), the kept ghost values (blocks from there on,
+// with fidelity) and the clock (the first thread of a driver step). The
+// averages change active faces of the new level, the copies its ghost
+// elements, and nothing of the step reads the clock after the update.
+__global__ void __launch_bounds__(256) k_finish_step(K c, const SeamPair *pairs, int n,
+                                                     unsigned keep_from, int clock) {
+  if (clock && blockIdx.x == 0 && threadIdx.x == 0) advance_clock(c);
+  if (blockIdx.x < keep_from) {
+    K next = c;
+    next.cur = c.old;
+    next.old = c.cur;
+    sync_phi(next, pairs, n, 0, tid());
+  } else {
+    keep_ghosts(c, (blockIdx.x - keep_from) * 256L + threadIdx.x);
+  }
 }
 
 }  // namespace
@@ -2432,7 +2524,10 @@ void mark_stage(Problem &P, int stage) {
   ++P.stage_cursor;
 }
 
-int enqueue_phase(Problem &P, Phase phase) {
+// Kernels that need nothing of each other share a launch: on small grids a
+// step is the sum of its launches' latencies, 5-13 us each (16 x 12^2 cells a
+// face, default options: 33 launches, 236 us a step; 48 x 24^2: 462 us).
+int enqueue_phase(Problem &P, Phase phase, bool driver) {
   K c = make_k(P);
   const Layout &L = P.L;
   hipStream_t s = P.stream;
@@ -2445,41 +2540,62 @@ int enqueue_phase(Problem &P, Phase phase) {
 
   if (phase == PHASE_GHOSTS) {
     // cubedsphere_step.c:51-65
-    mark_stage(P, S_SYNC_PHI);
-    k_sync_phi<<<nblocks(P.n_seams, T), T, 0, s>>>(c, P.seams, P.n_seams, 1);
+    GhostWork g;
+    g.seams = P.seams;
+    g.cells = P.halo_cells;
+    g.faces = P.halo_faces;
+    g.n_seams = P.n_seams;
+    g.n_cells = P.n_halo_cells;
+    g.n_faces = P.n_halo_faces;
+    g.with_b = P.fidelity ? 1 : 0;
+    g.both = (P.fidelity || !P.old_halo_current) ? 1 : 0;
+    g.partial = nullptr;
+    g.n_partial = 0;
+    g.fraction = P.cfg.dt_fraction;
+    if (driver && P.cfl_folded) {
+      // the previous step's update folded this state's CFL dt
+      g.partial = P.cfl_slots;
+      g.n_partial = kCflSlots;
+    } else if (driver) {
+      mark_stage(P, S_CFL);
+      g.partial = P.cfl_partial;
+      g.n_partial = (int)nblocks(n_active, kCflThreads);
+      k_cfl<<<g.n_partial, kCflThreads, 0, s>>>(c, P.cfl_partial);
+    }
+    g.seam_blocks = nblocks(g.n_seams, kGhostThreads);
+    g.cell_blocks = nblocks(g.n_cells, kGhostThreads);
     mark_stage(P, S_HALO_CELLS);
-    k_halo_cells<<<nblocks(P.n_halo_cells, T), T, 0, s>>>(c, P.halo_cells, P.n_halo_cells,
-                                                         P.fidelity ? 1 : 0);
+    k_ghost_fill<<<(g.partial != nullptr ? 1u : 0u) + g.seam_blocks + g.cell_blocks +
+                       nblocks(g.n_faces, kGhostThreads),
+                   kGhostThreads, 0, s>>>(c, g);
     if (bd.outflow) {
       mark_stage(P, S_OUTFLOW);
       k_radial_outflow<<<nblocks(6L * 2 * L.ghost * L.NJ * L.NK, T), T, 0, s>>>(c);
     }
-    mark_stage(P, S_HALO_FACES);
-    k_halo_faces<<<nblocks(P.n_halo_faces, T), T, 0, s>>>(
-        c, P.halo_faces, P.n_halo_faces, (P.fidelity || !P.old_halo_current) ? 1 : 0);
     if (bd.earth_cells) {
       mark_stage(P, S_EARTH_CELLS);
-      k_earth_cells<<<nblocks(6L * 2 * L.ghost * L.NJ * L.NK, T), T, 0, s>>>(c, w);
-      mark_stage(P, S_EARTH_FACES);
+      EarthWork e;
+      unsigned blocks = nblocks(6L * 2 * L.ghost * L.NJ * L.NK, T);
       for (int d = 0; d < 3; ++d) {
         const long n_out = (L.NI + (d == 0)) - (L.ghost + L.nr + (d == 0));
-        const long n = 6L * (L.ghost + n_out) * (L.NJ + (d == 1)) * (L.NK + (d == 2));
-        k_earth_faces<<<nblocks(n, T), T, 0, s>>>(c, d, w);
+        e.face_blocks[d] =
+            nblocks(6L * (L.ghost + n_out) * (L.NJ + (d == 1)) * (L.NK + (d == 2)), T);
+        blocks += e.face_blocks[d];
       }
+      k_earth_ghosts<<<blocks, T, 0, s>>>(c, w, e);
       mark_stage(P, S_EARTH_RECOVER);
       // cubedsphere_earth_boundary.c:169 recovers every cell of both levels.
       // After a completed step the six face fluxes of an active cell are
       // those its B was last recovered from (the step ends with the seam
       // sync and a recovery), so only the non-active cells change; and
-      // ghost-cell B is never read by the step (see k_halo_cells), so with
+      // ghost-cell B is never read by the step (see halo_cell), so with
       // fidelity 0 only the first step's recovery of every cell runs.
-      for (int lev : {c.cur, c.old}) {
-        if (!P.b_recovered)
+      if (!P.b_recovered) {
+        for (int lev : {c.cur, c.old})
           k_recover<<<nblocks(n_cells, T), T, 0, s>>>(c, plane_phi(lev, 0), plane_b(lev, 0), 1,
                                                       0);
-        else if (P.fidelity)
-          k_recover_ghosts<<<nblocks(n_cells - n_active, T), T, 0, s>>>(c, plane_phi(lev, 0),
-                                                                        plane_b(lev, 0), 1);
+      } else if (P.fidelity) {
+        k_recover_ghosts<<<dim3(nblocks(n_cells - n_active, T), 2), T, 0, s>>>(c, 1);
       }
     }
   } else if (phase == PHASE_FLUX) {
@@ -2510,17 +2626,12 @@ int enqueue_phase(Problem &P, Phase phase) {
         k_face_flux<<<nblocks(n, 128), 128, 0, s>>>(c, d);
     }
     mark_stage(P, S_SYNC_FLUX);
+    const unsigned trap_from = nblocks(P.n_seams, T);
+    const unsigned blocks = trap_from + (bd.inner_trap ? nblocks(6L * L.n * L.n, T) : 0u);
     if (P.mixed)
-      k_sync_flux<float><<<nblocks(P.n_seams, T), T, 0, s>>>(c, P.seams, P.n_seams);
+      k_finish_flux<float><<<blocks, T, 0, s>>>(c, P.seams, P.n_seams, trap_from);
     else
-      k_sync_flux<double><<<nblocks(P.n_seams, T), T, 0, s>>>(c, P.seams, P.n_seams);
-    if (bd.inner_trap) {
-      mark_stage(P, S_INNER_TRAP);
-      if (P.mixed)
-        k_inner_trap<float><<<nblocks(6L * L.n * L.n, T), T, 0, s>>>(c);
-      else
-        k_inner_trap<double><<<nblocks(6L * L.n * L.n, T), T, 0, s>>>(c);
-    }
+      k_finish_flux<double><<<blocks, T, 0, s>>>(c, P.seams, P.n_seams, trap_from);
   } else if (phase == PHASE_EMF) {
     // cubedsphere_step.c:99-126 up to the seam EMF average; a hydrodynamic
     // step has no EMF
@@ -2567,27 +2678,20 @@ int enqueue_phase(Problem &P, Phase phase) {
     }
     if (bd.earth_emf) {
       mark_stage(P, S_EARTH_EMF);
-      for (int d = 0; d < 3; ++d) {
-        const int outer = L.ghost + L.nr;
-        const long n = 6L * (std::min(outer + 1, L.NI + (d != 0)) - (outer - 3)) *
-                       (L.NJ + (d != 1)) * (L.NK + (d != 2));
-        k_earth_emf_outer<<<nblocks(n, T), T, 0, s>>>(c, d, w);
-      }
-      k_earth_emf_diffusive<<<nblocks(6L * (L.n + 1) * (L.n + 1), T), T, 0, s>>>(c, w);
-      k_earth_emf_inner<<<nblocks(6L * (L.NJ + 1) * (L.NK + 1), T), T, 0, s>>>(c);
+      k_earth_emf<<<nblocks(6L * 5 * (L.NJ + 1) * (L.NK + 1), T), T, 0, s>>>(c, w);
     }
   } else {
     // cubedsphere_step.c:125-152
-    if (P.opt.mhd) {
-      mark_stage(P, S_SYNC_EDGES);
-      k_sync_edges<<<nblocks(P.n_edge_groups, T), T, 0, s>>>(c, P.edge_groups, P.edge_members,
-                                                             P.n_edge_groups);
-    }
-    mark_stage(P, S_UPDATE);
     // A driver step folds the new state's CFL dt into the slots that the
     // next step's dt rule reads (its seam cells after the final sync).
     unsigned long long *cfl = P.driver_cfl ? P.cfl_slots : nullptr;
-    if (cfl != nullptr) k_cfl_reset<<<1, kCflSlots, 0, s>>>(cfl);
+    const int edge_groups = P.opt.mhd ? P.n_edge_groups : 0;
+    if (edge_groups > 0 || cfl != nullptr) {
+      mark_stage(P, S_SYNC_EDGES);
+      k_sync_edges<<<nblocks(edge_groups, T) + 1, T, 0, s>>>(c, P.edge_groups, P.edge_members,
+                                                             edge_groups, cfl);
+    }
+    mark_stage(P, S_UPDATE);
     if (P.mixed)
       k_update<true><<<nblocks(n_active, 128), 128, 0, s>>>(c, cfl);
     else
@@ -2597,20 +2701,23 @@ int enqueue_phase(Problem &P, Phase phase) {
     K n = c;
     n.cur = c.old;
     n.old = c.cur;
+    const unsigned sync_blocks = P.opt.mhd ? nblocks(P.n_seams, T) : 0u;
+    const unsigned finish = sync_blocks + (P.fidelity ? nblocks(n_box, T) : 0u);
+    mark_stage(P, S_FINAL_SYNC);
+    if (finish > 0 || driver)
+      k_finish_step<<<std::max(finish, 1u), T, 0, s>>>(c, P.seams, P.opt.mhd ? P.n_seams : 0,
+                                                       P.fidelity ? sync_blocks
+                                                                  : std::max(sync_blocks, 1u),
+                                                       driver ? 1 : 0);
     if (P.opt.mhd) {
-      mark_stage(P, S_FINAL_SYNC);
-      k_sync_phi<<<nblocks(P.n_seams, T), T, 0, s>>>(n, P.seams, P.n_seams, 0);
       mark_stage(P, S_SEAM_RECOVER);
-      k_recover_list<<<nblocks(P.n_seam_cells, T), T, 0, s>>>(
-          n, P.seam_cells, P.plain ? nullptr : P.seam_geom, P.n_seam_cells, plane_phi(n.cur, 0),
-          plane_b(n.cur, 0), cfl);
-    }
-    if (P.fidelity) {
-      mark_stage(P, S_FIDELITY);
-      k_keep_ghosts<<<nblocks(n_box, T), T, 0, s>>>(c);
-      if (P.opt.mhd)
-        k_recover_ghosts<<<nblocks(n_cells - n_active, T), T, 0, s>>>(n, plane_phi(n.cur, 0),
-                                                                      plane_b(n.cur, 0), 0);
+      const unsigned seam_blocks = nblocks(P.n_seam_cells, T);
+      const unsigned recover =
+          seam_blocks + (P.fidelity ? nblocks(n_cells - n_active, T) : 0u);
+      if (recover > 0)
+        k_recover_list<<<recover, T, 0, s>>>(n, P.seam_cells, P.plain ? nullptr : P.seam_geom,
+                                             P.n_seam_cells, plane_phi(n.cur, 0),
+                                             plane_b(n.cur, 0), cfl, seam_blocks);
     }
     P.level = 1 - P.level;
     P.host_dirty = true;
@@ -3270,29 +3377,8 @@ int enqueue_step(Problem &P, bool explicit_dt) {
     return -1;
   }
   P.last_step_mixed = P.mixed;
-  K c = make_k(P);
-  const Layout &L = P.L;
-  hipStream_t s = P.stream;
-  const long n_active = 6L * L.nr * L.n * L.n;
-  if (!explicit_dt) {
-    if (P.cfl_folded) {
-      // the previous step's update folded this state's CFL dt
-      mark_stage(P, S_DT);
-      k_dt<<<1, kCflThreads, 0, s>>>(c, P.cfg.dt_fraction, P.cfl_slots, kCflSlots);
-    } else {
-      mark_stage(P, S_CFL);
-      const int ncfl = (int)nblocks(n_active, kCflThreads);
-      k_cfl<<<ncfl, kCflThreads, 0, s>>>(c, P.cfl_partial);
-      mark_stage(P, S_DT);
-      k_dt<<<1, kCflThreads, 0, s>>>(c, P.cfg.dt_fraction, P.cfl_partial, ncfl);
-    }
-  }
   for (Phase ph : {PHASE_GHOSTS, PHASE_FLUX, PHASE_EMF, PHASE_UPDATE})
-    if (enqueue_phase(P, ph) != 0) return -1;
-  if (!explicit_dt) {
-    mark_stage(P, S_CLOCK);
-    k_clock<<<1, 1, 0, s>>>(c);
-  }
+    if (enqueue_phase(P, ph, !explicit_dt) != 0) return -1;
   mark_stage(P, S_END);
   GCS_HIP(hipGetLastError());
   return 0;
