@@ -372,8 +372,9 @@ int upload_wind(Problem &P, int count, const double *time, const double *state);
 int pressure_control_noalloc(Problem &P, const double args[7], unsigned long long counts[2],
                              double maxima[2]);
 // With `driver` the first phase also runs the dt rule and the last one
-// advances the clock (enqueue_step of a driver step).
-int enqueue_phase(Problem &P, Phase phase, bool driver = false);
+// advances the clock (enqueue_step of a driver step); `whole`: the four
+// phases follow each other directly, with no host work between them.
+int enqueue_phase(Problem &P, Phase phase, bool driver = false, bool whole = false);
 // Constants derived from uploaded geometry and background: recovery
 // pivots, edge-B solve, B0 normal and edge-tangential components.
 int derive_constants(Problem &P);

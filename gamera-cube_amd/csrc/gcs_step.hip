@@ -138,11 +138,11 @@ GCS_DEV long tid() { return blockIdx.x * (long)blockDim.x + threadIdx.x; }
 // stencil neighbours of a block in the same L2. (A bijection of [0, nb).)
 // Used by the face-velocity and edge-EMF sweeps, whose 8-point stencils
 // reach across k-rows; plan-driven kernels keep the plain order.
-GCS_DEV unsigned block_xcd() {
-  const unsigned nb = gridDim.x, b = blockIdx.x;
+GCS_DEV unsigned block_xcd(unsigned b, unsigned nb) {
   const unsigned q = nb >> 3, r = nb & 7, x = b & 7, slot = b >> 3;
   return x * q + min(x, r) + slot;
 }
+GCS_DEV unsigned block_xcd() { return block_xcd(blockIdx.x, gridDim.x); }
 GCS_DEV long tid_xcd() { return block_xcd() * (long)blockDim.x + threadIdx.x; }
 
 constexpr int kCflThreads = 256;
@@ -311,15 +311,22 @@ template <typename T>
 GCS_DEV void sync_flux(const K &c, const SeamPair *pairs, int n, long t) {
   if (t >= n) return;
   const SeamPair sp = pairs[t];
+  // every load before the first store (the planes may alias for the compiler;
+  // interleaved, eight memory latencies followed each other: 22 us at 24^2)
+  T *a[8], *b[8], av[8], bv[8];
   for (int q = 0; q < 8; ++q) {
-    T *a = q < 5 ? fluid_plane<T>(c, sp.dir_a, q) + sp.a
+    a[q] = q < 5 ? fluid_plane<T>(c, sp.dir_a, q) + sp.a
                  : maxwell_plane<T>(c, sp.dir_a, q - 5) + sp.a;
-    T *b = q < 5 ? fluid_plane<T>(c, sp.dir_b, q) + sp.b
+    b[q] = q < 5 ? fluid_plane<T>(c, sp.dir_b, q) + sp.b
                  : maxwell_plane<T>(c, sp.dir_b, q - 5) + sp.b;
-    const T sign = (T)sp.sign;
-    const T common = T(0.5) * (*a + sign * *b);
-    *a = common;
-    *b = sign * common;
+    av[q] = *a[q];
+    bv[q] = *b[q];
+  }
+  const T sign = (T)sp.sign;
+  for (int q = 0; q < 8; ++q) {
+    const T common = T(0.5) * (av[q] + sign * bv[q]);
+    *a[q] = common;
+    *b[q] = sign * common;
   }
 }
 
@@ -383,21 +390,35 @@ GCS_DEV void halo_cell(const K &c, const HaloCell *e, int n, int with_b, long t)
     cu[q] = block_sum(c.p(plane_u(c.cur, q)), h.donor, sk, h.w);
     ou[q] = block_sum(c.p(plane_u(c.old, q)), h.donor, sk, h.w);
   }
-  // Nearest-donor fallback when either interpolated level is non-physical.
+  double cb[3] = {0.0, 0.0, 0.0}, ob[3] = {0.0, 0.0, 0.0};
+  if (with_b)
+    for (int d = 0; d < 3; ++d) {
+      cb[d] = block_sum(c.p(plane_b(c.cur, d)), h.donor, sk, h.w);
+      ob[d] = block_sum(c.p(plane_b(c.old, d)), h.donor, sk, h.w);
+    }
+  // Nearest-donor fallback when either interpolated level is non-physical;
+  // read only then, and before the first store, which no load may pass.
   const bool ok = halo_valid(cu) & halo_valid(ou);
-  const int src = h.nearest;
+  if (!ok) {
+    const int src = h.nearest;
+    for (int q = 0; q < 5; ++q) {
+      cu[q] = c.p(plane_u(c.cur, q))[src];
+      ou[q] = c.p(plane_u(c.old, q))[src];
+    }
+    if (with_b)
+      for (int d = 0; d < 3; ++d) {
+        cb[d] = c.p(plane_b(c.cur, d))[src];
+        ob[d] = c.p(plane_b(c.old, d))[src];
+      }
+  }
   for (int q = 0; q < 5; ++q) {
-    const double nc = c.p(plane_u(c.cur, q))[src], no = c.p(plane_u(c.old, q))[src];
-    c.p(plane_u(c.cur, q))[h.target] = ok ? cu[q] : nc;
-    c.p(plane_u(c.old, q))[h.target] = ok ? ou[q] : no;
+    c.p(plane_u(c.cur, q))[h.target] = cu[q];
+    c.p(plane_u(c.old, q))[h.target] = ou[q];
   }
   if (!with_b) return;
   for (int d = 0; d < 3; ++d) {
-    const double cb = block_sum(c.p(plane_b(c.cur, d)), h.donor, sk, h.w);
-    const double ob = block_sum(c.p(plane_b(c.old, d)), h.donor, sk, h.w);
-    const double nc = c.p(plane_b(c.cur, d))[src], no = c.p(plane_b(c.old, d))[src];
-    c.p(plane_b(c.cur, d))[h.target] = ok ? cb : nc;
-    c.p(plane_b(c.old, d))[h.target] = ok ? ob : no;
+    c.p(plane_b(c.cur, d))[h.target] = cb[d];
+    c.p(plane_b(c.old, d))[h.target] = ob[d];
   }
 }
 
@@ -428,7 +449,8 @@ GCS_DEV void halo_face(const K &c, const HaloFace *e, int n, int both, long t) {
 // take active cells' U and B, the averages change active faces only, and the
 // times and ratio that the dt rule sets are read from the next launch on.
 // On small grids a launch costs its latency, several us, whatever it does
-// (16 x 12^2: a step's 33 launches took 236 us; see enqueue_phase).
+// (16 x 12^2: a step's 33 launches took 236 us, its 12 take 105; see
+// enqueue_phase).
 struct GhostWork {
   const SeamPair *seams;
   const HaloCell *cells;
@@ -1222,13 +1244,13 @@ GCS_DEV void face_flux_face(const K &c, int d, int f, long at, long st, const Ce
 
 // The face flux with the stencil read from global memory (one face per
 // thread, 72 stencil loads per face).
-__global__ void __launch_bounds__(128) k_face_flux(K c, int d) {
+GCS_DEV void flux_plain(const K &c, int d, long tq) {
   const Layout &L = c.L;
   const int lo[3] = {L.ghost, L.ghost, L.ghost};
   const int hi[3] = {L.ghost + L.nr + (d == 0), L.ghost + L.n + (d == 1),
                      L.ghost + L.n + (d == 2)};
   int f, i, j, k;
-  if (!box(tid(), lo, hi, f, i, j, k)) return;
+  if (!box(tq, lo, hi, f, i, j, k)) return;
   const long at = L.at(f, i, j, k);
   const long st = d == 0 ? L.di() : d == 1 ? (long)L.SK : 1;
   face_flux_face(c, d, f, at, st, [&](int v, int n) {
@@ -1236,6 +1258,7 @@ __global__ void __launch_bounds__(128) k_face_flux(K c, int d) {
     return c.p(plane)[at + (n - 4) * st];
   });
 }
+__global__ void __launch_bounds__(128) k_face_flux(K c, int d) { flux_plain(c, d, tid()); }
 
 // LDS tiles of the face flux of direction D: TD faces along D by TT along a
 // transverse axis (k, or j for D = 2) at one position of the third axis.
@@ -1256,6 +1279,7 @@ struct FluxTile {
   // lanes of a wave read consecutive slots.
   GCS_DEV static int slot(int cd, int t) { return D == 2 ? t * CD + cd : cd * TT + t; }
   static constexpr int kStep = D == 2 ? 1 : TT;   // slot step along D
+  static constexpr int kLds = kVars * kSlots;     // doubles
   // blocks for a layout with nr radial and n angular active cells
   static unsigned blocks(int nr, int n) {
     const int act[3] = {nr, n, n};
@@ -1266,26 +1290,25 @@ struct FluxTile {
 // Four waves per SIMD: unbounded, the kernel takes 129 VGPRs and runs three;
 // bounded, it spills 8 registers a lane (0.89 / 0.91 -> 0.81 / 0.83 ms at
 // config 1; k_face_flux_rows likewise, 0.97 -> 0.90 ms).
-template <int D, int TD_, int TT_>
-__global__ void __launch_bounds__(TD_ * TT_, 4) k_face_flux_tiled(K c) {
-  using T = FluxTile<D, TD_, TT_>;
+// One tile (logical block b, tid of its T::kThreads threads, T::kLds doubles of
+// LDS); tiles beyond the last do nothing but pass the barrier.
+template <class T, int D>
+GCS_DEV void flux_tile(const K &c, unsigned b, int tid, double *s_cell) {
   constexpr int TD = T::TD, TT = T::TT, CD = T::CD, TA = T::TA, XA = T::XA;
   constexpr int kSlots = T::kSlots;
-  __shared__ double s_cell[T::kVars * kSlots];
   const Layout &L = c.L;
   const int act[3] = {L.nr, L.n, L.n};
   const int nd = act[D] + 1, nt = act[TA], nx = act[XA];
   const int ntd = (nd + TD - 1) / TD, ntt = (nt + TT - 1) / TT;
   // Tiles that share stencil cells (neighbours along D) are consecutive
   // logical blocks, and consecutive logical blocks run on one XCD (one L2).
-  unsigned b = block_xcd();
   const int td = (int)(b % (unsigned)ntd);
   b /= (unsigned)ntd;
   const int tt = (int)(b % (unsigned)ntt);
   b /= (unsigned)ntt;
   const int x = (int)(b % (unsigned)nx);
   const int f = (int)(b / (unsigned)nx);
-  if (f >= 6) return;
+  const bool live = f < 6;
   const int d0 = td * TD, t0 = tt * TT;             // tile origin (active-relative)
   const int nvd = min(TD, nd - d0), nvt = min(TT, nt - t0);
   auto at_of = [&](int ad, int at2) {
@@ -1303,11 +1326,11 @@ __global__ void __launch_bounds__(TD_ * TT_, 4) k_face_flux_tiled(K c) {
   int slot[kFill];
 #pragma unroll
   for (int r = 0; r < kFill; ++r) {
-    const int q = (int)threadIdx.x + r * T::kThreads;
+    const int q = tid + r * T::kThreads;
     const int cd = D == 2 ? q % CD : q / TT;
     const int t = D == 2 ? q / CD : q % TT;
     slot[r] = -1;
-    if (q >= kSlots || cd >= nvd + 7 || t >= nvt) continue;
+    if (!live || q >= kSlots || cd >= nvd + 7 || t >= nvt) continue;
     const long cell = at_of(d0 - 4 + cd, t0 + t);
     slot[r] = T::slot(cd, t);
     for (int v = 0; v < 5; ++v) fill[r][v] = c.p(P_WPRED + v)[cell];
@@ -1319,14 +1342,21 @@ __global__ void __launch_bounds__(TD_ * TT_, 4) k_face_flux_tiled(K c) {
     if (slot[r] >= 0)
       for (int v = 0; v < T::kVars; ++v) s_cell[v * kSlots + slot[r]] = fill[r][v];
   __syncthreads();
-  const int a = D == 2 ? (int)threadIdx.x % TD : (int)threadIdx.x / TT;
-  const int t = D == 2 ? (int)threadIdx.x / TD : (int)threadIdx.x % TT;
-  if (a >= nvd || t >= nvt) return;
+  const int a = D == 2 ? tid % TD : tid / TT;
+  const int t = D == 2 ? tid / TD : tid % TT;
+  if (!live || a >= nvd || t >= nvt) return;
   const long at = at_of(d0 + a, t0 + t);
   const long st = D == 0 ? L.di() : D == 1 ? (long)L.SK : 1;
   const double *base = s_cell + T::slot(a, t);
   face_flux_face(c, D, f, at, st,
                  [&](int v, int n) { return base[v * kSlots + n * T::kStep]; });
+}
+
+template <int D, int TD_, int TT_>
+__global__ void __launch_bounds__(TD_ * TT_, 4) k_face_flux_tiled(K c) {
+  using T = FluxTile<D, TD_, TT_>;
+  __shared__ double s_cell[T::kLds];
+  flux_tile<T, D>(c, block_xcd(), threadIdx.x, s_cell);
 }
 
 // Tile shapes of the FP64 face flux per direction.
@@ -1346,12 +1376,11 @@ constexpr int kRowFaces = 256, kRowMax = 12;
 constexpr int kRowSlots = kRowFaces + 7 * kRowMax;
 constexpr int kRowMinFaces = (kRowFaces - 1 + kRowMax - 2) / (kRowMax - 1);
 
-__global__ void __launch_bounds__(kRowFaces, 4) k_face_flux_rows(K c) {
-  __shared__ double s_cell[9 * kRowSlots];
+GCS_DEV void flux_rows(const K &c, unsigned b, double *s_cell) {
   const Layout &L = c.L;
   const int nf = L.n + 1;  // k-faces per row
   const long rows = 6L * L.nr * L.n, total = rows * nf;
-  const long q0 = (long)block_xcd() * kRowFaces;
+  const long q0 = (long)b * kRowFaces;
   if (q0 >= total) return;
   const int nq = (int)min((long)kRowFaces, total - q0);  // faces of this block
   const long row0 = q0 / nf;
@@ -1407,6 +1436,11 @@ __global__ void __launch_bounds__(kRowFaces, 4) k_face_flux_rows(K c) {
   face_flux_face(c, 2, f, at, 1, [&](int v, int n) { return base[v * kRowSlots + n]; });
 }
 
+__global__ void __launch_bounds__(kRowFaces, 4) k_face_flux_rows(K c) {
+  __shared__ double s_cell[9 * kRowSlots];
+  flux_rows(c, block_xcd(), s_cell);
+}
+
 // ---- fused face velocity + edge EMF, LDS tiles ------------------------------------
 //
 // For edge directions e = 0 (t1 = j, t2 = k) and e = 1 (t1 = k, t2 = i) a
@@ -1436,6 +1470,12 @@ struct EmfTile {
   // Row stride of the t2-face arrays: when the edge loop walks t1 (= k)
   // fastest, an odd stride keeps a wave's reads on distinct LDS banks.
   static constexpr int S2 = T1 == 2 ? (E2 | 1) : E2;
+  static constexpr int kLds = 4 * C1 * C2 + 5 * E1 * C2 + 2 * C1 * S2;  // doubles
+  static unsigned blocks(int nr, int n) {
+    const int act[3] = {nr, n, n};
+    return (unsigned)(6L * act[E] * ((act[T1] + 1 + E1 - 1) / E1) *
+                      ((act[T2] + 1 + E2 - 1) / E2));
+  }
   // (position along e, along t1, along t2) -> (i, j, k)
   GCS_DEV static void ijk(int ce, int a1, int a2, int &i, int &j, int &k) {
     int x[3];
@@ -1448,14 +1488,18 @@ struct EmfTile {
   }
 };
 
+// One tile (logical block `block`, 256 threads, T::kLds doubles of LDS).
 template <int E>
-__global__ void __launch_bounds__(256) k_edge_emf_tiled(K c) {
+GCS_DEV void emf_tile(const K &c, unsigned block, double *lds) {
   using T = EmfTile<E>;
   constexpr int E1 = T::E1, E2 = T::E2, C1 = T::C1, C2 = T::C2, S2 = T::S2;
   constexpr int t1 = T::T1, t2 = T::T2;
-  __shared__ double s_vol[C1 * C2], s_wv[3][C1 * C2];
-  __shared__ double s_fv[3][E1 * C2], s_a1[E1 * C2], s_b1[E1 * C2];
-  __shared__ double s_a2[C1 * S2], s_b2[C1 * S2];
+  double *s_vol = lds, *s_wv[3], *s_fv[3];
+  for (int m = 0; m < 3; ++m) s_wv[m] = lds + (1 + m) * C1 * C2;
+  double *at_faces = lds + 4 * C1 * C2;
+  for (int m = 0; m < 3; ++m) s_fv[m] = at_faces + m * E1 * C2;
+  double *s_a1 = at_faces + 3 * E1 * C2, *s_b1 = at_faces + 4 * E1 * C2;
+  double *s_a2 = at_faces + 5 * E1 * C2, *s_b2 = s_a2 + C1 * S2;
   const Layout &L = c.L;
   const int act[3] = {L.nr, L.n, L.n};
   // edge box: [g, g + act) along e, [g, g + act + 1) along t1 and t2
@@ -1464,7 +1508,7 @@ __global__ void __launch_bounds__(256) k_edge_emf_tiled(K c) {
   const int nt1 = (hi1 - lo1 + E1 - 1) / E1, nt2 = (hi2 - lo2 + E2 - 1) / E2;
   // consecutive logical blocks, neighbours along t2 that share fill cells,
   // run on one XCD (one L2)
-  long b = block_xcd();
+  long b = block;
   const int tile2 = (int)(b % nt2);
   b /= nt2;
   const int tile1 = (int)(b % nt1);
@@ -1621,6 +1665,12 @@ __global__ void __launch_bounds__(256) k_edge_emf_tiled(K c) {
   c.p(P_EMF + E)[at] = emf;
 }
 
+template <int E>
+__global__ void __launch_bounds__(256) k_edge_emf_tiled(K c) {
+  __shared__ double lds[EmfTile<E>::kLds];
+  emf_tile<E>(c, block_xcd(), lds);
+}
+
 // nonorthogonal_step.c:35-71 on the inner wall face.
 template <typename T>
 GCS_DEV void inner_trap(const K &c, long t) {
@@ -1660,14 +1710,14 @@ __global__ void k_finish_flux(K c, const SeamPair *pairs, int n, unsigned trap_f
 constexpr int kFaceVelocityRun = 8;
 
 template <int RM>
-__global__ void __launch_bounds__(128) k_face_velocity_i(K c) {
+GCS_DEV void face_velocity_i(const K &c, long tq) {
   const Layout &L = c.L;
   const int nf = L.nr + 1;  // i-faces of the active box along a column
   const int lo[3] = {0, L.ghost - 4, L.ghost - 4};
   const int hi[3] = {(nf + RM - 1) / RM, min(L.ghost + L.n + 4, L.NJ),
                      min(L.ghost + L.n + 4, L.NK)};
   int f, r, j, k;
-  if (!box(tid_xcd(), lo, hi, f, r, j, k)) return;
+  if (!box(tq, lo, hi, f, r, j, k)) return;
   const int i0 = L.ghost + r * RM;
   const int nv = min(RM, L.ghost + nf - i0);  // faces of this run
   const long si = L.di(), at0 = L.at(f, i0, j, k);
@@ -1689,6 +1739,10 @@ __global__ void __launch_bounds__(128) k_face_velocity_i(K c) {
         c.p(P_FVEL + e)[at0 + m * si] = ok ? central8(wv[e] + m) / iv : NAN;
     }
   }
+}
+template <int RM>
+__global__ void __launch_bounds__(128) k_face_velocity_i(K c) {
+  face_velocity_i<RM>(c, tid_xcd());
 }
 
 // nonorthogonal_sweep.c:223-259 one face per thread for the faces of
@@ -1726,14 +1780,14 @@ __global__ void __launch_bounds__(128) k_face_velocity(K c, int d) {
 
 // nonorthogonal_sweep.c:624-752 for edges of direction e bounding the
 // active box.
-__global__ void __launch_bounds__(128) k_edge_emf(K c, int e) {
+GCS_DEV void edge_emf_plain(const K &c, int e, long tq) {
   const Layout &L = c.L;
   const int t1 = (e + 1) % 3, t2 = (e + 2) % 3;
   const int lo[3] = {L.ghost, L.ghost, L.ghost};
   const int hi[3] = {L.ghost + L.nr + (e != 0), L.ghost + L.n + (e != 1),
                      L.ghost + L.n + (e != 2)};
   int f, i, j, k;
-  if (!box(tid_xcd(), lo, hi, f, i, j, k)) return;
+  if (!box(tq, lo, hi, f, i, j, k)) return;
   const long at = L.at(f, i, j, k);
   if (!c.b(Q_VALID + e)[at] || !c.b(Q_EBOK + e)[at]) {
     c.fail(51, at);
@@ -1808,7 +1862,76 @@ __global__ void __launch_bounds__(128) k_edge_emf(K c, int e) {
   }
   c.p(P_EMF + e)[at] = emf;
 }
+__global__ void __launch_bounds__(128) k_edge_emf(K c, int e) {
+  edge_emf_plain(c, e, tid_xcd());
+}
 
+// ---- small grids: the sweeps in two launches -------------------------------------
+//
+// On a small grid a sweep's launch is one latency (10-13 us each at 12^2 cells,
+// 15-30 us at 24^2, where its blocks fill a fraction of the chip), so the
+// sweeps that need only the predictor's results run as one launch, block
+// range by block range: the face fluxes of the three directions, the i- and
+// j-edge EMFs and the i-face velocities. The second launch holds what needs
+// those: the k-edge EMF, the flux averages and the inner trap. A block has
+// 256 threads, so it takes two flux tiles. Every device function is the
+// separate kernels'.
+constexpr int kSweepThreads = 256;
+constexpr int kSweepLds =
+    EmfTile<1>::kLds > 2 * FluxTileI::kLds ? EmfTile<1>::kLds : 2 * FluxTileI::kLds;
+static_assert(kSweepLds >= EmfTile<0>::kLds && kSweepLds >= 9 * kRowSlots &&
+                  kSweepLds >= 2 * FluxTileJ::kLds && 2 * FluxTileI::kThreads == kSweepThreads &&
+                  2 * FluxTileJ::kThreads == kSweepThreads && kRowFaces == kSweepThreads,
+              "the sweeps' blocks share one shape");
+
+// Blocks of each part, each rounded up to a multiple of 8 so that a part's
+// block b runs on XCD b % 8 like a launch of its own.
+struct SweepWork {
+  unsigned blocks[6];   // flux i, j, k, EMF i, j, face velocity
+  unsigned real[6];     // of these, with work
+  int rows;             // k-face flux in LDS rows (else one face per thread)
+};
+
+__global__ void __launch_bounds__(kSweepThreads, 2) k_sweeps(K c, SweepWork g) {
+  __shared__ double lds[kSweepLds];
+  unsigned b = blockIdx.x;
+  int part = 0;
+  for (; part < 5 && b >= g.blocks[part]; ++part) b -= g.blocks[part];
+  b = block_xcd(b, g.blocks[part]);
+  if (b >= g.real[part]) return;
+  const int half = threadIdx.x / (kSweepThreads / 2), tid = threadIdx.x % (kSweepThreads / 2);
+  const long tq = b * (long)kSweepThreads + threadIdx.x;
+  if (part == 0)
+    flux_tile<FluxTileI, 0>(c, 2 * b + half, tid, lds + half * FluxTileI::kLds);
+  else if (part == 1)
+    flux_tile<FluxTileJ, 1>(c, 2 * b + half, tid, lds + half * FluxTileJ::kLds);
+  else if (part == 2 && g.rows)
+    flux_rows(c, b, lds);
+  else if (part == 2)
+    flux_plain(c, 2, tq);
+  else if (part == 3)
+    emf_tile<0>(c, b, lds);
+  else if (part == 4)
+    emf_tile<1>(c, b, lds);
+  else
+    face_velocity_i<kFaceVelocityRun>(c, tq);
+}
+
+__global__ void __launch_bounds__(128) k_sweeps_end(K c, const SeamPair *pairs, int n,
+                                                    unsigned flux_blocks, unsigned trap_blocks) {
+  unsigned b = blockIdx.x;
+  if (b < flux_blocks) {
+    sync_flux<double>(c, pairs, n, b * 128L + threadIdx.x);
+    return;
+  }
+  b -= flux_blocks;
+  if (b < trap_blocks) {
+    inner_trap<double>(c, b * 128L + threadIdx.x);
+    return;
+  }
+  b -= trap_blocks;
+  edge_emf_plain(c, 2, b * 128L + threadIdx.x);
+}
 
 // ---- mixed precision: FP32 reconstruction, fluxes and EMF ---------------------
 //
@@ -1940,8 +2063,9 @@ GCS_DEV void face_flux_face_fp32(const K &c, int d, int f, long at, long st, con
 // Four waves per SIMD: the rare FP64 fallback reconstruction otherwise
 // lifts the kernel to 154 VGPRs and three waves; bounded, it spills 84
 // bytes a lane on that path only (0.75 -> 0.63 ms per direction at config 1).
-__global__ void __launch_bounds__(128, 4) k_face_flux_fp32(K c, int d) {
+__global__ void __launch_bounds__(128, 4) k_face_flux_fp32(K c) {
   const Layout &L = c.L;
+  const int d = blockIdx.y;
   const int lo[3] = {L.ghost, L.ghost, L.ghost};
   const int hi[3] = {L.ghost + L.nr + (d == 0), L.ghost + L.n + (d == 1),
                      L.ghost + L.n + (d == 2)};
@@ -1955,10 +2079,11 @@ __global__ void __launch_bounds__(128, 4) k_face_flux_fp32(K c, int d) {
   });
 }
 
-__global__ void k_face_velocity_fp32(K c, int d) {
+__global__ void k_face_velocity_fp32(K c, int first) {
   using R = float;
   using namespace mixed;
   const Layout &L = c.L;
+  const int d = first + blockIdx.y;
   int lo[3], hi[3];
   const int ext[3] = {L.NI, L.NJ, L.NK};
   const int act[3] = {L.nr, L.n, L.n};
@@ -2023,10 +2148,11 @@ __global__ void __launch_bounds__(128) k_face_velocity_i_fp32(K c) {
   }
 }
 
-__global__ void __launch_bounds__(128) k_edge_emf_fp32(K c, int e) {
+__global__ void __launch_bounds__(128) k_edge_emf_fp32(K c) {
   using R = float;
   using namespace mixed;
   const Layout &L = c.L;
+  const int e = blockIdx.y;
   const int t1 = (e + 1) % 3, t2 = (e + 2) % 3;
   const int lo[3] = {L.ghost, L.ghost, L.ghost};
   const int hi[3] = {L.ghost + L.nr + (e != 0), L.ghost + L.n + (e != 1),
@@ -2108,20 +2234,20 @@ __global__ void __launch_bounds__(128) k_edge_emf_fp32(K c, int e) {
   c.p(P_EMF + e)[at] = (double)emf;
 }
 
-// The Earth boundary's three EMF stages, one thread per edge position (i, j,
-// k) of the shells they touch, for its edges of the three directions in the
-// stages' order: each edge is changed by its own position's thread only, so
-// the stages need no launch of their own. Radial slots 0-3 are the shells
-// outer - 3 .. outer, slot 4 the inner wall where it is none of them.
+// The Earth boundary's three EMF stages, one thread per edge (direction
+// blockIdx.y) of the shells they touch, in the stages' order: each edge is
+// changed by its own thread only, so the stages need no launch of their own.
+// Radial slots 0-3 are the shells outer - 3 .. outer, slot 4 the inner wall
+// where it is none of them.
 //  * cubedsphere_earth_boundary.c:445-489: outer shells blend toward the wind
 //    line integral -(V x B) . l;
-//  * :362-443: diffusive wind EMF on the outer wall;
+//  * :362-443: diffusive wind EMF on the outer wall (J and K edges);
 //  * :429-440: E_t = 0 on the inner wall shell, or with the ionosphere ready,
 //    -(potential difference) / potential norm along each wall edge
 //    (cubedsphere_mi_dipole.c:478-503).
 __global__ void __launch_bounds__(256) k_earth_emf(K c, WindSeries w) {
   const Layout &L = c.L;
-  const int outer = L.ghost + L.nr;
+  const int outer = L.ghost + L.nr, d = blockIdx.y;
   const int lo[3] = {0, 0, 0}, hi[3] = {5, L.NJ + 1, L.NK + 1};
   int f, slot, j, k;
   if (!box(tid(), lo, hi, f, slot, j, k)) return;
@@ -2129,72 +2255,68 @@ __global__ void __launch_bounds__(256) k_earth_emf(K c, WindSeries w) {
   const int i = slot == 4 ? L.ghost : outer - 3 + slot;
   const long at = L.at(f, i, j, k);
   const long step[3] = {L.di(), (long)L.SK, 1};
-  bool ok[3];
-  for (int d = 0; d < 3; ++d)
-    ok[d] = i < L.NI + (d != 0) && j < L.NJ + (d != 1) && k < L.NK + (d != 2) &&
-            c.b(Q_VALID + d)[at];
-  double sw[3][8], wt[3];
+  // Edge extents: I (NI, NJ+1, NK+1), J (NI+1, NJ, NK+1), K (NI+1, NJ+1, NK).
+  auto valid = [&](int e) {
+    return i < L.NI + (e != 0) && j < L.NJ + (e != 1) && k < L.NK + (e != 2) &&
+           c.b(Q_VALID + e)[at];
+  };
+  if (!valid(d)) return;
+  auto sample = [&](int e, double sw[8], double &wt) {
+    double x[3];
+    for (int m = 0; m < 3; ++m) x[m] = 0.5 * (c.p(P_VERT + m)[at] + c.p(P_VERT + m)[at + step[e]]);
+    return sample_wind(w, x, c.sc->wall_time + 0.5 * c.sc->wall_dt, sw, wt);
+  };
+  double emf = c.p(P_EMF + d)[at];
   if (i >= outer - 3) {
-    for (int d = 0; d < 3; ++d) {
-      if (!ok[d]) continue;
-      double x[3];
-      for (int m = 0; m < 3; ++m)
-        x[m] = 0.5 * (c.p(P_VERT + m)[at] + c.p(P_VERT + m)[at + step[d]]);
-      if (!sample_wind(w, x, c.sc->wall_time + 0.5 * c.sc->wall_dt, sw[d], wt[d])) {
-        c.fail(61, at);
+    double sw[8], wt;
+    if (!sample(d, sw, wt)) {
+      c.fail(61, at);
+      return;
+    }
+    double weight = wt;
+    if (i < outer) weight /= 1.0 + (double)(outer - i);
+    const double *vv = sw + 2, *bb = sw + 5;
+    const double el[3] = {-(vv[1] * bb[2] - vv[2] * bb[1]), -(vv[2] * bb[0] - vv[0] * bb[2]),
+                          -(vv[0] * bb[1] - vv[1] * bb[0])};
+    const int eb = P_EDGE + EDGE_PLANES * d;
+    const double len = c.p(eb + EO_LEN)[at];
+    double line = 0.0;
+    for (int m = 0; m < 3; ++m) line += el[m] * c.p(eb + EO_N + m)[at] * len;
+    emf = (1.0 - weight) * emf + weight * line;
+    if (d > 0 && i == outer && j >= L.ghost && j <= L.ghost + L.n && k >= L.ghost &&
+        k <= L.ghost + L.n && valid(3 - d)) {
+      const long si = step[0], sj = step[1];
+      auto dens = [&](int dir, long fa, double &out) {
+        const double area = c.p(P_FACE + FACE_PLANES * dir + FO_AREA)[fa];
+        if (!(area > 0.0)) return false;
+        const double cf = c.p(plane_phi(c.cur, dir))[fa], of = c.p(plane_phi(c.old, dir))[fa];
+        out = (cf + c.sc->ratio * (cf - of)) / area;  // the predictor's Phi*
+        return (bool)isfinite(out);
+      };
+      double bikp, bikm, bkip, bkim, bjip, bjim, bijp, bijm;
+      if (!dens(0, at, bikp) || !dens(0, at - 1, bikm) || !dens(2, at, bkip) ||
+          !dens(2, at - si, bkim) || !dens(1, at, bjip) || !dens(1, at - si, bjim) ||
+          !dens(0, at, bijp) || !dens(0, at - sj, bijm)) {
+        c.fail(62, at);
         return;
       }
-      double weight = wt[d];
-      if (i < outer) weight /= 1.0 + (double)(outer - i);
-      const double *vv = sw[d] + 2, *bb = sw[d] + 5;
-      const double el[3] = {-(vv[1] * bb[2] - vv[2] * bb[1]), -(vv[2] * bb[0] - vv[0] * bb[2]),
-                            -(vv[0] * bb[1] - vv[1] * bb[0])};
-      const int eb = P_EDGE + EDGE_PLANES * d;
-      const double len = c.p(eb + EO_LEN)[at];
-      double line = 0.0;
-      for (int m = 0; m < 3; ++m) line += el[m] * c.p(eb + EO_N + m)[at] * len;
-      double *emf = c.p(P_EMF + d) + at;
-      *emf = (1.0 - weight) * *emf + weight * line;
+      const double curl = d == 1 ? (bikp - bikm) - (bkip - bkim) : (bjip - bjim) - (bijp - bijm);
+      const double dl = sqrt(c.p(P_EDGE + EDGE_PLANES * 1 + EO_LEN)[at] *
+                             c.p(P_EDGE + EDGE_PLANES * 2 + EO_LEN)[at]);
+      // the wind at the position's other wall edge
+      double so[8], wo;
+      if (!(dl > 0.0) || !sample(3 - d, so, wo)) {
+        c.fail(63, at);
+        return;
+      }
+      const double c2 = w.by * w.by + w.bz * w.bz;
+      const double front = fmax(fabs(sw[2]), fabs(so[2])) / sqrt(1.0 + c2);
+      const double speed = fmin(front, c.o.wall_cfl * dl / c.sc->wall_dt);
+      emf += wt * speed * curl * dl;
     }
   }
-  // Edge extents: J (NI+1, NJ, NK+1), K (NI+1, NJ+1, NK). The wind samples of
-  // the two edges are those of the blend above.
-  if (i == outer && j >= L.ghost && j <= L.ghost + L.n && k >= L.ghost && k <= L.ghost + L.n &&
-      ok[1] && ok[2]) {
-    const long si = step[0], sj = step[1];
-    auto dens = [&](int dir, long fa, double &out) {
-      const double area = c.p(P_FACE + FACE_PLANES * dir + FO_AREA)[fa];
-      if (!(area > 0.0)) return false;
-      const double cf = c.p(plane_phi(c.cur, dir))[fa], of = c.p(plane_phi(c.old, dir))[fa];
-      out = (cf + c.sc->ratio * (cf - of)) / area;  // the predictor's Phi*
-      return (bool)isfinite(out);
-    };
-    double bikp, bikm, bkip, bkim, bjip, bjim, bijp, bijm;
-    if (!dens(0, at, bikp) || !dens(0, at - 1, bikm) || !dens(2, at, bkip) ||
-        !dens(2, at - si, bkim) || !dens(1, at, bjip) || !dens(1, at - si, bjim) ||
-        !dens(0, at, bijp) || !dens(0, at - sj, bijm)) {
-      c.fail(62, at);
-      return;
-    }
-    const double cj = (bikp - bikm) - (bkip - bkim);
-    const double ck = (bjip - bjim) - (bijp - bijm);
-    const double dl = sqrt(c.p(P_EDGE + EDGE_PLANES * 1 + EO_LEN)[at] *
-                           c.p(P_EDGE + EDGE_PLANES * 2 + EO_LEN)[at]);
-    if (!(dl > 0.0)) {
-      c.fail(63, at);
-      return;
-    }
-    const double c2 = w.by * w.by + w.bz * w.bz;
-    const double front = fmax(fabs(sw[1][2]), fabs(sw[2][2])) / sqrt(1.0 + c2);
-    const double speed = fmin(front, c.o.wall_cfl * dl / c.sc->wall_dt);
-    c.p(P_EMF + 1)[at] += wt[1] * speed * cj * dl;
-    c.p(P_EMF + 2)[at] += wt[2] * speed * ck * dl;
-  }
-  if (i != L.ghost) return;
-  // J edges span (NI+1, NJ, NK+1), K edges (NI+1, NJ+1, NK).
-  for (int d = 1; d <= 2; ++d) {
-    if (!ok[d]) continue;
-    double emf = 0.0;
+  if (d > 0 && i == L.ghost) {
+    emf = 0.0;
     if (c.mi.potential != nullptr) {
       const long end = at + step[d];
       const double a[3] = {c.p(P_VERT)[at], c.p(P_VERT + 1)[at], c.p(P_VERT + 2)[at]};
@@ -2206,8 +2328,8 @@ __global__ void __launch_bounds__(256) k_earth_emf(K c, WindSeries w) {
       }
       emf = -(pb - pa) / c.mi.potential_norm;
     }
-    c.p(P_EMF + d)[at] = emf;
   }
+  c.p(P_EMF + d)[at] = emf;
 }
 
 // ---- update ------------------------------------------------------------------------
@@ -2524,10 +2646,43 @@ void mark_stage(Problem &P, int stage) {
   ++P.stage_cursor;
 }
 
+// Launch the FP64 sweeps of a small grid, fluxes and EMFs, in two launches
+// (k_sweeps, k_sweeps_end). The line lies where the separate launches, each
+// with its own registers and LDS, catch up (us a step, separate / joint, graph
+// launches): 14 k cells 149 / 95, 166 k 322 / 273, 393 k 509 / 449, 911 k 989
+// / 960, 1.33 M 1286 / 1295.
+constexpr long kJointCells = 1000000;
+
+static void launch_sweeps(Problem &P, const K &c) {
+  const Layout &L = P.L;
+  const long n_k = 6L * L.nr * L.n * (L.n + 1);
+  const long wide_j = std::min(L.ghost + L.n + 4, L.NJ) - (L.ghost - 4);
+  SweepWork g;
+  g.rows = L.n + 1 >= kRowMinFaces ? 1 : 0;
+  g.real[0] = (FluxTileI::blocks(L.nr, L.n) + 1) / 2;
+  g.real[1] = (FluxTileJ::blocks(L.nr, L.n) + 1) / 2;
+  g.real[2] = nblocks(n_k, kSweepThreads);
+  g.real[3] = EmfTile<0>::blocks(L.nr, L.n);
+  g.real[4] = EmfTile<1>::blocks(L.nr, L.n);
+  g.real[5] = nblocks(6L * ((L.nr + kFaceVelocityRun) / kFaceVelocityRun) * wide_j * wide_j,
+                      kSweepThreads);
+  unsigned blocks = 0;
+  for (int q = 0; q < 6; ++q) {
+    g.blocks[q] = (g.real[q] + 7) / 8 * 8;
+    blocks += g.blocks[q];
+  }
+  k_sweeps<<<blocks, kSweepThreads, 0, P.stream>>>(c, g);
+  const unsigned flux = nblocks(P.n_seams, 128);
+  const unsigned trap = P.bnd.inner_trap ? nblocks(6L * L.n * L.n, 128) : 0u;
+  const unsigned edges = nblocks(6L * (L.nr + 1) * (L.n + 1) * L.n, 128);
+  k_sweeps_end<<<flux + trap + edges, 128, 0, P.stream>>>(c, P.seams, P.n_seams, flux, trap);
+}
+
 // Kernels that need nothing of each other share a launch: on small grids a
 // step is the sum of its launches' latencies, 5-13 us each (16 x 12^2 cells a
-// face, default options: 33 launches, 236 us a step; 48 x 24^2: 462 us).
-int enqueue_phase(Problem &P, Phase phase, bool driver) {
+// face, default options: 33 launches 236 us a step, 12 launches 105; 48 x
+// 24^2: 462, 331).
+int enqueue_phase(Problem &P, Phase phase, bool driver, bool whole) {
   K c = make_k(P);
   const Layout &L = P.L;
   hipStream_t s = P.stream;
@@ -2535,8 +2690,21 @@ int enqueue_phase(Problem &P, Phase phase, bool driver) {
   const long n_active = 6L * L.nr * L.n * L.n;
   const long n_cells = 6L * L.NI * L.NJ * L.NK;
   const long n_box = 6L * (L.NI + 1) * (L.NJ + 1) * (L.NK + 1);
+  // The largest direction's faces and edges, the columns of the k-edges'
+  // i-face velocities and the faces of each direction's velocity sweep.
+  const long n_faces = 6L * std::max((L.nr + 1L) * L.n * L.n, (long)L.nr * (L.n + 1) * L.n);
+  const long n_edges = 6L * std::max((long)L.nr * (L.n + 1) * (L.n + 1), (L.nr + 1L) * L.n * (L.n + 1));
+  const long wide_i = std::min(L.ghost + L.nr + 4, L.NI) - (L.ghost - 4);
+  const long wide_j = std::min(L.ghost + L.n + 4, L.NJ) - (L.ghost - 4);
+  const long n_columns = wide_j * wide_j;
+  const long n_velocity[3] = {6L * (L.nr + 1) * n_columns, 6L * wide_i * (L.n + 1) * wide_j,
+                              6L * wide_i * wide_j * (L.n + 1)};
   const WindSeries &w = P.wind_series;
   const StepBoundary &bd = P.bnd;
+  // Fluxes and EMF sweeps in joint launches (launch_sweeps): whole steps of
+  // small FP64 grids.
+  const bool joint = whole && !P.mixed && !P.plain && !P.profiling && P.opt.mhd &&
+                     n_active <= kJointCells;
 
   if (phase == PHASE_GHOSTS) {
     // cubedsphere_step.c:51-65
@@ -2605,14 +2773,21 @@ int enqueue_phase(Problem &P, Phase phase, bool driver) {
       k_predict<true><<<nblocks(n_box, T), T, 0, s>>>(c);
     else
       k_predict<false><<<nblocks(n_box, T), T, 0, s>>>(c);
-    for (int d = 0; d < 3; ++d) {
+    if (joint) {
+      launch_sweeps(P, c);
+      return 0;
+    }
+    if (P.mixed) {
+      // The FP32 kernels read half the bytes and are faster without tiles;
+      // the three directions share a launch (blockIdx.y).
+      mark_stage(P, S_FACE_FLUX0);
+      k_face_flux_fp32<<<dim3(nblocks(n_faces, 128), 3), 128, 0, s>>>(c);
+    }
+    for (int d = 0; d < (P.mixed ? 0 : 3); ++d) {
       const long n = 6L * (L.nr + (d == 0)) * (L.n + (d == 1)) * (L.n + (d == 2));
       mark_stage(P, S_FACE_FLUX0 + d);
-      // FP64: LDS tiles along i and j, LDS rows along k. The FP32 kernels
-      // read half the bytes and are faster without tiles.
-      if (P.mixed)
-        k_face_flux_fp32<<<nblocks(n, 128), 128, 0, s>>>(c, d);
-      else if (P.plain)
+      // FP64: LDS tiles along i and j, LDS rows along k.
+      if (P.plain)
         k_face_flux<<<nblocks(n, 128), 128, 0, s>>>(c, d);
       else if (d == 0)
         k_face_flux_tiled<0, FluxTileI::TD, FluxTileI::TT>
@@ -2636,49 +2811,42 @@ int enqueue_phase(Problem &P, Phase phase, bool driver) {
     // cubedsphere_step.c:99-126 up to the seam EMF average; a hydrodynamic
     // step has no EMF
     if (!P.opt.mhd) return 0;
-    mark_stage(P, S_FACE_VELOCITY);
-    const int act[3] = {L.nr, L.n, L.n};
-    // FP64: the i-face velocities for the k-edges only; the j- and i-edges
-    // compute their t1-face velocities inside their LDS tiles.
-    for (int d = 0; d < (P.mixed || P.plain ? 3 : 1); ++d) {
-      long n = 6;
-      const int ext[3] = {L.NI, L.NJ, L.NK};
-      for (int a = 0; a < 3; ++a)
-        n *= a == d ? act[a] + 1 : std::min(L.ghost + act[a] + 4, ext[a]) - (L.ghost - 4);
-      if (P.plain && !P.mixed)
-        k_face_velocity<<<nblocks(n, 128), 128, 0, s>>>(c, d);
-      else if (P.mixed && d == 0 && !P.plain)  // 128 threads: the kernel's launch bound
-        k_face_velocity_i_fp32<kFaceVelocityRun><<<nblocks(6L * ((L.nr + kFaceVelocityRun) / kFaceVelocityRun) *
-                                                                (n / (6L * (L.nr + 1))), 128), 128, 0, s>>>(c);
-      else if (P.mixed)
-        k_face_velocity_fp32<<<nblocks(n, T), T, 0, s>>>(c, d);
-      else
-        // 128 threads: the kernel's launch bound
-        k_face_velocity_i<kFaceVelocityRun><<<nblocks(6L * ((L.nr + kFaceVelocityRun) / kFaceVelocityRun) *
-                                                           (n / (6L * (L.nr + 1))), 128), 128, 0, s>>>(c);
-    }
-    for (int e = 0; e < 3; ++e) {
-      const long n = 6L * (L.nr + (e != 0)) * (L.n + (e != 1)) * (L.n + (e != 2));
-      mark_stage(P, S_EDGE_EMF0 + e);
-      if (P.mixed) {
-        k_edge_emf_fp32<<<nblocks(n, 128), 128, 0, s>>>(c, e);
-      } else if (e == 2 || P.plain) {
-        k_edge_emf<<<nblocks(n, 128), 128, 0, s>>>(c, e);
-      } else {
-        const int t1 = (e + 1) % 3, t2 = (e + 2) % 3;
-        const int e1 = e == 0 ? EmfTile<0>::E1 : EmfTile<1>::E1;
-        const int e2 = e == 0 ? EmfTile<0>::E2 : EmfTile<1>::E2;
-        const long tiles = 6L * act[e] * ((act[t1] + 1 + e1 - 1) / e1) *
-                           ((act[t2] + 1 + e2 - 1) / e2);
-        if (e == 0)
-          k_edge_emf_tiled<0><<<(unsigned)tiles, 256, 0, s>>>(c);
+    const long n_runs = 6L * ((L.nr + kFaceVelocityRun) / kFaceVelocityRun) * n_columns;
+    if (joint) {
+      // the sweeps ran with the fluxes
+    } else if (P.mixed) {
+      mark_stage(P, S_FACE_VELOCITY);
+      if (!P.plain)  // 128 threads: the kernel's launch bound
+        k_face_velocity_i_fp32<kFaceVelocityRun><<<nblocks(n_runs, 128), 128, 0, s>>>(c);
+      const int first = P.plain ? 0 : 1;
+      long n = n_velocity[1];
+      if (P.plain) n = std::max(n, n_velocity[0]);
+      k_face_velocity_fp32<<<dim3(nblocks(n, T), 3 - first), T, 0, s>>>(c, first);
+      mark_stage(P, S_EDGE_EMF0);
+      k_edge_emf_fp32<<<dim3(nblocks(n_edges, 128), 3), 128, 0, s>>>(c);
+    } else {
+      // FP64: the i-face velocities for the k-edges only; the j- and i-edges
+      // compute their t1-face velocities inside their LDS tiles.
+      mark_stage(P, S_FACE_VELOCITY);
+      if (P.plain)
+        for (int d = 0; d < 3; ++d)
+          k_face_velocity<<<nblocks(n_velocity[d], 128), 128, 0, s>>>(c, d);
+      else  // 128 threads: the kernel's launch bound
+        k_face_velocity_i<kFaceVelocityRun><<<nblocks(n_runs, 128), 128, 0, s>>>(c);
+      for (int e = 0; e < 3; ++e) {
+        const long n = 6L * (L.nr + (e != 0)) * (L.n + (e != 1)) * (L.n + (e != 2));
+        mark_stage(P, S_EDGE_EMF0 + e);
+        if (e == 2 || P.plain)
+          k_edge_emf<<<nblocks(n, 128), 128, 0, s>>>(c, e);
+        else if (e == 0)
+          k_edge_emf_tiled<0><<<EmfTile<0>::blocks(L.nr, L.n), 256, 0, s>>>(c);
         else
-          k_edge_emf_tiled<1><<<(unsigned)tiles, 256, 0, s>>>(c);
+          k_edge_emf_tiled<1><<<EmfTile<1>::blocks(L.nr, L.n), 256, 0, s>>>(c);
       }
     }
     if (bd.earth_emf) {
       mark_stage(P, S_EARTH_EMF);
-      k_earth_emf<<<nblocks(6L * 5 * (L.NJ + 1) * (L.NK + 1), T), T, 0, s>>>(c, w);
+      k_earth_emf<<<dim3(nblocks(6L * 5 * (L.NJ + 1) * (L.NK + 1), T), 3), T, 0, s>>>(c, w);
     }
   } else {
     // cubedsphere_step.c:125-152
@@ -3378,7 +3546,7 @@ int enqueue_step(Problem &P, bool explicit_dt) {
   }
   P.last_step_mixed = P.mixed;
   for (Phase ph : {PHASE_GHOSTS, PHASE_FLUX, PHASE_EMF, PHASE_UPDATE})
-    if (enqueue_phase(P, ph, !explicit_dt) != 0) return -1;
+    if (enqueue_phase(P, ph, !explicit_dt, true) != 0) return -1;
   mark_stage(P, S_END);
   GCS_HIP(hipGetLastError());
   return 0;
