@@ -99,6 +99,10 @@ void free_problem(Problem *P) {
     if (g.exec) (void)hipGraphExecDestroy(g.exec);
   (void)hipFree(P->planes_alloc);
   if (P->pinned != nullptr) (void)hipHostFree(P->pinned);
+  (void)hipFree(P->packed);
+  for (hipEvent_t e : P->copied)
+    if (e != nullptr) (void)hipEventDestroy(e);
+  for (HostArray &a : P->host_arrays) free_array(a);
   (void)hipFree(P->planes32_alloc);
   (void)hipFree(P->bytes);
   (void)hipFree(P->scalars);
@@ -185,62 +189,106 @@ int check_failure(Problem &P) {
 
 namespace {
 
-// Copy one component plane of one cube face to the host in the
-// reference's k-fastest order for extent e.
-int fetch(Problem &P, int plane, int face, const size_t e[3], int ncomp,
-          int comp, std::vector<double> &out) {
+// The consecutive planes of a field whose host array interleaves them, and
+// its extent; false for the fields that are laid out otherwise.
+bool field_planes(const Problem &P, int field, int &first, int &ncomp, size_t e[3]) {
   const Layout &L = P.L;
-  std::vector<double> buf(L.face_stride);
-  GCS_HIP(hipMemcpy(buf.data(), P.plane(plane) + face * L.face_stride,
-                    L.face_stride * sizeof(double), hipMemcpyDeviceToHost));
-  for (size_t i = 0; i < e[0]; ++i)
-    for (size_t j = 0; j < e[1]; ++j)
-      for (size_t k = 0; k < e[2]; ++k)
-        out[((i * e[1] + j) * e[2] + k) * ncomp + comp] =
-            buf[(i * L.SJ + j) * L.SK + k];
-  return 0;
+  const int cur = P.level, old = 1 - P.level;
+  auto cells = [&](int p, int n) {
+    first = p;
+    ncomp = n;
+    e[0] = L.NI;
+    e[1] = L.NJ;
+    e[2] = L.NK;
+    return true;
+  };
+  auto faces = [&](int d, int p, int n) {
+    first = p;
+    ncomp = n;
+    face_extent(L, d, e);
+    return true;
+  };
+  auto edges = [&](int d, int p, int n) {
+    first = p;
+    ncomp = n;
+    edge_extent(L, d, e);
+    return true;
+  };
+  switch (field) {
+    case GCS_FIELD_CONSERVED: return cells(plane_u(cur, 0), 5);
+    case GCS_FIELD_OLD_CONSERVED: return cells(plane_u(old, 0), 5);
+    case GCS_FIELD_PREDICTED_CONSERVED: return cells(P_UPRED, 5);
+    case GCS_FIELD_CELL_MAGNETIC: return cells(plane_b(cur, 0), 3);
+    case GCS_FIELD_OLD_CELL_MAGNETIC: return cells(plane_b(old, 0), 3);
+    case GCS_FIELD_PREDICTED_CELL_MAGNETIC: return cells(P_BPRED, 3);
+    case GCS_FIELD_BG_CELL_MAGNETIC: return cells(P_B0C, 3);
+    case GCS_FIELD_BG_CELL_FORCE: return cells(P_FORCE, 3);
+    case GCS_FIELD_VERTEX:
+      first = P_VERT;
+      ncomp = 3;
+      e[0] = L.NI + 1;
+      e[1] = L.NJ + 1;
+      e[2] = L.NK + 1;
+      return true;
+    default: break;
+  }
+  if (field >= GCS_FIELD_FACE_FLUX && field < GCS_FIELD_HYDRO_RATE) {
+    const int d = (field - GCS_FIELD_FACE_FLUX) % 3;
+    switch ((field - GCS_FIELD_FACE_FLUX) / 3) {
+      case 0: return faces(d, plane_phi(cur, d), 1);
+      case 1: return faces(d, plane_phi(old, d), 1);
+      case 2: return faces(d, P_PHIPRED + d, 1);
+      case 3: return edges(d, P_EMF + d, 1);
+      case 4: return faces(d, P_FLUID + 5 * d, 5);
+      default: return faces(d, P_MAXWELL + 3 * d, 3);
+    }
+  }
+  if (field >= GCS_FIELD_FACE_GEOMETRY && field < GCS_FIELD_FACE_GEOMETRY + 3)
+    return faces(field - GCS_FIELD_FACE_GEOMETRY,
+                 P_FACE + FACE_PLANES * (field - GCS_FIELD_FACE_GEOMETRY), FACE_PLANES);
+  if (field >= GCS_FIELD_EDGE_GEOMETRY && field < GCS_FIELD_EDGE_GEOMETRY + 3)
+    return edges(field - GCS_FIELD_EDGE_GEOMETRY,
+                 P_EDGE + EDGE_PLANES * (field - GCS_FIELD_EDGE_GEOMETRY), 10);
+  if (field >= GCS_FIELD_BG_FACE_MAGNETIC && field < GCS_FIELD_COUNT) {
+    const int d = (field - GCS_FIELD_BG_FACE_MAGNETIC) % 3;
+    switch ((field - GCS_FIELD_BG_FACE_MAGNETIC) / 3) {
+      case 0: return faces(d, P_B0F + 3 * d, 3);
+      case 1: return faces(d, P_B0FLUX + d, 1);
+      default: return edges(d, P_B0E + 3 * d, 3);
+    }
+  }
+  return false;
 }
+
+// Fields of the state, whose host memory is kept from step to step.
+bool state_field(int field) { return field < GCS_FIELD_VERTEX; }
+
+// A field's arrays are fetched for all six cube faces at once up to this
+// many doubles in all (4 MiB): below it a transfer is one latency, whatever
+// its size, and programs read the faces in turn.
+constexpr size_t kSixFaces = 1UL << 19;
 
 }  // namespace
 
-int download_field(Problem &P, int face, int field, std::vector<double> &out) {
-  const Layout &L = P.L;
-  const int cur = P.level, old = 1 - P.level;
-  size_t ce[3] = {(size_t)L.NI, (size_t)L.NJ, (size_t)L.NK};
-  size_t ve[3] = {(size_t)L.NI + 1, (size_t)L.NJ + 1, (size_t)L.NK + 1};
-  const size_t ncell = ce[0] * ce[1] * ce[2];
+// A field whose host array interleaves whole planes.
+static int fetch_planes(Problem &P, int face, int field, int first, int ncomp,
+                        const size_t e[3]) {
   // The mixed form keeps the predicted state and the face fluxes in FP32.
   const bool widened = field == GCS_FIELD_PREDICTED_CONSERVED ||
                        field == GCS_FIELD_PREDICTED_CELL_MAGNETIC ||
                        (field >= GCS_FIELD_FACE_FLUX + 12 && field < GCS_FIELD_HYDRO_RATE);
   if (widened && P.last_step_mixed && widen_mixed(P) != 0) return -1;
-  auto planes = [&](int first, int ncomp, const size_t e[3]) {
-    out.assign(e[0] * e[1] * e[2] * ncomp, 0.0);
-    for (int q = 0; q < ncomp; ++q)
-      if (fetch(P, first + q, face, e, ncomp, q, out) != 0) return -1;
-    return 0;
-  };
-  if (field == GCS_FIELD_CONSERVED) return planes(plane_u(cur, 0), 5, ce);
-  if (field == GCS_FIELD_OLD_CONSERVED) return planes(plane_u(old, 0), 5, ce);
-  if (field == GCS_FIELD_PREDICTED_CONSERVED) return planes(P_UPRED, 5, ce);
-  if (field == GCS_FIELD_CELL_MAGNETIC) return planes(plane_b(cur, 0), 3, ce);
-  if (field == GCS_FIELD_OLD_CELL_MAGNETIC) return planes(plane_b(old, 0), 3, ce);
-  if (field == GCS_FIELD_PREDICTED_CELL_MAGNETIC) return planes(P_BPRED, 3, ce);
-  if (field >= GCS_FIELD_FACE_FLUX && field < GCS_FIELD_HYDRO_RATE) {
-    const int group = (field - GCS_FIELD_FACE_FLUX) / 3;
-    const int d = (field - GCS_FIELD_FACE_FLUX) % 3;
-    size_t fe[3], ee[3];
-    face_extent(L, d, fe);
-    edge_extent(L, d, ee);
-    switch (group) {
-      case 0: return planes(plane_phi(cur, d), 1, fe);
-      case 1: return planes(plane_phi(old, d), 1, fe);
-      case 2: return planes(P_PHIPRED + d, 1, fe);
-      case 3: return planes(P_EMF + d, 1, ee);
-      case 4: return planes(P_FLUID + 5 * d, 5, fe);
-      default: return planes(P_MAXWELL + 3 * d, 3, fe);
-    }
-  }
+  const bool all = 6 * e[0] * e[1] * e[2] * (size_t)ncomp <= kSixFaces;
+  HostArray *out[6];
+  const int from = all ? 0 : face, faces = all ? 6 : 1;
+  for (int f = 0; f < faces; ++f) out[f] = &P.host_arrays[(from + f) * GCS_FIELD_COUNT + field];
+  return planes_to_arrays(P, first, ncomp, from, faces, e, out);
+}
+
+int download_field(Problem &P, int face, int field, std::vector<double> &out) {
+  const Layout &L = P.L;
+  size_t ce[3] = {(size_t)L.NI, (size_t)L.NJ, (size_t)L.NK};
+  const size_t ncell = ce[0] * ce[1] * ce[2];
   if (field == GCS_FIELD_HYDRO_RATE || field == GCS_FIELD_MAXWELL_RATE) {
     // active cells: what the last fidelity step's update stored in the
     // face-velocity planes; ghost cells (and steps without fidelity): zero
@@ -253,7 +301,6 @@ int download_field(Problem &P, int face, int field, std::vector<double> &out) {
     return box_planes_to_host(P, nc == 5 ? P_FVEL : P_FVEL + 5, nc, face, ce, lo, hi,
                               out.data());
   }
-  if (field == GCS_FIELD_VERTEX) return planes(P_VERT, 3, ve);
   if (field == GCS_FIELD_CELL_GEOMETRY) {
     // gamera_no_cell_geometry: volume, centroid, face[3][2], cfl_length[3].
     const int per = sizeof(gamera_no_cell_geometry) / sizeof(double);
@@ -285,32 +332,22 @@ int download_field(Problem &P, int face, int field, std::vector<double> &out) {
       if (put(P_CFL + d, 4 + 6 * FACE_PLANES + d, 0, 0, 0) != 0) return -1;
     return 0;
   }
-  if (field >= GCS_FIELD_FACE_GEOMETRY && field < GCS_FIELD_FACE_GEOMETRY + 3) {
-    const int d = field - GCS_FIELD_FACE_GEOMETRY;
-    size_t fe[3];
-    face_extent(L, d, fe);
-    return planes(P_FACE + FACE_PLANES * d, FACE_PLANES, fe);
-  }
-  if (field >= GCS_FIELD_EDGE_GEOMETRY && field < GCS_FIELD_EDGE_GEOMETRY + 3) {
-    const int d = field - GCS_FIELD_EDGE_GEOMETRY;
-    size_t ee[3];
-    edge_extent(L, d, ee);
-    return planes(P_EDGE + EDGE_PLANES * d, 10, ee);
-  }
-  if (field == GCS_FIELD_BG_CELL_MAGNETIC) return planes(P_B0C, 3, ce);
-  if (field == GCS_FIELD_BG_CELL_FORCE) return planes(P_FORCE, 3, ce);
-  if (field >= GCS_FIELD_BG_FACE_MAGNETIC && field < GCS_FIELD_COUNT) {
-    const int group = (field - GCS_FIELD_BG_FACE_MAGNETIC) / 3;
-    const int d = (field - GCS_FIELD_BG_FACE_MAGNETIC) % 3;
-    size_t fe[3], ee[3];
-    face_extent(L, d, fe);
-    edge_extent(L, d, ee);
-    if (group == 0) return planes(P_B0F + 3 * d, 3, fe);
-    if (group == 1) return planes(P_B0FLUX + d, 1, fe);
-    return planes(P_B0E + 3 * d, 3, ee);
-  }
   set_error("unknown field id");
   return -1;
+}
+
+// Drop the host arrays of a state that has moved on: the state's memory is
+// kept for the next download, the others' is given back.
+static void refresh_host(Problem &P) {
+  if (!P.host_dirty) return;
+  P.host_arrays.resize(6 * GCS_FIELD_COUNT);
+  for (size_t q = 0; q < P.host_arrays.size(); ++q) {
+    P.host_arrays[q].valid = false;
+    if (!state_field((int)(q % GCS_FIELD_COUNT))) free_array(P.host_arrays[q]);
+  }
+  P.host_fields.assign(6 * GCS_FIELD_COUNT, {});
+  P.host_valid.assign(18, {});
+  P.host_dirty = false;
 }
 
 int download_valid(Problem &P, int face, int dir, std::vector<uint8_t> &out) {
@@ -476,10 +513,15 @@ int gcs_problem_field(Problem *P, int face, int field, double **data,
       field >= GCS_FIELD_COUNT || data == nullptr || count == nullptr)
     return -1;
   if (hipStreamSynchronize(P->stream) != hipSuccess) return -1;
-  if (P->host_dirty) {
-    P->host_fields.assign(6 * GCS_FIELD_COUNT, {});
-    P->host_valid.assign(18, {});
-    P->host_dirty = false;
+  gcs::refresh_host(*P);
+  int first, ncomp;
+  size_t e[3];
+  if (gcs::field_planes(*P, field, first, ncomp, e)) {
+    gcs::HostArray &a = P->host_arrays[face * GCS_FIELD_COUNT + field];
+    if (!a.valid && gcs::fetch_planes(*P, face, field, first, ncomp, e) != 0) return -1;
+    *data = a.data;
+    *count = a.count;
+    return 0;
   }
   std::vector<double> &v = P->host_fields[face * GCS_FIELD_COUNT + field];
   if (v.empty() && gcs::download_field(*P, face, field, v) != 0) return -1;
@@ -491,11 +533,7 @@ int gcs_problem_field(Problem *P, int face, int field, double **data,
 int gcs_problem_edge_valid(Problem *P, int face, int dir, unsigned char **data,
                            size_t *count) {
   if (P == nullptr || face < 0 || face >= 6 || dir < 0 || dir > 2) return -1;
-  if (P->host_dirty) {
-    P->host_fields.assign(6 * GCS_FIELD_COUNT, {});
-    P->host_valid.assign(18, {});
-    P->host_dirty = false;
-  }
+  gcs::refresh_host(*P);
   std::vector<uint8_t> &v = P->host_valid[face * 3 + dir];
   if (v.empty() && gcs::download_valid(*P, face, dir, v) != 0) return -1;
   *data = v.data();

@@ -136,6 +136,15 @@ struct StepBoundary {
 // is exact, so neither the order nor the slot of a contribution matters).
 constexpr int kCflSlots = 1024;
 
+// A host array in the reference's layout; its memory is kept from step to
+// step (a fresh one costs a page fault per page), `valid` says whether it
+// holds the current state.
+struct HostArray {
+  double *data = nullptr;
+  size_t count = 0, capacity = 0;
+  bool valid = false;
+};
+
 struct Problem {
   gcs_problem_config cfg;
   StepOptions opt;
@@ -169,7 +178,9 @@ struct Problem {
   int *edge_groups = nullptr;      // CSR offsets, n_edge_groups + 1
   int n_edge_groups = 0;
   int n_edge_members = 0;
-  // host mirrors of reference-layout arrays (allocated on first request)
+  // host mirrors of reference-layout arrays (allocated on first request):
+  // arrays that are planes of the device layout, and the others
+  std::vector<HostArray> host_arrays;
   std::vector<std::vector<double>> host_fields;
   std::vector<std::vector<uint8_t>> host_valid;
   bool host_dirty = true;
@@ -218,6 +229,9 @@ struct Problem {
   size_t stage_cursor = 0;
   double *pinned = nullptr;        // pinned host buffer for plane transfers
   size_t pinned_count = 0;         // its size in doubles
+  double *packed = nullptr;        // device buffer of interleaved arrays to download
+  size_t packed_count = 0;         // its size in doubles
+  hipEvent_t copied[2] = {nullptr, nullptr};  // halves of `pinned` in use by a download
   MiState *mi = nullptr;           // ionosphere coupling (mi_enabled)
   MiView mi_view;                  // what the step kernels read
 
@@ -378,7 +392,11 @@ int enqueue_phase(Problem &P, Phase phase, bool driver = false, bool whole = fal
 // Constants derived from uploaded geometry and background: recovery
 // pivots, edge-B solve, B0 normal and edge-tangential components.
 int derive_constants(Problem &P);
-// Copy one reference-layout field of one cube face to the host.
+// Interleave ncomp consecutive planes of `faces` cube faces, extent ext, into
+// P.packed ([face][i][j][k][component]) on the problem's stream.
+int pack_planes(Problem &P, int first, int ncomp, int face, int faces, const size_t ext[3]);
+// Copy one reference-layout field of one cube face to the host (fields that
+// are not whole planes of the device layout).
 int download_field(Problem &P, int face, int field, std::vector<double> &out);
 int download_valid(Problem &P, int face, int dir, std::vector<uint8_t> &out);
 int upload_field(Problem &P, int face, int field, const double *data,

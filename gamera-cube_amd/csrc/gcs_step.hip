@@ -3554,6 +3554,44 @@ int enqueue_step(Problem &P, bool explicit_dt) {
 
 }  // namespace gcs
 
+// ---- downloads: planes to interleaved arrays ---------------------------------------
+
+namespace gcs {
+
+// One (i, j) row of one cube face per block: out[row][k][c] from the ncomp
+// planes. A memory copy; interleaving here instead of on the host lets the
+// array cross PCIe once and be copied whole there.
+__global__ void __launch_bounds__(128) k_pack(const double *planes, long plane_stride,
+                                              long face_stride, int sj, int sk, int e1, int e2,
+                                              int ncomp, double *out) {
+  const int i = blockIdx.x / e1, j = blockIdx.x - i * e1, n = e2 * ncomp;
+  const double *row = planes + blockIdx.y * face_stride + ((long)i * sj + j) * sk;
+  double *to = out + ((long)blockIdx.y * gridDim.x + blockIdx.x) * n;
+  for (int q = threadIdx.x; q < n; q += 128) {
+    const int k = q / ncomp;
+    to[q] = row[(q - k * ncomp) * plane_stride + k];
+  }
+}
+
+int pack_planes(Problem &P, int first, int ncomp, int face, int faces, const size_t ext[3]) {
+  const Layout &L = P.L;
+  const size_t need = ext[0] * ext[1] * ext[2] * (size_t)ncomp * faces;
+  if (P.packed_count < need) {
+    (void)hipFree(P.packed);
+    P.packed = nullptr;
+    P.packed_count = 0;
+    GCS_HIP(hipMalloc(&P.packed, need * sizeof(double)));
+    P.packed_count = need;
+  }
+  k_pack<<<dim3((unsigned)(ext[0] * ext[1]), faces), 128, 0, P.stream>>>(
+      P.plane(first) + face * L.face_stride, L.total, L.face_stride, L.SJ, L.SK, (int)ext[1],
+      (int)ext[2], ncomp, P.packed);
+  GCS_HIP(hipGetLastError());
+  return 0;
+}
+
+}  // namespace gcs
+
 // ---- measurement: a plain copy kernel ----------------------------------------------
 
 namespace gcs {

@@ -25,4 +25,11 @@ int host_to_planes(Problem &P, int first, int ncomp, int face,
 int box_planes_to_host(Problem &P, int first, int ncomp, int face, const size_t ext[3],
                        const size_t lo[3], const size_t hi[3], double *host);
 
+// Host arrays of `faces` cube faces from `face` on, interleaved [element]
+// [ncomp] with extent ext, from ncomp consecutive planes; allocates them.
+struct HostArray;
+int planes_to_arrays(Problem &P, int first, int ncomp, int face, int faces,
+                     const size_t ext[3], HostArray *const out[]);
+void free_array(HostArray &a);
+
 }  // namespace gcs
