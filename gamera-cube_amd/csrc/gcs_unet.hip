@@ -1,14 +1,16 @@
 // The ionosphere warm-start network on the device: a 4-level U-Net (32 base
 // channels) whose 3x3 convolutions, their input and weight gradients run as
 // implicit GEMMs on the matrix cores (bf16 operands, fp32 accumulation,
-// v_mfma_f32_16x16x16_bf16), with pooling, the fused upsample+concat of the
-// decoder inputs, the 1x1 head, the loss and Adam as plain kernels.
+// v_mfma_f32_16x16x16_bf16). Everything between two convolutions is part of
+// their operand loads or epilogues: bias and ReLU, pooling, the decoder's
+// upsample + concatenation, the 1x1 head, and in the backward pass the ReLU
+// mask and the sums over pooled, upsampled and skipped gradients. A forward
+// pass is 14 launches, a backward pass 18; gradients are deterministic.
 //
-// Tensors are NHWC: H = colatitude rows (zero padding beyond the pole and
-// the low-latitude edge), W = longitude columns (periodic), C innermost so a
-// lane's four consecutive k values of an MFMA operand are one 8-byte load.
-// The network is defined layer by layer in kLayers; the numpy statement of
-// the same network is the oracle the tests compare with.
+// H = colatitude rows (zero padding beyond the pole and the low-latitude
+// edge), W = longitude columns (periodic). The network is defined layer by
+// layer in kLayers; the numpy statement of the same network is the oracle the
+// tests compare with.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -27,6 +29,8 @@ namespace unet {
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
@@ -41,6 +45,9 @@ __device__ __host__ inline uint16_t to_bf16(float f) {
   return (uint16_t)(u >> 16);
 }
 __device__ inline float from_bf16(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
+__device__ inline uint32_t pack2(float a, float b) {
+  return (uint32_t)to_bf16(a) | ((uint32_t)to_bf16(b) << 16);
+}
 
 __device__ inline long gtid() { return blockIdx.x * (long)blockDim.x + threadIdx.x; }
 
@@ -49,235 +56,523 @@ __device__ inline long gtid() { return blockIdx.x * (long)blockDim.x + threadIdx
 __device__ inline f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
+// Eight products per lane as two of these, in the order of the channels. (The
+// 16 x 16 x 32 instruction takes them at once, but the convolutions are not
+// bound by the matrix cores.)
+__device__ inline f32x4 mfma32(u32x4 a, u32x4 b, f32x4 c) {
+  c = mfma16(__builtin_bit_cast(bf16x4, u32x2{a[0], a[1]}),
+             __builtin_bit_cast(bf16x4, u32x2{b[0], b[1]}), c);
+  return mfma16(__builtin_bit_cast(bf16x4, u32x2{a[2], a[3]}),
+                __builtin_bit_cast(bf16x4, u32x2{b[2], b[3]}), c);
+}
 
-// The input of a convolution: channels [0, c0) from src0 (at half
-// resolution when up0, read with nearest upsampling), channels [c0, c0+c1)
-// from src1. Both are bf16 NHWC.
-struct ConvIn {
-  const uint16_t *src0 = nullptr, *src1 = nullptr;
-  int c0 = 0, c1 = 0, up0 = 0;
+// ---- tensors -------------------------------------------------------------------
+//
+// Activations and masked gradients exist twice. NHWC (channels innermost) is
+// what a convolution reads, with each 32 channels in the order of a
+// wavefront's results and operands: quarter q of the lanes holds channels 4q ..
+// 4q + 3 and 16 + 4q .. 16 + 4q + 3, which lie together as 16 bytes. Planar
+// [channel][sample][row][padded row of pixels] is what a weight gradient reads:
+// its sum runs over pixels, and eight consecutive pixels of a channel are one
+// lane's operand. Both are written by the epilogue that has the values in
+// registers. Planar rows are padded to a multiple of
+// eight pixels; the first pad element repeats pixel 0 (longitude is
+// periodic), the others stay zero, and gradients are zero in the whole pad.
+struct Grid {
+  int N, H, W;      // samples, rows, columns
+  int wp, batches;  // planar row pitch and samples per channel
+  __device__ int pixel(int n, int y, int x) const { return (n * H + y) * W + x; }
+  __device__ long plane(int c, int n, int y) const {
+    return (((long)c * batches + n) * H + y) * wp;
+  }
 };
 
-// Four consecutive input channels ci..ci+3 at pixel (n, yy, xx) of the
-// output grid H x W; yy outside [0, H) reads zeros.
-__device__ inline bf16x4 load_in4(const ConvIn &in, int n, int yy, int xx, int H, int W,
-                                  int ci) {
-  bf16x4 v = {0, 0, 0, 0};
-  if (yy < 0 || yy >= H) return v;
-  if (ci < in.c0) {
-    const long p = in.up0 ? ((long)(n * (H >> 1) + (yy >> 1)) * (W >> 1) + (xx >> 1))
-                          : ((long)(n * H + yy) * W + xx);
-    v = *(const bf16x4 *)(in.src0 + p * in.c0 + ci);
-  } else {
-    const long p = (long)(n * H + yy) * W + xx;
-    v = *(const bf16x4 *)(in.src1 + p * in.c1 + (ci - in.c0));
+// The input of a convolution: channels [0, c0) from src0 (at half resolution,
+// read with nearest upsampling), channels [c0, c0 + c1) from src1, NHWC; or
+// fp32 features (the network's input), rounded to bf16 as they are read.
+struct ConvIn {
+  const uint16_t *src0 = nullptr, *src1 = nullptr;
+  const float *f32 = nullptr;
+  const uint16_t *zero = nullptr;  // what rows outside the grid read: 64 zero bytes
+  int c0 = 0, c1 = 0;
+};
+
+// What a convolution does with its sums.
+enum Epilogue {
+  EP_FORWARD,  // + bias, ReLU, store; optionally the 2 x 2 mean pool and the 1 x 1 head
+  EP_PLAIN,    // input gradient of a plain layer: mask by act > 0, store
+  EP_POOL,     // of a layer that reads a pooled activation: spread over 2 x 2 fine
+               // pixels, add the skip's gradient, mask, store at the fine grid
+  EP_CAT       // of a decoder input: sum 2 x 2 into the coarse activation (channels
+               // < c0: mask, store) or keep the skip's gradient (fp32)
+};
+struct ConvOut {
+  Grid g;                       // of `out` (EP_POOL: fine, EP_CAT: coarse)
+  uint16_t *out = nullptr, *planar = nullptr;
+  const float *bias = nullptr;  // EP_FORWARD
+  Grid gp;                      // pooled grid
+  uint16_t *pooled = nullptr, *pooled_planar = nullptr;
+  const float *head_w = nullptr, *head_b = nullptr;
+  float *head_out = nullptr;
+  const uint16_t *act = nullptr;  // NHWC activation whose ReLU masks the gradient
+  float *skip = nullptr;          // EP_POOL: read; EP_CAT: written; NHWC
+  int c0 = 0;                     // EP_CAT: channels of the upsampled part
+};
+
+// The lane's eight channels (quarter q of the 32 from c on) of pixel (n, y, x).
+__device__ inline void store8(const Grid &g, uint16_t *nhwc, uint16_t *planar, int C, int n, int y,
+                              int x, int c, int q, u32x4 v, bool wrap) {
+  *(u32x4 *)(nhwc + (long)g.pixel(n, y, x) * C + c + 8 * q) = v;
+  const long step = (long)g.batches * g.H * g.wp;
+  uint16_t *p = planar + g.plane(c + 4 * q, n, y);
+  for (int i = 0; i < 8; ++i) {
+    const uint16_t e = (uint16_t)(i & 1 ? v[i >> 1] >> 16 : v[i >> 1]);
+    uint16_t *at = p + (i < 4 ? i : 12 + i) * step;
+    at[x] = e;
+    if (wrap && x == 0 && g.W < g.wp) at[g.W] = e;
   }
-  return v;
+}
+// Element i of a packed operand, widened.
+__device__ inline float element(u32x4 v, int i) {
+  return from_bf16((uint16_t)(i & 1 ? v[i >> 1] >> 16 : v[i >> 1]));
+}
+__device__ inline u32x4 pack8(const float z[8]) {
+  return u32x4{pack2(z[0], z[1]), pack2(z[2], z[3]), pack2(z[4], z[5]), pack2(z[6], z[7])};
 }
 
-__device__ inline uint16_t load_in1(const ConvIn &in, int n, int yy, int xx, int H, int W,
-                                    int ci) {
-  if (yy < 0 || yy >= H) return 0;
-  if (ci < in.c0) {
-    const long p = in.up0 ? ((long)(n * (H >> 1) + (yy >> 1)) * (W >> 1) + (xx >> 1))
-                          : ((long)(n * H + yy) * W + xx);
-    return in.src0[p * in.c0 + ci];
-  }
-  const long p = (long)(n * H + yy) * W + xx;
-  return in.src1[p * in.c1 + (ci - in.c0)];
+// The value of the neighbouring lane (l ^ 1).
+__device__ inline float lane_xor1(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xb1, 0xf, 0xf, true));
 }
 
-__device__ inline int wrap(int x, int W) { return x < 0 ? x + W : (x >= W ? x - W : x); }
+// 3x3 convolution as an implicit GEMM on 32 output channels x 32 pixels (two
+// rows of 16, so that a wavefront holds whole 2 x 2 blocks) per wavefront:
+// rows = output channels (weights packed in operand order, k_pack_weights),
+// columns = pixels, k = (tap, input channel) in steps of 32 channels. Operands
+// come straight from L1 / L2 as 16-byte loads, four loads per four MFMAs, the
+// loads of kAhead steps in flight; wk wavefronts of a block share one tile and
+// split its steps. What bounds it is the latency of a launch and of the loads
+// at the small grids, L2 traffic (16 flops a byte) at the large ones. Measured
+// with the kernel before, which gathered 8 bytes per lane and MFMA: the 14
+// layers of 2 x 128 x 256, 930 -> 174 us (130 TFLOP/s); a layer of 8 x 32 x 64,
+// 60 -> 11 us.
+constexpr int kAhead = 4;
 
-// 3x3 convolution as an implicit GEMM: out[m][co] = sum_k A[m][k] B[k][co]
-// with m = pixel (n, y, x), k = (ky*3 + kx)*cin + ci, A = input patch,
-// B[k][co] = w[co][k] (bf16 [cout][9][cin]). A block of 256 threads computes
-// 64 pixels x 64 output channels; wave w owns pixels 16w..16w+15 of the
-// tile. Epilogue: + bias, ReLU, bf16 store (out_bf) or fp32 store (out_f).
-// Requires cin % 16 == 0, c0 % 4 == 0, cout % 16 == 0.
-__global__ void __launch_bounds__(256) k_conv3(ConvIn in, int N, int H, int W,
-                                               const uint16_t *w, const float *bias,
-                                               int cout, int relu, uint16_t *out_bf,
-                                               float *out_f) {
+constexpr int kConvLds = 3 * 16 * 64;  // floats of a block
+
+struct ConvWork {
+  ConvIn in;
+  Grid g;
+  int cout, wk;
+  const uint16_t *w;
+  ConvOut o;
+};
+
+template <int EP, bool F32, bool CAT>
+__device__ inline void conv_block(const ConvWork &job, int block, float *s_part) {
+  const ConvIn &in = job.in;
+  const Grid &g = job.g;
+  const ConvOut &o = job.o;
+  const uint16_t *__restrict__ w = job.w;
+  const int cout = job.cout, wk = job.wk;
+  const int cin = in.c0 + in.c1, spt = cin >> 5, steps = 9 * spt;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int ks = wave % wk, sub = wave / wk;
+  const int ctiles = cout >> 5, xt = (g.W + 15) >> 4, yt = (g.H + 1) >> 1;
+  const int tiles = ctiles * xt * yt * g.N;
+  const int tile = block * ((int)(blockDim.x >> 6) / wk) + sub;
+  const bool live = tile < tiles;
+  int r = live ? tile : 0;
+  const int ct = r % ctiles;
+  r /= ctiles;
+  const int tx = r % xt;
+  r /= xt;
+  const int y0 = 2 * (r % yt), n = r / yt;
+  const int col = lane & 15, q = lane >> 4;
+  const int x = 16 * tx + col, xc = min(x, g.W - 1);
+  f32x4 acc[2][2];  // [16 channels][row of pixels]
+  for (int a = 0; a < 2; ++a)
+    for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint16_t *wt = w + ((long)(2 * ct) * steps * 64 + lane) * 8;
+  const long wnext = (long)steps * 64 * 8;
+  const int s_begin = live ? ks * steps / wk : 0, s_end = live ? (ks + 1) * steps / wk : 0;
+  // One step's operands as loaded: nothing touches a loaded value before its
+  // use, and every step loads (the last ones again, past the end), so that the
+  // wait before a product leaves the loads of the steps ahead in flight.
+  struct Step {
+    u32x4 a[2], b[2], b2[F32 ? 2 : 1];
+  };
+  // The next step to load: its tap's pixels (a row outside the grid reads
+  // zeros, whatever the channel) and its first channel.
+  int ls = s_begin, tap = s_begin / spt, lc = s_begin - tap * spt;
+  const uint16_t *px[2], *px0[2];
+  int inside[2];  // all ones, or zero
+  auto set_tap = [&]() {
+    const int ky = tap / 3, kx = tap - 3 * ky;
+    int xx = xc + kx - 1;
+    xx = xx < 0 ? g.W - 1 : xx >= g.W ? 0 : xx;
+    for (int t = 0; t < 2; ++t) {
+      const int yy = y0 + t + ky - 1;
+      const bool in_grid = yy >= 0 && yy < g.H;
+      inside[t] = in_grid ? -1 : 0;
+      const int at = g.pixel(n, yy, xx);
+      if (F32)
+        px[t] = in_grid ? (const uint16_t *)(in.f32 + (long)at * cin + 4 * q) : in.zero;
+      else
+        px[t] = in_grid ? in.src1 + (long)at * in.c1 + 8 * q : in.zero;
+      if (CAT) {
+        const int up = (n * (g.H >> 1) + (yy >> 1)) * (g.W >> 1) + (xx >> 1);
+        px0[t] = in_grid ? in.src0 + (long)up * in.c0 + 8 * q : in.zero;
+      }
+    }
+  };
+  set_tap();
+  auto load = [&](Step &o) {
+    const uint16_t *ws = wt + (long)min(ls, steps - 1) * 512;
+    const int c = lc * 32;
+    for (int t = 0; t < 2; ++t) {
+      o.a[t] = *(const u32x4 *)(ws + t * wnext);
+      if (F32) {
+        o.b[t] = *(const u32x4 *)px[t];
+        o.b2[t] = *(const u32x4 *)(px[t] + (32 & inside[t]));  // 16 floats on
+      } else if (CAT && c < in.c0) {
+        o.b[t] = *(const u32x4 *)(px0[t] + (c & inside[t]));
+      } else {
+        o.b[t] = *(const u32x4 *)(px[t] + ((c - in.c0) & inside[t]));
+      }
+    }
+    ++ls;
+    if (++lc == spt) {
+      lc = 0;
+      if (tap < 8) ++tap;
+      set_tap();
+    }
+  };
+  auto operand = [&](const Step &o, int v) {
+    if (!F32) return o.b[v];
+    const f32x4 lo = __builtin_bit_cast(f32x4, o.b[v]),
+                hi = __builtin_bit_cast(f32x4, o.b2[F32 ? v : 0]);
+    return u32x4{pack2(lo[0], lo[1]), pack2(lo[2], lo[3]), pack2(hi[0], hi[1]),
+                 pack2(hi[2], hi[3])};
+  };
+  if (s_begin < s_end) {
+    Step ahead[kAhead];
+#pragma unroll
+    for (int p = 0; p < kAhead; ++p) load(ahead[p]);
+    auto use = [&](const Step &o) {
+      for (int v = 0; v < 2; ++v) {
+        const u32x4 b = operand(o, v);
+        for (int t = 0; t < 2; ++t) acc[t][v] = mfma32(o.a[t], b, acc[t][v]);
+      }
+    };
+    int left = s_end - s_begin;
+    for (; left >= kAhead; left -= kAhead) {
+#pragma unroll
+      for (int p = 0; p < kAhead; ++p) {
+        use(ahead[p]);
+        load(ahead[p]);
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < kAhead - 1; ++p)
+      if (p < left) use(ahead[p]);
+  }
+  if (wk > 1) {
+    // partial sums of the other wavefronts of the tile, in their order
+    float *mine = s_part + (sub * (wk - 1) + ks - 1) * 1024;
+    if (ks > 0)
+      for (int t = 0; t < 4; ++t)
+        for (int i = 0; i < 4; ++i) mine[(4 * t + i) * 64 + lane] = acc[t >> 1][t & 1][i];
+    __syncthreads();
+    if (ks > 0) return;
+    for (int p = 1; p < wk; ++p) {
+      const float *other = s_part + (sub * (wk - 1) + p - 1) * 1024;
+      for (int t = 0; t < 4; ++t)
+        for (int i = 0; i < 4; ++i) acc[t >> 1][t & 1][i] += other[(4 * t + i) * 64 + lane];
+    }
+  }
+  if (!live) return;
+  // lane: channels c + 4q + 0..3 and c + 16 + 4q + 0..3 of pixels (y0 + v, x)
+  const bool xin = x < g.W;
+  const int c = 32 * ct;
+  float sum[2][8];
+  for (int v = 0; v < 2; ++v)
+    for (int i = 0; i < 8; ++i) sum[v][i] = acc[i >> 2][v][i & 3];
+  if (EP == EP_FORWARD) {
+    const f32x4 b0 = *(const f32x4 *)(o.bias + c + 4 * q),
+                b1 = *(const f32x4 *)(o.bias + c + 16 + 4 * q);
+    u32x4 z[2];
+    for (int v = 0; v < 2; ++v) {
+      for (int i = 0; i < 8; ++i)
+        sum[v][i] = fmaxf(sum[v][i] + (i < 4 ? b0[i & 3] : b1[i & 3]), 0.f);
+      z[v] = pack8(sum[v]);
+      if (xin && y0 + v < g.H) store8(o.g, o.out, o.planar, cout, n, y0 + v, x, c, q, z[v], true);
+    }
+    if (o.pooled != nullptr) {
+      // mean of the stored (rounded) values, in the order (0,0) (0,1) (1,0) (1,1)
+      float m[8];
+      for (int i = 0; i < 8; ++i) {
+        const float top = element(z[0], i), low = element(z[1], i);
+        const float top1 = lane_xor1(top), low1 = lane_xor1(low);
+        m[i] = 0.25f * (((top + top1) + low) + low1);
+      }
+      if (xin && !(col & 1))
+        store8(o.gp, o.pooled, o.pooled_planar, cout, n, y0 >> 1, x >> 1, c, q, pack8(m), true);
+    }
+    if (o.head_out != nullptr) {
+      const f32x4 h0 = *(const f32x4 *)(o.head_w + 4 * q),
+                  h1 = *(const f32x4 *)(o.head_w + 16 + 4 * q);
+      for (int v = 0; v < 2; ++v) {
+        float s = 0.f;
+        for (int i = 0; i < 8; ++i) s += element(z[v], i) * (i < 4 ? h0[i & 3] : h1[i & 3]);
+        // the wavefront's four quarters; 32 channels are one tile
+        s += __shfl_xor(s, 16, 64);
+        s += __shfl_xor(s, 32, 64);
+        if (q == 0 && xin && y0 + v < g.H) o.head_out[g.pixel(n, y0 + v, x)] = s + o.head_b[0];
+      }
+    }
+  } else if (EP == EP_PLAIN) {
+    for (int v = 0; v < 2; ++v) {
+      if (!xin || y0 + v >= g.H) continue;
+      const u32x4 m = *(const u32x4 *)(o.act + (long)g.pixel(n, y0 + v, x) * cout + c + 8 * q);
+      for (int i = 0; i < 8; ++i) sum[v][i] = element(m, i) > 0.f ? sum[v][i] : 0.f;
+      store8(o.g, o.out, o.planar, cout, n, y0 + v, x, c, q, pack8(sum[v]), false);
+    }
+  } else if (EP == EP_POOL) {
+    for (int v = 0; v < 2; ++v) {
+      if (!xin || y0 + v >= g.H) continue;
+      for (int f = 0; f < 4; ++f) {
+        const int fy = 2 * (y0 + v) + (f >> 1), fx = 2 * x + (f & 1);
+        const long p = (long)o.g.pixel(n, fy, fx) * cout + c + 8 * q;
+        const f32x4 s0 = *(const f32x4 *)(o.skip + p), s1 = *(const f32x4 *)(o.skip + p + 4);
+        const u32x4 m = *(const u32x4 *)(o.act + p);
+        float z[8];
+        for (int i = 0; i < 8; ++i)
+          z[i] = element(m, i) > 0.f ? (i < 4 ? s0[i & 3] : s1[i & 3]) + 0.25f * sum[v][i] : 0.f;
+        store8(o.g, o.out, o.planar, cout, n, fy, fx, c, q, pack8(z), false);
+      }
+    }
+  } else if (c < o.c0) {  // EP_CAT, upsampled part
+    float z[8];
+    for (int i = 0; i < 8; ++i) {
+      const float top1 = lane_xor1(sum[0][i]), low1 = lane_xor1(sum[1][i]);
+      z[i] = ((sum[0][i] + top1) + sum[1][i]) + low1;
+    }
+    if (xin && !(col & 1)) {
+      const u32x4 m =
+          *(const u32x4 *)(o.act + (long)o.g.pixel(n, y0 >> 1, x >> 1) * o.c0 + c + 8 * q);
+      for (int i = 0; i < 8; ++i)
+        if (!(element(m, i) > 0.f)) z[i] = 0.f;
+      store8(o.g, o.out, o.planar, o.c0, n, y0 >> 1, x >> 1, c, q, pack8(z), false);
+    }
+  } else if (xin) {  // EP_CAT, skip part, kept in the same channel order
+    for (int v = 0; v < 2; ++v)
+      if (y0 + v < g.H) {
+        float *p = o.skip + (long)g.pixel(n, y0 + v, x) * (cout - o.c0) + (c - o.c0) + 8 * q;
+        *(f32x4 *)p = f32x4{sum[v][0], sum[v][1], sum[v][2], sum[v][3]};
+        *(f32x4 *)(p + 4) = f32x4{sum[v][4], sum[v][5], sum[v][6], sum[v][7]};
+      }
+  }
+}
+
+// A forward layer. Its sums are not split: another order of a sum flips the
+// rounding and the ReLU of values near a tie, and the network carries that on.
+// One wavefront to a block up to 1024 tiles (four a CU), so that a deep
+// layer's few long sums have a CU's load path each and neighbouring XCDs read
+// different weights, else four (forward pass of 2 x 32 x 64: 236 us as blocks
+// of four, 197 so; of 2 x 128 x 256: 521, 493).
+template <bool F32, bool CAT>
+__global__ void __launch_bounds__(256) k_conv(ConvWork job) {
+  conv_block<EP_FORWARD, F32, CAT>(job, blockIdx.x, nullptr);
+}
+
+// Weight and bias gradients: gw[co][tap][ci] += sum over pixels of gz[co] x
+// input[ci, shifted by the tap]. Rows = 32 output channels, columns = 16
+// input channels, the reduction over pixels in steps of 32 (four groups of
+// eight consecutive pixels of a row, one group per quarter of the wavefront).
+// The three taps of a kernel row differ by one pixel, so a lane loads its
+// eight pixels and one on each side once and shifts them in registers: eleven
+// loads feed 18 MFMAs. A block's four wavefronts take `per_wave` steps each
+// and add up in LDS; the blocks' slices of the pixels are added by k_grad_sum
+// in their order, so that gradients are the same in every run. Blocks of input
+// tile 0 also sum gz itself (a product with ones) for the bias. What bounds it
+// is the latency of its few steps at the small grids, the loads' L2 traffic at
+// the large ones. Per layer, 8 x 128 x 256: 296 -> 39 us, 8 x 32 x 64: 66 -> 11
+// (before: 2-byte gathers, atomics).
+struct GradIn {
+  const uint16_t *src0 = nullptr, *src1 = nullptr;  // planar; src0 at half resolution
+  Grid g0;                                           // of src0
+  int c0 = 0, c1 = 0;
+};
+
+constexpr int kGradLds = 18 * 256 + 32;  // floats of a block
+
+struct GradWork {
+  GradIn in;
+  Grid g;
+  const uint16_t *gz;  // planar
+  int cout, per_wave, blocks;
+  float *part;         // [slice][weights, bias] partial sums
+};
+
+__device__ inline void wgrad_block(const GradWork &job, int block, float *s_sum) {
+  const GradIn &in = job.in;
+  const Grid &g = job.g;
+  const uint16_t *__restrict__ gz = job.gz;
+  const int per_wave = job.per_wave;
   const int cin = in.c0 + in.c1;
-  const int M = N * H * W;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int row = lane & 15, kq = (lane >> 4) * 4;
-  const int m = blockIdx.x * 64 + wave * 16 + row;
-  const int mm = m < M ? m : 0;
-  const int n = mm / (H * W), y = (mm / W) % H, x = mm % W;
-  const int co0 = blockIdx.y * 64;
-  const int nsub = min(4, (cout - co0) / 16);
-  f32x4 acc[4];
-  for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int ky = 0; ky < 3; ++ky) {
-    const int yy = y + ky - 1;
-    for (int kx = 0; kx < 3; ++kx) {
-      const int xx = wrap(x + kx - 1, W);
-      const long kbase = (long)(ky * 3 + kx) * cin;
-      for (int ci0 = 0; ci0 < cin; ci0 += 16) {
-        const bf16x4 a = load_in4(in, n, yy, xx, H, W, ci0 + kq);
-        for (int t = 0; t < 4; ++t) {
-          if (t >= nsub) break;
-          const int co = co0 + 16 * t + row;
-          const bf16x4 b = *(const bf16x4 *)(w + (long)co * 9 * cin + kbase + ci0 + kq);
-          acc[t] = mfma16(a, b, acc[t]);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 15, q = lane >> 4;
+  const int ctiles = cin / 16, tile = block % (ctiles * (job.cout / 32));
+  const int slice = block / (ctiles * (job.cout / 32));
+  const int ci0 = (tile % ctiles) * 16, co0 = (tile / ctiles) * 32;
+  const int xg_n = g.wp >> 3, groups = g.N * g.H * xg_n;
+  const int step0 = (slice * 4 + wave) * per_wave;
+  const bool up = ci0 < in.c0;  // a tile lies in one part
+  const int ci = ci0 + col;
+  f32x4 acc[2][9], bsum[2];
+  for (int t = 0; t < 2; ++t) {
+    bsum[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < 9; ++k) acc[t][k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  // this quarter's group of eight pixels: (n, y, xg)
+  int gi = step0 * 4 + q;
+  int xg = gi % xg_n, y = (gi / xg_n) % g.H, n = gi / (xg_n * g.H);
+  const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+  for (int s = 0; s < per_wave; ++s, gi += 4) {
+    if (4 * (step0 + s) >= groups) break;  // uniform
+    const bool in_range = gi < groups;
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    u32x4 a[2] = {zero, zero}, mid[3] = {zero, zero, zero};
+    uint32_t left[3] = {0u, 0u, 0u}, right[3] = {0u, 0u, 0u};
+    if (in_range) {
+      for (int t = 0; t < 2; ++t)
+        a[t] = *(const u32x4 *)(gz + g.plane(co0 + 16 * t + col, n, y) + 8 * xg);
+      const bool last = 8 * xg + 8 >= g.W;  // right neighbour wraps (or is pad)
+      for (int ky = 0; ky < 3; ++ky) {
+        const int yy = y + ky - 1;
+        if (yy < 0 || yy >= g.H) continue;
+        if (up) {
+          const uint16_t *p = in.src0 + in.g0.plane(ci, n, yy >> 1);
+          const u32x2 e = *(const u32x2 *)(p + 4 * xg);
+          mid[ky] = u32x4{(e[0] & 0xffffu) * 0x10001u, (e[0] >> 16) * 0x10001u,
+                          (e[1] & 0xffffu) * 0x10001u, (e[1] >> 16) * 0x10001u};
+          left[ky] = p[xg == 0 ? in.g0.W - 1 : 4 * xg - 1];
+          right[ky] = p[last ? 0 : 4 * xg + 4];
+        } else {
+          const uint16_t *p = in.src1 + g.plane(ci - in.c0, n, yy);
+          mid[ky] = *(const u32x4 *)(p + 8 * xg);
+          left[ky] = p[xg == 0 ? g.W - 1 : 8 * xg - 1];
+          right[ky] = p[last ? 0 : 8 * xg + 8];
         }
       }
     }
-  }
-  for (int t = 0; t < nsub; ++t) {
-    const int co = co0 + 16 * t + row;
-    const float bco = bias != nullptr ? bias[co] : 0.f;
-    for (int i = 0; i < 4; ++i) {
-      const int p = blockIdx.x * 64 + wave * 16 + kq + i;
-      if (p >= M) continue;
-      float v = acc[t][i] + bco;
-      if (relu) v = fmaxf(v, 0.f);
-      if (out_bf != nullptr) out_bf[(long)p * cout + co] = to_bf16(v);
-      else out_f[(long)p * cout + co] = v;
+    if (ci0 == 0)
+      for (int t = 0; t < 2; ++t) bsum[t] = mfma32(a[t], ones, bsum[t]);
+    for (int ky = 0; ky < 3; ++ky) {
+      const u32x4 m = mid[ky];
+      const uint32_t m01 = __builtin_amdgcn_alignbit(m[1], m[0], 16),
+                     m12 = __builtin_amdgcn_alignbit(m[2], m[1], 16),
+                     m23 = __builtin_amdgcn_alignbit(m[3], m[2], 16);
+      const u32x4 b[3] = {u32x4{(m[0] << 16) | left[ky], m01, m12, m23}, m,
+                          u32x4{m01, m12, m23, (m[3] >> 16) | (right[ky] << 16)}};
+      for (int kx = 0; kx < 3; ++kx)
+        for (int t = 0; t < 2; ++t)
+          acc[t][3 * ky + kx] = mfma32(a[t], b[kx], acc[t][3 * ky + kx]);
     }
-  }
-}
-
-// Weight gradient: gw[co][k] += sum_m gz[m][co] A[m][k] over the pixel
-// chunk [blockIdx.z * chunk, +chunk). GEMM rows = co (A operand gz^T),
-// columns = k (B operand = input patch), reduction over pixels. A block of
-// 256 threads owns 64 co x 64 k; wave w owns co rows 16w..16w+15. The
-// block's partial sums are added to gw with fp32 atomics.
-__global__ void __launch_bounds__(256) k_wgrad3(ConvIn in, int N, int H, int W,
-                                                const uint16_t *gz, int cout, float *gw,
-                                                int chunk) {
-  const int cin = in.c0 + in.c1;
-  const int K = 9 * cin;
-  const int M = N * H * W;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int row = lane & 15, kq = (lane >> 4) * 4;
-  const int k0 = blockIdx.x * 64;
-  const int co = blockIdx.y * 64 + wave * 16 + row;  // A-operand row of this lane
-  const bool co_ok = blockIdx.y * 64 + wave * 16 < cout;
-  const int nsub = min(4, (K - k0) / 16);
-  if (!co_ok) return;
-  // this lane's B-operand columns (one per sub-tile): k -> (ky, kx, ci)
-  int kky[4], kkx[4], kci[4];
-  for (int t = 0; t < 4; ++t) {
-    const int k = k0 + 16 * t + row;
-    const int kk = k < K ? k : 0;
-    const int tap = kk / cin;
-    kky[t] = tap / 3;
-    kkx[t] = tap % 3;
-    kci[t] = kk - tap * cin;
-  }
-  f32x4 acc[4];
-  for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int m_begin = blockIdx.z * chunk, m_end = min(M, m_begin + chunk);
-  for (int m0 = m_begin; m0 < m_end; m0 += 16) {
-    bf16x4 a;
-    int pn[4], py[4], px[4];
-    for (int i = 0; i < 4; ++i) {
-      const int m = m0 + kq + i;
-      const bool ok = m < m_end;
-      const int mm = ok ? m : m_begin;
-      a[i] = ok ? (short)gz[(long)mm * cout + co] : (short)0;
-      pn[i] = mm / (H * W);
-      py[i] = (mm / W) % H;
-      px[i] = ok ? mm % W : -1000000;  // marks a padding pixel
-    }
-    for (int t = 0; t < nsub; ++t) {
-      bf16x4 b;
-      for (int i = 0; i < 4; ++i) {
-        if (px[i] < -1000) {
-          b[i] = 0;
-          continue;
-        }
-        const int yy = py[i] + kky[t] - 1, xx = wrap(px[i] + kkx[t] - 1, W);
-        b[i] = (short)load_in1(in, pn[i], yy, xx, H, W, kci[t]);
+    xg += 4;
+    while (xg >= xg_n) {
+      xg -= xg_n;
+      if (++y == g.H) {
+        y = 0;
+        ++n;
       }
-      acc[t] = mfma16(a, b, acc[t]);
     }
   }
-  // D[co = 4(l/16)+i][k = l%16] within the wave's 16 x 64 strip
-  for (int t = 0; t < nsub; ++t) {
-    const int k = k0 + 16 * t + row;
-    for (int i = 0; i < 4; ++i) {
-      const int c = blockIdx.y * 64 + wave * 16 + kq + i;
-      if (c < cout && k < K) atomicAdd(&gw[(long)c * K + k], acc[t][i]);
+  // element i of a sum: output channel 16 t + 4 q + i, input channel col; the
+  // wavefronts add theirs in turn
+  for (int turn = 0; turn < 4; ++turn) {
+    if (wave == turn) {
+      for (int t = 0; t < 2; ++t)
+        for (int k = 0; k < 9; ++k)
+          for (int i = 0; i < 4; ++i) {
+            float *e = &s_sum[((16 * t + 4 * q + i) * 9 + k) * 16 + col];
+            *e = turn == 0 ? acc[t][k][i] : *e + acc[t][k][i];
+          }
+      if (col == 0)
+        for (int t = 0; t < 2; ++t)
+          for (int i = 0; i < 4; ++i) {
+            float *e = &s_sum[18 * 256 + 16 * t + 4 * q + i];
+            *e = turn == 0 ? bsum[t][i] : *e + bsum[t][i];
+          }
     }
+    __syncthreads();
   }
-}
-
-// Bias gradient: gb[co] += sum over the pixel chunk of gz[m][co].
-__global__ void k_colsum(const uint16_t *gz, int M, int cout, float *gb, int chunk) {
-  const int co = threadIdx.x;
-  if (co >= cout) return;
-  const int m0 = blockIdx.x * chunk, m1 = min(M, m0 + chunk);
-  float s = 0.f;
-  for (int m = m0; m < m1; ++m) s += from_bf16(gz[(long)m * cout + co]);
-  atomicAdd(&gb[co], s);
-}
-
-// gz = bf16(g * (act > 0))
-__global__ void k_relu_grad(const float *g, const uint16_t *act, long count, uint16_t *gz) {
-  const long t = gtid();
-  if (t >= count) return;
-  gz[t] = to_bf16(from_bf16(act[t]) > 0.f ? g[t] : 0.f);
-}
-
-// 2x2 mean pool, bf16 in and out; (N, H, W) is the input grid.
-__global__ void k_pool(const uint16_t *in, int N, int H, int W, int C, uint16_t *out) {
-  const long t = gtid();
-  const int h2 = H >> 1, w2 = W >> 1;
-  if (t >= (long)N * h2 * w2 * C) return;
-  const int c = (int)(t % C);
-  const long p = t / C;
-  const int x = (int)(p % w2), y = (int)((p / w2) % h2), n = (int)(p / ((long)w2 * h2));
-  float s = 0.f;
-  for (int dy = 0; dy < 2; ++dy)
-    for (int dx = 0; dx < 2; ++dx)
-      s += from_bf16(in[(((long)n * H + 2 * y + dy) * W + 2 * x + dx) * C + c]);
-  out[t] = to_bf16(0.25f * s);
-}
-
-// g_fine[n,y,x,c] += 0.25 g_coarse[n,y/2,x/2,c] (pool backward), fine grid.
-__global__ void k_pool_back(const float *gc, int N, int H, int W, int C, float *gf) {
-  const long t = gtid();
-  if (t >= (long)N * H * W * C) return;
-  const int c = (int)(t % C);
-  const long p = t / C;
-  const int x = (int)(p % W), y = (int)((p / W) % H), n = (int)(p / ((long)W * H));
-  gf[t] += 0.25f * gc[(((long)n * (H >> 1) + (y >> 1)) * (W >> 1) + (x >> 1)) * C + c];
-}
-
-// Split the input gradient of a decoder conv (fine grid N x H x W, c0 + c1
-// channels): the upsampled part sums over each 2x2 block into the coarse
-// tensor's gradient, the skip part adds to the skip's gradient.
-__global__ void k_split_back(const float *gcat, int N, int H, int W, int c0, int c1,
-                             float *gcoarse, float *gskip) {
-  const long t = gtid();
-  const int h2 = H >> 1, w2 = W >> 1;
-  const long ncoarse = (long)N * h2 * w2 * c0;
-  const long nskip = (long)N * H * W * c1;
-  const int cin = c0 + c1;
-  if (t < ncoarse) {
-    const int c = (int)(t % c0);
-    const long p = t / c0;
-    const int x = (int)(p % w2), y = (int)((p / w2) % h2), n = (int)(p / ((long)w2 * h2));
-    float s = 0.f;
-    for (int dy = 0; dy < 2; ++dy)
-      for (int dx = 0; dx < 2; ++dx)
-        s += gcat[(((long)n * H + 2 * y + dy) * W + 2 * x + dx) * cin + c];
-    gcoarse[t] += s;
-  } else if (t < ncoarse + nskip) {
-    const long u = t - ncoarse;
-    const int c = (int)(u % c1);
-    const long p = u / c1;
-    gskip[u] += gcat[p * cin + c0 + c];
+  const long weights = 9L * cin * job.cout;
+  float *part = job.part + slice * (weights + job.cout);
+  for (int t = threadIdx.x; t < 18 * 256; t += 256) {
+    const int co = co0 + t / 144, k = (t / 16) % 9;
+    part[((long)co * 9 + k) * cin + ci0 + (t & 15)] = s_sum[t];
   }
+  if (ci0 == 0 && threadIdx.x < 32) part[weights + co0 + threadIdx.x] = s_sum[18 * 256 + threadIdx.x];
 }
 
-__global__ void k_add(const float *a, long count, float *out) {
-  const long t = gtid();
-  if (t < count) out[t] += a[t];
+__global__ void __launch_bounds__(256) k_wgrad(GradWork job) {
+  __shared__ float lds[kGradLds];
+  wgrad_block(job, blockIdx.x, lds);
+}
+
+// Both products of a layer's backward pass, which need only the masked
+// gradient of its output, in one launch: the weight gradient's blocks first,
+// then the input gradient's convolution (20 training steps of 8 x 32 x 64:
+// 13.3 -> 11.1 ms against two launches, 8 x 128 x 256 the same within 1 %).
+template <int EP>
+__global__ void __launch_bounds__(256) k_backward(GradWork grad, ConvWork conv) {
+  __shared__ float lds[kGradLds > kConvLds ? kGradLds : kConvLds];
+  if ((int)blockIdx.x < grad.blocks)
+    wgrad_block(grad, blockIdx.x, lds);
+  else
+    conv_block<EP, false, false>(conv, blockIdx.x - grad.blocks, lds);
+}
+
+// gradients = the slices' partial sums of every convolution parameter, in the
+// slices' order (the head's are k_head_sum's).
+struct SliceTable {
+  int begin[kLayerCount + 1];     // the layers' first parameters
+  int slices[kLayerCount];
+  long part[kLayerCount];         // their partial sums
+};
+__global__ void __launch_bounds__(256) k_grad_sum(const float *part, SliceTable table,
+                                                  float *grads) {
+  const int t = (int)gtid();
+  if (t >= table.begin[kLayerCount]) return;
+  int l = 0;
+  while (l + 1 < kLayerCount && t >= table.begin[l + 1]) ++l;
+  const int size = table.begin[l + 1] - table.begin[l];
+  const float *p = part + table.part[l] + (t - table.begin[l]);
+  float s = 0.f;
+  for (int q = 0; q < table.slices[l]; ++q) s += p[(long)q * size];
+  grads[t] = s;
+}
+
+// fp32 features to the planar bf16 input (the first layer's weight gradient):
+// a block transposes 64 pixels of a row through LDS.
+__global__ void __launch_bounds__(256) k_planar_input(const float *in, Grid g, uint16_t *out) {
+  __shared__ uint16_t s[64][kInChannels + 2];
+  const int xt = (g.W + 63) / 64;
+  const int x0 = (blockIdx.x % xt) * 64, row = blockIdx.x / xt;  // row = n H + y
+  const int nx = min(64, g.W - x0);
+  for (int t = threadIdx.x; t < nx * kInChannels; t += 256)
+    s[t / kInChannels][t % kInChannels] =
+        to_bf16(in[((long)row * g.W + x0) * kInChannels + t]);
+  __syncthreads();
+  const int n = row / g.H, y = row % g.H, x = threadIdx.x & 63;
+  if (x >= nx) return;
+  for (int c = threadIdx.x >> 6; c < kInChannels; c += 4) {
+    uint16_t *p = out + g.plane(c, n, y);
+    p[x0 + x] = s[x][c];
+    if (x0 + x == 0 && g.W < g.wp) p[g.W] = s[x][c];
+  }
 }
 
 __global__ void k_fill(float *p, long count, float v) {
@@ -285,35 +580,51 @@ __global__ void k_fill(float *p, long count, float v) {
   if (t < count) p[t] = v;
 }
 
-// 1x1 head: out[m] = sum_c act[m][c] w[c] + b (fp32 out).
-__global__ void k_head(const uint16_t *act, int M, int C, const float *w, const float *b,
-                       float *out) {
-  const long m = gtid();
-  if (m >= M) return;
-  float s = 0.f;
-  for (int c = 0; c < C; ++c) s += from_bf16(act[m * C + c]) * w[c];
-  out[m] = s + b[0];
+// Head backward: gz = bf16(g w, masked by act > 0), gw[c] += sum g act[c], gb
+// += sum g. Four threads per pixel, eight channels each.
+// Each block leaves its 33 sums in part and k_head_sum adds them up: 256 blocks'
+// atomics on 33 neighbouring words took 86 us.
+__global__ void __launch_bounds__(256) k_head_back(const uint16_t *act, const float *gout, Grid g,
+                                                   const float *w, uint16_t *gz,
+                                                   uint16_t *gz_planar, float *part) {
+  // wavefront q of the block: channels 4q .. + 3 and 16 + 4q .. + 3
+  const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int M = g.N * g.H * g.W;
+  float sum[8], total = 0.f, hw[8];
+  for (int i = 0; i < 8; ++i) {
+    sum[i] = 0.f;
+    hw[i] = w[(i < 4 ? i : 12 + i) + 4 * q];
+  }
+  for (int m = blockIdx.x * 64 + lane; m < M; m += gridDim.x * 64) {
+    const float gm = gout[m];
+    const u32x4 v = *(const u32x4 *)(act + (long)m * kHeadIn + 8 * q);
+    float z[8];
+    for (int i = 0; i < 8; ++i) {
+      const float a = element(v, i);
+      sum[i] += gm * a;
+      z[i] = a > 0.f ? gm * hw[i] : 0.f;
+    }
+    total += gm;
+    const int x = m % g.W, y = (m / g.W) % g.H, n = m / (g.W * g.H);
+    store8(g, gz, gz_planar, kHeadIn, n, y, x, 0, q, pack8(z), false);
+  }
+  for (int i = 0; i < 8; ++i) {
+    float s = sum[i];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+    if (lane == 0) part[blockIdx.x * (kHeadIn + 1) + (i < 4 ? i : 12 + i) + 4 * q] = s;
+  }
+  if (q == 0) {
+    for (int off = 32; off > 0; off >>= 1) total += __shfl_down(total, off, 64);
+    if (lane == 0) part[blockIdx.x * (kHeadIn + 1) + kHeadIn] = total;
+  }
 }
 
-// Head backward: g_act[m][c] = g[m] w[c]; gw[c] += sum g[m] act[m][c];
-// gb += sum g[m] (block partials, then atomics).
-__global__ void k_head_back(const uint16_t *act, const float *g, int M, int C, const float *w,
-                            float *gact, float *gw, float *gb) {
-  __shared__ float red[kT];
-  const long m = gtid();
-  const float gm = m < M ? g[m] : 0.f;
-  if (m < M)
-    for (int c = 0; c < C; ++c) gact[m * C + c] = gm * w[c];
-  for (int c = 0; c <= C; ++c) {
-    red[threadIdx.x] = m < M ? (c < C ? gm * from_bf16(act[m * C + c]) : gm) : 0.f;
-    __syncthreads();
-    for (int s = kT / 2; s > 0; s >>= 1) {
-      if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) atomicAdd(c < C ? &gw[c] : gb, red[0]);
-    __syncthreads();
-  }
+// gw and gb follow each other in the parameters' order: one wavefront each.
+__global__ void __launch_bounds__(64) k_head_sum(const float *part, int blocks, float *gw) {
+  float s = 0.f;
+  for (int b = threadIdx.x; b < blocks; b += 64) s += part[b * (kHeadIn + 1) + blockIdx.x];
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+  if (threadIdx.x == 0) gw[blockIdx.x] = s;
 }
 
 // Mean square error: loss += sum (out - target)^2 / M; g = 2 (out - target) / M.
@@ -371,8 +682,37 @@ __global__ void k_mse_rel(const float *out, const float *target, int B, int P,
   if (threadIdx.x == 0) atomicAdd(loss, red[0]);
 }
 
+// Where each convolution's weights live: [cout][9][cin] at w in the
+// parameters, and at `packed` in the two bf16 copies in operand order.
+struct PackTable {
+  int w[kLayerCount], packed[kLayerCount], cin[kLayerCount], cout[kLayerCount];
+};
+
+// bf16 copies of parameter t (a convolution weight) in the order k_conv reads:
+// [16 output channels][step of 32 k][lane][8], k = (tap, input channel), lane
+// l holding output channel l % 16 and input channels 4q .. + 3 and 16 + 4q .. +
+// 3 of the step's 32, q = l / 16. `back` is the
+// input gradient's convolution: channels exchanged, taps reversed.
+__device__ inline void pack_weight(const PackTable &p, int t, float v, uint16_t *fwd,
+                                   uint16_t *back) {
+  int l = 0;
+  while (l + 1 < kLayerCount && t >= p.w[l + 1]) ++l;
+  const int cin = p.cin[l], cout = p.cout[l], r = t - p.w[l];
+  if (r >= cout * 9 * cin) return;  // a bias
+  const int ci = r % cin, tap = (r / cin) % 9, co = r / (9 * cin);
+  const uint16_t b = to_bf16(v);
+  auto at = [](int row, int tp, int c, int channels) {
+    const int spt = channels >> 5, step = tp * spt + (c >> 5);
+    const int lane = (row & 15) + 16 * ((c >> 2) & 3), e = (c & 3) + 4 * ((c >> 4) & 1);
+    return (((row >> 4) * 9 * spt + step) * 64 + lane) * 8 + e;
+  };
+  fwd[p.packed[l] + at(co, tap, ci, cin)] = b;
+  back[p.packed[l] + at(ci, 8 - tap, co, cout)] = b;
+}
+
 __global__ void k_adam(float *p, const float *g, float *mo, float *ve, long count, float lr,
-                       float b1, float b2, float c1, float c2, float eps) {
+                       float b1, float b2, float c1, float c2, float eps, PackTable table,
+                       uint16_t *fwd, uint16_t *back) {
   const long t = gtid();
   if (t >= count) return;
   const float gt = g[t];
@@ -380,26 +720,15 @@ __global__ void k_adam(float *p, const float *g, float *mo, float *ve, long coun
   const float v = b2 * ve[t] + (1.f - b2) * gt * gt;
   mo[t] = m;
   ve[t] = v;
-  p[t] -= lr * (m / c1) / (sqrtf(v / c2) + eps);
+  const float w = p[t] - lr * (m / c1) / (sqrtf(v / c2) + eps);
+  p[t] = w;
+  pack_weight(table, (int)t, w, fwd, back);
 }
 
-// bf16 weights [cout][9][cin] and the flipped, transposed copy
-// [cin][9][cout] (tap (ky, kx) -> (2 - ky, 2 - kx)) used by the input grad.
-__global__ void k_prep_weights(const float *w, int cin, int cout, uint16_t *wb,
-                               uint16_t *wf) {
+__global__ void k_pack_weights(const float *p, long count, PackTable table, uint16_t *fwd,
+                               uint16_t *back) {
   const long t = gtid();
-  if (t >= (long)cout * 9 * cin) return;
-  const int ci = (int)(t % cin);
-  const int tap = (int)((t / cin) % 9);
-  const int co = (int)(t / (9L * cin));
-  const uint16_t v = to_bf16(w[t]);
-  wb[t] = v;
-  wf[((long)ci * 9 + (8 - tap)) * cout + co] = v;
-}
-
-__global__ void k_to_bf16(const float *in, long count, uint16_t *out) {
-  const long t = gtid();
-  if (t < count) out[t] = to_bf16(in[t]);
+  if (t < count) pack_weight(table, (int)t, p[t], fwd, back);
 }
 
 // GEMM check of the MFMA operand layout: C[M][N] = A[M][K] B[K][N], bf16 in
@@ -420,6 +749,13 @@ __global__ void k_gemm_check(const uint16_t *A, const uint16_t *B, int M, int N,
   }
   for (int i = 0; i < 4; ++i) C[(long)(m0 + kq + i) * N + n0 + row] = acc[i];
 }
+
+// Wavefronts of a weight-gradient launch over all its tiles: fewer leave the
+// chip idle, more write and read more partial sums (8 samples of 128 x 256,
+// loss and gradients with transfers: 512 3.65 ms, 1024 3.48, 2048 3.62, 4096
+// 3.80; of 32 x 64: 1.09, 1.07, 1.12, 1.11).
+constexpr int kGradWaves = 1024;
+constexpr int kHeadBlocks = 512;  // most blocks of k_head_back
 
 unsigned nb(long n, int t = kT) { return (unsigned)((n + t - 1) / t); }
 
@@ -453,6 +789,27 @@ static int act_level(int a) {
 }
 static int act_channels(int a) { return a == 0 ? kInChannels : kLayers[a - 1].cout; }
 
+static Grid grid_of(const Net &n, int level, int batch) {
+  Grid g;
+  g.N = batch;
+  g.H = n.H >> level;
+  g.W = n.W >> level;
+  g.wp = (g.W + 7) / 8 * 8;
+  g.batches = n.max_batch;
+  return g;
+}
+
+static PackTable pack_table(const Net &n) {
+  PackTable t;
+  for (int l = 0; l < kLayerCount; ++l) {
+    t.w[l] = (int)n.w_off[l];
+    t.packed[l] = (int)n.wbf_off[l];
+    t.cin[l] = kLayers[l].cin;
+    t.cout[l] = kLayers[l].cout;
+  }
+  return t;
+}
+
 Net::~Net() {
   for (void *p : allocations) (void)hipFree(p);
 }
@@ -465,6 +822,23 @@ static T *dalloc(Net &net, size_t count) {
   if (hipMalloc(&p, count * sizeof(T)) != hipSuccess) p = nullptr;
   net.allocations.push_back(p);
   return (T *)p;
+}
+
+// The pixel slices of a layer's weight gradient: blocks of four wavefronts of
+// per_wave steps, about kGradWaves wavefronts over all tiles of the layer.
+static int grad_slices(const Net &n, int l, int batch, int &per_wave) {
+  const LayerSpec &L = kLayers[l];
+  const Grid g = grid_of(n, act_level(l + 1), batch);
+  const int tiles = (L.cin / 16) * (L.cout / 32);
+  const int steps = (g.N * g.H * (g.wp / 8) + 3) / 4;
+  const int waves = std::max(4, kGradWaves / tiles);  // per tile
+  per_wave = std::max(2, (steps + waves - 1) / waves);
+  return (steps + 4 * per_wave - 1) / (4 * per_wave);
+}
+
+// Zero bf16 values (an even number of them, in memory of whole words).
+static void fill_zero(Net &n, uint16_t *p, long count) {
+  k_fill<<<nb(count / 2), kT, 0, n.stream>>>((float *)p, count / 2, 0.f);
 }
 
 Net *create(int H, int W, int max_batch, uint64_t seed) {
@@ -503,30 +877,42 @@ Net *create(int H, int W, int max_batch, uint64_t seed) {
     n.wbf_off[l] = wo;
     wo += (size_t)kLayers[l].cout * 9 * kLayers[l].cin;
   }
-  long max_scratch = 0;
+  // activations and masked gradients, NHWC and planar (with zeroed pads);
+  // activation 0, the input, has no gradient and no NHWC copy
   for (int a = 0; a < kActs; ++a) {
-    const int lv = act_level(a);
-    const long pix = (long)max_batch * (H >> lv) * (W >> lv);
-    n.act[a] = dalloc<uint16_t>(n, pix * act_channels(a));
-    n.gact[a] = dalloc<float>(n, pix * act_channels(a));
-  }
-  for (int l = 0; l < kLayerCount; ++l) {
-    const int lv = act_level(l + 1);
-    const long pix = (long)max_batch * (H >> lv) * (W >> lv);
-    max_scratch = std::max(max_scratch, pix * (long)kLayers[l].cin);
-    max_scratch = std::max(max_scratch, pix * (long)kLayers[l].cout);
+    const Grid g = grid_of(n, act_level(a), max_batch);
+    const long pix = (long)max_batch * g.H * g.W * act_channels(a);
+    const long planar = (long)max_batch * g.H * g.wp * act_channels(a);
+    n.act_planar[a] = dalloc<uint16_t>(n, planar);
+    n.planar_count[a] = planar;
+    if (a == 0) continue;
+    n.act[a] = dalloc<uint16_t>(n, pix);
+    n.gz[a] = dalloc<uint16_t>(n, pix);
+    n.gz_planar[a] = dalloc<uint16_t>(n, planar);
   }
   for (int p = 0; p < 3; ++p) {
-    const long pix = (long)max_batch * (H >> (p + 1)) * (W >> (p + 1));
-    n.pooled[p] = dalloc<uint16_t>(n, pix * kLayers[2 * p + 1].cout);
+    const Grid g = grid_of(n, p + 1, max_batch);
+    const int ch = kLayers[2 * p + 1].cout;
+    n.pooled[p] = dalloc<uint16_t>(n, (long)max_batch * g.H * g.W * ch);
+    n.pooled_planar[p] = dalloc<uint16_t>(n, (long)max_batch * g.H * g.wp * ch);
+    n.skip[p] = dalloc<float>(n, (long)max_batch * 4 * g.H * g.W * ch);
   }
-  n.scratch = dalloc<float>(n, max_scratch);
-  n.gz = dalloc<uint16_t>(n, max_scratch);
   const long pix0 = (long)max_batch * H * W;
   n.out = dalloc<float>(n, pix0);
   n.gout = dalloc<float>(n, pix0);
   n.target = dalloc<float>(n, pix0);
   n.input = dalloc<float>(n, pix0 * kInChannels);
+  long part = 0;
+  for (int l = 0; l < kLayerCount; ++l) {
+    const long size = (long)kLayers[l].cout * (9 * kLayers[l].cin + 1);
+    int most = 0, per_wave;
+    for (int b = 1; b <= max_batch; ++b) most = std::max(most, grad_slices(n, l, b, per_wave));
+    n.part_off[l] = part;
+    part += size * most;
+  }
+  n.grad_part = dalloc<float>(n, part);
+  n.zero = dalloc<uint16_t>(n, 32);
+  n.head_part = dalloc<float>(n, kHeadBlocks * (kHeadIn + 1));
   n.loss = dalloc<float>(n, 1);
   n.energy = dalloc<float>(n, max_batch);
   for (void *p : n.allocations)
@@ -540,6 +926,15 @@ Net *create(int H, int W, int max_batch, uint64_t seed) {
     delete net;
     return nullptr;
   }
+  for (int a = 0; a < kActs; ++a) {
+    fill_zero(n, n.act_planar[a], n.planar_count[a]);
+    if (a > 0) fill_zero(n, n.gz_planar[a], n.planar_count[a]);
+  }
+  for (int p = 0; p < 3; ++p) {
+    const Grid g = grid_of(n, p + 1, max_batch);
+    fill_zero(n, n.pooled_planar[p], (long)max_batch * g.H * g.wp * kLayers[2 * p + 1].cout);
+  }
+  fill_zero(n, n.zero, 32);
   // He-normal conv weights, zero biases, a small head
   std::mt19937_64 rng(seed);
   std::normal_distribution<float> normal(0.f, 1.f);
@@ -564,11 +959,8 @@ void destroy(Net *net) {
 }
 
 static int prep_weights(Net &n) {
-  for (int l = 0; l < kLayerCount; ++l) {
-    const LayerSpec &L = kLayers[l];
-    k_prep_weights<<<nb((long)L.cout * 9 * L.cin), kT, 0, n.stream>>>(
-        n.params + n.w_off[l], L.cin, L.cout, n.wbf + n.wbf_off[l], n.wflip + n.wbf_off[l]);
-  }
+  k_pack_weights<<<nb((long)n.param_count), kT, 0, n.stream>>>(
+      n.params, (long)n.param_count, pack_table(n), n.wbf, n.wflip);
   GCS_HIP(hipGetLastError());
   return 0;
 }
@@ -602,7 +994,10 @@ int get_array(Net &n, int which, float *host, size_t count) {
 static ConvIn layer_input(const Net &n, int l) {
   const LayerSpec &L = kLayers[l];
   ConvIn in;
-  if (L.kind == IN_PLAIN) {
+  if (l == 0) {
+    in.f32 = n.input;
+    in.c1 = L.cin;
+  } else if (L.kind == IN_PLAIN) {
     in.src1 = n.act[L.src];
     in.c1 = L.cin;
   } else if (L.kind == IN_POOL) {
@@ -611,89 +1006,163 @@ static ConvIn layer_input(const Net &n, int l) {
   } else {
     in.src0 = n.act[L.src];
     in.c0 = act_channels(L.src);
-    in.up0 = 1;
     in.src1 = n.act[L.src2];
     in.c1 = act_channels(L.src2);
   }
   return in;
 }
 
+static int conv_tiles(const ConvWork &job) {
+  return (job.cout / 32) * ((job.g.W + 15) / 16) * ((job.g.H + 1) / 2) * job.g.N;
+}
+
+// An input gradient's wavefronts that share one tile's sum: until the launch
+// has about two per SIMD, a layer's few tiles are split along k, but into no
+// less than five steps each (20 training steps of 8 x 32 x 64: not split 12.3
+// ms, split 11.8; down to one step it is no faster, and short sums' rounding
+// stays that of one chain).
+static int split_k(int tiles, int steps) {
+  int wk = tiles >= 2048 ? 1 : tiles >= 1024 ? 2 : 4;
+  while (wk > 1 && steps / wk < 5) wk /= 2;
+  return wk;
+}
+
+static ConvWork conv_work(const ConvIn &in, const uint16_t *zero, const Grid &g, int cout,
+                          const uint16_t *w, const ConvOut &o) {
+  ConvWork job;
+  job.in = in;
+  job.in.zero = zero;
+  job.g = g;
+  job.cout = cout;
+  job.wk = 1;
+  job.w = w;
+  job.o = o;
+  return job;
+}
+
 // Forward pass over `batch` samples whose fp32 input features are already
 // in n.input ([N][H][W][kInChannels]); output in n.out.
 int forward_device(Net &n, int batch) {
-  hipStream_t s = n.stream;
-  const long pix0 = (long)batch * n.H * n.W;
-  k_to_bf16<<<nb(pix0 * kInChannels), kT, 0, s>>>(n.input, pix0 * kInChannels, n.act[0]);
   for (int l = 0; l < kLayerCount; ++l) {
     const LayerSpec &L = kLayers[l];
     const int lv = act_level(l + 1);
-    const int H = n.H >> lv, W = n.W >> lv;
-    if (L.kind == IN_POOL) {
-      const int src = L.src;  // the pre-pool activation at level lv - 1
-      k_pool<<<nb((long)batch * H * W * L.cin), kT, 0, s>>>(
-          n.act[src], batch, H * 2, W * 2, L.cin, n.pooled[(l - 2) / 2]);
-    }
     const ConvIn in = layer_input(n, l);
-    const long M = (long)batch * H * W;
-    k_conv3<<<dim3(nb(M, 64), (L.cout + 63) / 64), 256, 0, s>>>(
-        in, batch, H, W, n.wbf + n.wbf_off[l], n.params + n.b_off[l], L.cout, 1,
-        n.act[l + 1], nullptr);
+    ConvOut o;
+    o.g = grid_of(n, lv, batch);
+    o.out = n.act[l + 1];
+    o.planar = n.act_planar[l + 1];
+    o.bias = n.params + n.b_off[l];
+    if (l + 1 < kLayerCount && kLayers[l + 1].kind == IN_POOL) {
+      o.gp = grid_of(n, lv + 1, batch);
+      o.pooled = n.pooled[lv];
+      o.pooled_planar = n.pooled_planar[lv];
+    }
+    if (l == kLayerCount - 1) {
+      o.head_w = n.params + n.head_w_off;
+      o.head_b = n.params + n.head_b_off;
+      o.head_out = n.out;
+    }
+    const ConvWork job = conv_work(in, n.zero, o.g, L.cout, n.wbf + n.wbf_off[l], o);
+    const int waves = conv_tiles(job) <= 1024 ? 1 : 4;
+    const int blocks = (conv_tiles(job) + waves - 1) / waves, threads = 64 * waves;
+    if (l == 0)
+      k_conv<true, false><<<blocks, threads, 0, n.stream>>>(job);
+    else if (L.kind == IN_CAT)
+      k_conv<false, true><<<blocks, threads, 0, n.stream>>>(job);
+    else
+      k_conv<false, false><<<blocks, threads, 0, n.stream>>>(job);
   }
-  k_head<<<nb(pix0), kT, 0, s>>>(n.act[kActs - 1], (int)pix0, kHeadIn,
-                                  n.params + n.head_w_off, n.params + n.head_b_off, n.out);
   GCS_HIP(hipGetLastError());
   return 0;
 }
 
-// Backward pass from n.gout (fp32, d loss / d out); gradients in n.grads.
+// Weight and bias gradient of layer l from gz of its output.
+static GradWork grad_work(const Net &n, int l, int batch) {
+  const LayerSpec &L = kLayers[l];
+  const int lv = act_level(l + 1);
+  const Grid g = grid_of(n, lv, batch);
+  GradIn in;
+  if (L.kind == IN_CAT) {
+    in.src0 = n.act_planar[L.src];
+    in.c0 = act_channels(L.src);
+    in.g0 = grid_of(n, lv + 1, batch);
+    in.src1 = n.act_planar[L.src2];
+    in.c1 = act_channels(L.src2);
+  } else {
+    in.src1 = L.kind == IN_POOL ? n.pooled_planar[(l - 2) / 2] : n.act_planar[L.src];
+    in.c1 = L.cin;
+  }
+  GradWork job;
+  job.in = in;
+  job.g = g;
+  job.gz = n.gz_planar[l + 1];
+  job.cout = L.cout;
+  const int slices = grad_slices(n, l, batch, job.per_wave);
+  job.blocks = slices * (L.cin / 16) * (L.cout / 32);
+  job.part = n.grad_part + n.part_off[l];
+  return job;
+}
+
+// Backward pass from n.gout (fp32, d loss / d out) of the last forward pass;
+// gradients in n.grads.
 int backward_device(Net &n, int batch) {
   hipStream_t s = n.stream;
-  const long pix0 = (long)batch * n.H * n.W;
-  k_fill<<<nb((long)n.param_count), kT, 0, s>>>(n.grads, (long)n.param_count, 0.f);
-  for (int a = 1; a < kActs; ++a) {
-    const int lv = act_level(a);
-    const long cnt = (long)batch * (n.H >> lv) * (n.W >> lv) * act_channels(a);
-    k_fill<<<nb(cnt), kT, 0, s>>>(n.gact[a], cnt, 0.f);
-  }
-  k_head_back<<<nb(pix0), kT, 0, s>>>(n.act[kActs - 1], n.gout, (int)pix0, kHeadIn,
-                                       n.params + n.head_w_off, n.gact[kActs - 1],
-                                       n.grads + n.head_w_off, n.grads + n.head_b_off);
+  const Grid g0 = grid_of(n, 0, batch);
+  k_planar_input<<<(unsigned)(batch * n.H * ((n.W + 63) / 64)), 256, 0, s>>>(n.input, g0,
+                                                                            n.act_planar[0]);
+  const unsigned head_blocks = std::min((unsigned)kHeadBlocks, nb((long)batch * n.H * n.W, 64));
+  k_head_back<<<head_blocks, 256, 0, s>>>(n.act[kActs - 1], n.gout, g0, n.params + n.head_w_off,
+                                          n.gz[kActs - 1], n.gz_planar[kActs - 1], n.head_part);
+  k_head_sum<<<kHeadIn + 1, 64, 0, s>>>(n.head_part, (int)head_blocks, n.grads + n.head_w_off);
   for (int l = kLayerCount - 1; l >= 0; --l) {
     const LayerSpec &L = kLayers[l];
     const int lv = act_level(l + 1);
-    const int H = n.H >> lv, W = n.W >> lv;
-    const long M = (long)batch * H * W;
-    k_relu_grad<<<nb(M * L.cout), kT, 0, s>>>(n.gact[l + 1], n.act[l + 1], M * L.cout, n.gz);
-    // Pixel chunks small enough that the sums run in parallel: a bias sum
-    // is one thread's loop over its chunk, and a weight-gradient launch has
-    // (K / 64) (cout / 64) blocks per chunk, as few as five at level 0.
-    const int chunk = 64;
-    k_colsum<<<nb(M, chunk), 256, 0, s>>>(n.gz, (int)M, L.cout, n.grads + n.b_off[l], chunk);
-    const ConvIn in = layer_input(n, l);
-    const int K = 9 * L.cin;
-    const int wchunk = 256;
-    k_wgrad3<<<dim3((K + 63) / 64, (L.cout + 63) / 64, nb(M, wchunk)), 256, 0, s>>>(
-        in, batch, H, W, n.gz, L.cout, n.grads + n.w_off[l], wchunk);
-    if (l == 0) continue;  // no gradient for the input features
-    // input gradient = conv of gz with the flipped, transposed weights
-    ConvIn gin;
-    gin.src1 = n.gz;
-    gin.c1 = L.cout;
-    k_conv3<<<dim3(nb(M, 64), (L.cin + 63) / 64), 256, 0, s>>>(
-        gin, batch, H, W, n.wflip + n.wbf_off[l], nullptr, L.cin, 0, nullptr, n.scratch);
-    if (L.kind == IN_PLAIN) {
-      k_add<<<nb(M * L.cin), kT, 0, s>>>(n.scratch, M * L.cin, n.gact[L.src]);
-    } else if (L.kind == IN_POOL) {
-      const int src = L.src;  // fine-grid activation
-      k_pool_back<<<nb(4 * M * L.cin), kT, 0, s>>>(n.scratch, batch, 2 * H, 2 * W, L.cin,
-                                                    n.gact[src]);
-    } else {
-      const int c0 = act_channels(L.src), c1 = act_channels(L.src2);
-      const long cnt = (long)batch * (H / 2) * (W / 2) * c0 + M * c1;
-      k_split_back<<<nb(cnt), kT, 0, s>>>(n.scratch, batch, H, W, c0, c1, n.gact[L.src],
-                                          n.gact[L.src2]);
+    const GradWork grad = grad_work(n, l, batch);
+    if (l == 0) {  // no gradient for the input features
+      k_wgrad<<<grad.blocks, 256, 0, s>>>(grad);
+      break;
     }
+    // input gradient = conv of gz with the flipped, transposed weights; its
+    // epilogue leaves the masked gradient of layer l - 1's output
+    const Grid g = grid_of(n, lv, batch);
+    ConvIn gin;
+    gin.src1 = n.gz[l + 1];
+    gin.c1 = L.cout;
+    ConvOut o;
+    o.out = n.gz[L.src];
+    o.planar = n.gz_planar[L.src];
+    o.act = n.act[L.src];
+    if (L.kind == IN_PLAIN) {
+      o.g = g;
+    } else if (L.kind == IN_POOL) {
+      o.g = grid_of(n, lv - 1, batch);
+      o.skip = n.skip[lv - 1];  // kept by the decoder layer of the fine grid
+    } else {
+      o.g = grid_of(n, lv + 1, batch);
+      o.skip = n.skip[lv];
+      o.c0 = act_channels(L.src);
+    }
+    ConvWork conv = conv_work(gin, n.zero, g, L.cin, n.wflip + n.wbf_off[l], o);
+    const int tiles = conv_tiles(conv);
+    conv.wk = split_k(tiles, 9 * L.cout / 32);
+    const int per_block = 4 / conv.wk;
+    const unsigned all = (unsigned)(grad.blocks + (tiles + per_block - 1) / per_block);
+    if (L.kind == IN_PLAIN)
+      k_backward<EP_PLAIN><<<all, 256, 0, s>>>(grad, conv);
+    else if (L.kind == IN_POOL)
+      k_backward<EP_POOL><<<all, 256, 0, s>>>(grad, conv);
+    else
+      k_backward<EP_CAT><<<all, 256, 0, s>>>(grad, conv);
   }
+  SliceTable table;
+  for (int l = 0; l < kLayerCount; ++l) {
+    int per_wave;
+    table.begin[l] = (int)n.w_off[l];
+    table.slices[l] = grad_slices(n, l, batch, per_wave);
+    table.part[l] = n.part_off[l];
+  }
+  table.begin[kLayerCount] = (int)n.head_w_off;
+  k_grad_sum<<<nb((long)n.head_w_off), 256, 0, s>>>(n.grad_part, table, n.grads);
   GCS_HIP(hipGetLastError());
   return 0;
 }
@@ -723,10 +1192,11 @@ int adam_device(Net &n, float lr) {
   ++n.adam_t;
   const float c1 = 1.f - std::pow(b1, (float)n.adam_t);
   const float c2 = 1.f - std::pow(b2, (float)n.adam_t);
-  k_adam<<<nb((long)n.param_count), kT, 0, n.stream>>>(n.params, n.grads, n.adam_m, n.adam_v,
-                                                       (long)n.param_count, lr, b1, b2, c1,
-                                                       c2, 1e-8f);
-  return prep_weights(n);
+  k_adam<<<nb((long)n.param_count), kT, 0, n.stream>>>(
+      n.params, n.grads, n.adam_m, n.adam_v, (long)n.param_count, lr, b1, b2, c1, c2, 1e-8f,
+      pack_table(n), n.wbf, n.wflip);
+  GCS_HIP(hipGetLastError());
+  return 0;
 }
 
 int check_batch(const Net &n, int batch) {

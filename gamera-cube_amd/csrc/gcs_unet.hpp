@@ -38,15 +38,20 @@ struct Net {
   size_t head_w_off = 0, head_b_off = 0;
   float *params = nullptr, *grads = nullptr, *adam_m = nullptr, *adam_v = nullptr;
   int adam_t = 0;
-  uint16_t *wbf = nullptr, *wflip = nullptr;  // bf16 weights, flipped-transposed copy
-  uint16_t *act[kActs] = {};                  // bf16 activations
-  float *gact[kActs] = {};                    // fp32 activation gradients
-  uint16_t *pooled[3] = {};                   // pooled encoder outputs
-  float *scratch = nullptr;                   // input gradient of one layer
-  uint16_t *gz = nullptr;                     // masked output gradient, bf16
-  float *input = nullptr;                     // fp32 features [N][H][W][16]
+  uint16_t *wbf = nullptr, *wflip = nullptr;  // bf16 weights in operand order, and flipped
+  uint16_t *act[kActs] = {};                  // bf16 activations, NHWC
+  uint16_t *act_planar[kActs] = {};           // and planar, rows padded
+  uint16_t *gz[kActs] = {}, *gz_planar[kActs] = {};  // masked gradients likewise
+  long planar_count[kActs] = {};
+  uint16_t *pooled[3] = {}, *pooled_planar[3] = {};  // pooled encoder outputs
+  float *skip[3] = {};                        // decoder's gradient of the skip, by level
+  float *input = nullptr;                     // fp32 features [N][H][W][32]
   float *out = nullptr, *gout = nullptr, *target = nullptr;
   float *loss = nullptr;
+  uint16_t *zero = nullptr;                   // 64 zero bytes
+  float *grad_part = nullptr;                 // weight gradients by pixel slice
+  long part_off[kLayerCount] = {};            // and each layer's place there
+  float *head_part = nullptr;                 // block sums of the head's gradient
   float *energy = nullptr;                    // per-sample target mean square
   // potential = out * out_scale * R^2 * scale / SigmaP (set on the first
   // training batch so that targets have unit RMS)
