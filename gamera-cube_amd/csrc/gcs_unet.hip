@@ -150,37 +150,37 @@ __device__ inline float lane_xor1(float v) {
 // rows = output channels (weights packed in operand order, k_pack_weights),
 // columns = pixels, k = (tap, input channel) in steps of 32 channels. Operands
 // come straight from L1 / L2 as 16-byte loads, four loads per four MFMAs, the
-// loads of kAhead steps in flight; wk wavefronts of a block share one tile and
-// split its steps. What bounds it is the latency of a launch and of the loads
-// at the small grids, L2 traffic (16 flops a byte) at the large ones. Measured
-// with the kernel before, which gathered 8 bytes per lane and MFMA: the 14
-// layers of 2 x 128 x 256, 930 -> 174 us (130 TFLOP/s); a layer of 8 x 32 x 64,
-// 60 -> 11 us.
+// loads of kAhead steps in flight. A tile's sum is one chain: another order
+// flips the rounding and the ReLU of values near a tie, and the network and
+// its training carry that on (with the deep layers' input gradients split into
+// four, 20 training steps took 10.9 instead of 11.2 ms but ended up to 1e-2
+// away; now they end as near as two runs that add gradients in another order).
+// What bounds it is the latency of a launch and of the loads at the small
+// grids, L2 traffic (16 flops a byte) at the large ones. Measured with the
+// kernel before, which gathered 8 bytes per lane and MFMA: the 14 layers of
+// 2 x 128 x 256, 930 -> 174 us (130 TFLOP/s); a layer of 8 x 32 x 64, 60 -> 11.
 constexpr int kAhead = 4;
-
-constexpr int kConvLds = 3 * 16 * 64;  // floats of a block
 
 struct ConvWork {
   ConvIn in;
   Grid g;
-  int cout, wk;
+  int cout;
   const uint16_t *w;
   ConvOut o;
 };
 
 template <int EP, bool F32, bool CAT>
-__device__ inline void conv_block(const ConvWork &job, int block, float *s_part) {
+__device__ inline void conv_block(const ConvWork &job, int block) {
   const ConvIn &in = job.in;
   const Grid &g = job.g;
   const ConvOut &o = job.o;
   const uint16_t *__restrict__ w = job.w;
-  const int cout = job.cout, wk = job.wk;
+  const int cout = job.cout;
   const int cin = in.c0 + in.c1, spt = cin >> 5, steps = 9 * spt;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int ks = wave % wk, sub = wave / wk;
   const int ctiles = cout >> 5, xt = (g.W + 15) >> 4, yt = (g.H + 1) >> 1;
   const int tiles = ctiles * xt * yt * g.N;
-  const int tile = block * ((int)(blockDim.x >> 6) / wk) + sub;
+  const int tile = block * (int)(blockDim.x >> 6) + wave;
   const bool live = tile < tiles;
   int r = live ? tile : 0;
   const int ct = r % ctiles;
@@ -195,7 +195,6 @@ __device__ inline void conv_block(const ConvWork &job, int block, float *s_part)
     for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
   const uint16_t *wt = w + ((long)(2 * ct) * steps * 64 + lane) * 8;
   const long wnext = (long)steps * 64 * 8;
-  const int s_begin = live ? ks * steps / wk : 0, s_end = live ? (ks + 1) * steps / wk : 0;
   // One step's operands as loaded: nothing touches a loaded value before its
   // use, and every step loads (the last ones again, past the end), so that the
   // wait before a product leaves the loads of the steps ahead in flight.
@@ -204,7 +203,7 @@ __device__ inline void conv_block(const ConvWork &job, int block, float *s_part)
   };
   // The next step to load: its tap's pixels (a row outside the grid reads
   // zeros, whatever the channel) and its first channel.
-  int ls = s_begin, tap = s_begin / spt, lc = s_begin - tap * spt;
+  int ls = 0, tap = 0, lc = 0;
   const uint16_t *px[2], *px0[2];
   int inside[2];  // all ones, or zero
   auto set_tap = [&]() {
@@ -255,7 +254,7 @@ __device__ inline void conv_block(const ConvWork &job, int block, float *s_part)
     return u32x4{pack2(lo[0], lo[1]), pack2(lo[2], lo[3]), pack2(hi[0], hi[1]),
                  pack2(hi[2], hi[3])};
   };
-  if (s_begin < s_end) {
+  if (live) {
     Step ahead[kAhead];
 #pragma unroll
     for (int p = 0; p < kAhead; ++p) load(ahead[p]);
@@ -265,7 +264,7 @@ __device__ inline void conv_block(const ConvWork &job, int block, float *s_part)
         for (int t = 0; t < 2; ++t) acc[t][v] = mfma32(o.a[t], b, acc[t][v]);
       }
     };
-    int left = s_end - s_begin;
+    int left = steps;
     for (; left >= kAhead; left -= kAhead) {
 #pragma unroll
       for (int p = 0; p < kAhead; ++p) {
@@ -276,20 +275,6 @@ __device__ inline void conv_block(const ConvWork &job, int block, float *s_part)
 #pragma unroll
     for (int p = 0; p < kAhead - 1; ++p)
       if (p < left) use(ahead[p]);
-  }
-  if (wk > 1) {
-    // partial sums of the other wavefronts of the tile, in their order
-    float *mine = s_part + (sub * (wk - 1) + ks - 1) * 1024;
-    if (ks > 0)
-      for (int t = 0; t < 4; ++t)
-        for (int i = 0; i < 4; ++i) mine[(4 * t + i) * 64 + lane] = acc[t >> 1][t & 1][i];
-    __syncthreads();
-    if (ks > 0) return;
-    for (int p = 1; p < wk; ++p) {
-      const float *other = s_part + (sub * (wk - 1) + p - 1) * 1024;
-      for (int t = 0; t < 4; ++t)
-        for (int i = 0; i < 4; ++i) acc[t >> 1][t & 1][i] += other[(4 * t + i) * 64 + lane];
-    }
   }
   if (!live) return;
   // lane: channels c + 4q + 0..3 and c + 16 + 4q + 0..3 of pixels (y0 + v, x)
@@ -323,11 +308,15 @@ __device__ inline void conv_block(const ConvWork &job, int block, float *s_part)
       const f32x4 h0 = *(const f32x4 *)(o.head_w + 4 * q),
                   h1 = *(const f32x4 *)(o.head_w + 16 + 4 * q);
       for (int v = 0; v < 2; ++v) {
+        // in the order of the channels (32 are one tile): a quarter adds four
+        // and hands the sum to the next
         float s = 0.f;
-        for (int i = 0; i < 8; ++i) s += element(z[v], i) * (i < 4 ? h0[i & 3] : h1[i & 3]);
-        // the wavefront's four quarters; 32 channels are one tile
-        s += __shfl_xor(s, 16, 64);
-        s += __shfl_xor(s, 32, 64);
+        for (int h = 0; h < 8; ++h) {
+          const int first = h < 4 ? 0 : 4;
+          for (int i = first; i < first + 4; ++i)
+            s += element(z[v], i) * (i < 4 ? h0[i & 3] : h1[i & 3]);
+          s = __shfl(s, 16 * (h & 3) + col, 64);
+        }
         if (q == 0 && xin && y0 + v < g.H) o.head_out[g.pixel(n, y0 + v, x)] = s + o.head_b[0];
       }
     }
@@ -375,15 +364,13 @@ __device__ inline void conv_block(const ConvWork &job, int block, float *s_part)
   }
 }
 
-// A forward layer. Its sums are not split: another order of a sum flips the
-// rounding and the ReLU of values near a tie, and the network carries that on.
-// One wavefront to a block up to 1024 tiles (four a CU), so that a deep
+// A forward layer. One wavefront to a block up to 1024 tiles (four a CU), so that a deep
 // layer's few long sums have a CU's load path each and neighbouring XCDs read
 // different weights, else four (forward pass of 2 x 32 x 64: 236 us as blocks
 // of four, 197 so; of 2 x 128 x 256: 521, 493).
 template <bool F32, bool CAT>
 __global__ void __launch_bounds__(256) k_conv(ConvWork job) {
-  conv_block<EP_FORWARD, F32, CAT>(job, blockIdx.x, nullptr);
+  conv_block<EP_FORWARD, F32, CAT>(job, blockIdx.x);
 }
 
 // Weight and bias gradients: gw[co][tap][ci] += sum over pixels of gz[co] x
@@ -528,11 +515,11 @@ __global__ void __launch_bounds__(256) k_wgrad(GradWork job) {
 // 13.3 -> 11.1 ms against two launches, 8 x 128 x 256 the same within 1 %).
 template <int EP>
 __global__ void __launch_bounds__(256) k_backward(GradWork grad, ConvWork conv) {
-  __shared__ float lds[kGradLds > kConvLds ? kGradLds : kConvLds];
+  __shared__ float lds[kGradLds];
   if ((int)blockIdx.x < grad.blocks)
     wgrad_block(grad, blockIdx.x, lds);
   else
-    conv_block<EP, false, false>(conv, blockIdx.x - grad.blocks, lds);
+    conv_block<EP, false, false>(conv, blockIdx.x - grad.blocks);
 }
 
 // gradients = the slices' partial sums of every convolution parameter, in the
@@ -1016,17 +1003,6 @@ static int conv_tiles(const ConvWork &job) {
   return (job.cout / 32) * ((job.g.W + 15) / 16) * ((job.g.H + 1) / 2) * job.g.N;
 }
 
-// An input gradient's wavefronts that share one tile's sum: until the launch
-// has about two per SIMD, a layer's few tiles are split along k, but into no
-// less than five steps each (20 training steps of 8 x 32 x 64: not split 12.3
-// ms, split 11.8; down to one step it is no faster, and short sums' rounding
-// stays that of one chain).
-static int split_k(int tiles, int steps) {
-  int wk = tiles >= 2048 ? 1 : tiles >= 1024 ? 2 : 4;
-  while (wk > 1 && steps / wk < 5) wk /= 2;
-  return wk;
-}
-
 static ConvWork conv_work(const ConvIn &in, const uint16_t *zero, const Grid &g, int cout,
                           const uint16_t *w, const ConvOut &o) {
   ConvWork job;
@@ -1034,7 +1010,6 @@ static ConvWork conv_work(const ConvIn &in, const uint16_t *zero, const Grid &g,
   job.in.zero = zero;
   job.g = g;
   job.cout = cout;
-  job.wk = 1;
   job.w = w;
   job.o = o;
   return job;
@@ -1143,10 +1118,7 @@ int backward_device(Net &n, int batch) {
       o.c0 = act_channels(L.src);
     }
     ConvWork conv = conv_work(gin, n.zero, g, L.cin, n.wflip + n.wbf_off[l], o);
-    const int tiles = conv_tiles(conv);
-    conv.wk = split_k(tiles, 9 * L.cout / 32);
-    const int per_block = 4 / conv.wk;
-    const unsigned all = (unsigned)(grad.blocks + (tiles + per_block - 1) / per_block);
+    const unsigned all = (unsigned)(grad.blocks + (conv_tiles(conv) + 3) / 4);
     if (L.kind == IN_PLAIN)
       k_backward<EP_PLAIN><<<all, 256, 0, s>>>(grad, conv);
     else if (L.kind == IN_POOL)
