@@ -1,6 +1,8 @@
 // Copies between device planes and reference-layout host arrays.
 #pragma once
 
+#include <hip/hip_runtime.h>
+
 #include <cstddef>
 
 namespace gcs {
@@ -31,5 +33,22 @@ struct HostArray;
 int planes_to_arrays(Problem &P, int first, int ncomp, int face, int faces,
                      const size_t ext[3], HostArray *const out[]);
 void free_array(HostArray &a);
+
+// Two pinned chunks that flat arrays cross PCIe in, owned by one caller (its
+// calls are in order on one stream). Without buffers (never made, or no pinned
+// memory) and for short arrays the copies are direct.
+struct Staging {
+  char *buf[2] = {};
+  hipEvent_t done[2] = {};
+  Staging() = default;
+  Staging(const Staging &) = delete;
+  Staging &operator=(const Staging &) = delete;
+  ~Staging();
+  void make();
+};
+// The host array has been read when stage_up returns, and been written when
+// stage_down does (which also waits for the stream's earlier work).
+int stage_up(Staging &g, hipStream_t stream, const void *host, void *dev, size_t bytes);
+int stage_down(Staging &g, hipStream_t stream, const void *dev, void *host, size_t bytes);
 
 }  // namespace gcs

@@ -913,6 +913,7 @@ Net *create(int H, int W, int max_batch, uint64_t seed) {
     delete net;
     return nullptr;
   }
+  n.stage.make();
   for (int a = 0; a < kActs; ++a) {
     fill_zero(n, n.act_planar[a], n.planar_count[a]);
     if (a > 0) fill_zero(n, n.gz_planar[a], n.planar_count[a]);
@@ -957,8 +958,7 @@ int set_params(Net &n, const float *host, size_t count) {
     set_error("warm-start network: parameter count mismatch");
     return -1;
   }
-  GCS_HIP(hipMemcpyAsync(n.params, host, count * sizeof(float), hipMemcpyHostToDevice,
-                         n.stream));
+  if (stage_up(n.stage, n.stream, host, n.params, count * sizeof(float)) != 0) return -1;
   k_fill<<<nb((long)count), kT, 0, n.stream>>>(n.adam_m, (long)count, 0.f);
   k_fill<<<nb((long)count), kT, 0, n.stream>>>(n.adam_v, (long)count, 0.f);
   n.adam_t = 0;
@@ -972,10 +972,8 @@ int get_array(Net &n, int which, float *host, size_t count) {
     set_error("warm-start network: parameter count mismatch");
     return -1;
   }
-  GCS_HIP(hipMemcpyAsync(host, which == 0 ? n.params : n.grads, count * sizeof(float),
-                         hipMemcpyDeviceToHost, n.stream));
-  GCS_HIP(hipStreamSynchronize(n.stream));
-  return 0;
+  return stage_down(n.stage, n.stream, which == 0 ? n.params : n.grads, host,
+                    count * sizeof(float));
 }
 
 static ConvIn layer_input(const Net &n, int l) {

@@ -11,6 +11,7 @@
 
 #include "gamera_cs_unet.h"
 #include "gcs_device.hpp"
+#include "gcs_transfer.hpp"
 
 namespace gcs {
 namespace unet {
@@ -57,6 +58,7 @@ struct Net {
   // training batch so that targets have unit RMS)
   double out_scale = 1.0;
   hipStream_t stream = nullptr;
+  Staging stage;  // for arrays from and to the host
   std::vector<void *> allocations;
   ~Net();
 };

@@ -17,8 +17,7 @@ const Net *as_net(const gcs_unet *p) { return reinterpret_cast<const Net *>(p); 
 Problem *as_problem(gcs_problem *p) { return reinterpret_cast<Problem *>(p); }
 
 int upload(Net &n, const float *host, float *dev, size_t count) {
-  if (hipMemcpyAsync(dev, host, count * sizeof(float), hipMemcpyHostToDevice, n.stream) !=
-      hipSuccess) {
+  if (gcs::stage_up(n.stage, n.stream, host, dev, count * sizeof(float)) != 0) {
     gcs::set_error("warm-start network: upload failed");
     return -1;
   }
@@ -26,9 +25,7 @@ int upload(Net &n, const float *host, float *dev, size_t count) {
 }
 
 int download(Net &n, const float *dev, float *host, size_t count) {
-  if (hipMemcpyAsync(host, dev, count * sizeof(float), hipMemcpyDeviceToHost, n.stream) !=
-          hipSuccess ||
-      hipStreamSynchronize(n.stream) != hipSuccess) {
+  if (gcs::stage_down(n.stage, n.stream, dev, host, count * sizeof(float)) != 0) {
     gcs::set_error("warm-start network: download failed");
     return -1;
   }

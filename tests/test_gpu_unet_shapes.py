@@ -51,3 +51,21 @@ def test_network_at_ragged_grids(gpu, n, h, w):
     assert err <= 5e-2
     assert net.gradients(x, target) == pytest.approx(loss, rel=1e-6)
     assert np.array_equal(net.grads(), got)
+
+
+@pytest.mark.parametrize("n", [15, 16, 17, 25])
+def test_large_batches_match_single_samples(gpu, n):
+    """Around the size from which features are uploaded in chunks (16 samples
+    of 64 x 128 are 16 MiB; 17 and 25 end inside a chunk): every sample gives
+    the bits it gives by itself, and parameters come back as they went."""
+    ws = importlib.import_module("gamera-cube_amd.warm_start")
+    print(f"batch of {n}", flush=True)
+    rng = np.random.default_rng(n)
+    net = ws.WarmStartNet(64, 128, n, seed=3)
+    params = rng.standard_normal(net.param_count).astype(np.float32) * 0.02
+    net.set_params(params)
+    assert np.array_equal(net.params(), params)
+    x = rng.standard_normal((n, 64, 128, 32)).astype(np.float32)
+    out = net.forward(x)
+    for k in (0, n // 2, n - 1):
+        assert np.array_equal(net.forward(x[k:k + 1])[0], out[k])
