@@ -1,8 +1,8 @@
 """The network's kernels at the grids where their tiles can go wrong: columns
 that end inside a 16-pixel tile and inside an 8-pixel group at every level, an
 odd number of rows and a single column at the coarsest level, one sample of a
-larger batch after a full one (stale samples must not count), and sizes that
-split their sums differently. Against the numpy oracle with the tolerances of
+larger batch after a full one (stale samples must not count), and sizes on
+both sides of a forward block's rule and of the pixel slices. Against the numpy oracle with the tolerances of
 test_gpu_unet.py (forward 2e-2, gradients as one vector by relative L2 5e-2:
 bf16 steps of 2^-8 that different fp32 orders flip); a second run must give the
 same bits."""
