@@ -20,8 +20,11 @@
 // reference's by rounding, and the converged potential agrees with it to the
 // solve's tolerance. Both hemispheres run in the same launches. The solves
 // keep their vectors in registers, one wavefront per ring (k_ring_cg,
-// k_ring_bicgstab); where their workgroups cannot all be resident, one
-// workgroup per hemisphere solves instead (k_mi_cg, k_mi_bicgstab).
+// k_ring_bicgstab). Where their workgroups cannot all be resident, a fixed
+// number of workgroups solves the tensor system (k_mi_bicgstab_pair) and one
+// workgroup per hemisphere the Pedersen one (k_mi_cg); without cooperative
+// launches one workgroup per hemisphere solves either (k_mi_bicgstab).
+#include <hip/hip_cooperative_groups.h>
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
@@ -92,10 +95,14 @@ struct MiState {
   // potential plus the network's answer for the current residual
   unet::Net *net = nullptr;
   double *warm_scale = nullptr;  // [2] residual-current RMS, [2] step lengths
-  // exchange buffers of the register-resident solve (null: one workgroup
-  // per hemisphere solves instead) and its workgroups per hemisphere
+  // exchange buffers of the register-resident solve (null: its workgroups do
+  // not fit) and its workgroups per hemisphere
   unsigned long long *ring_words = nullptr;
   int ring_groups = 0;
+  // of the tensor solve by grid-wide barriers (null: not used): partial sums
+  // and the per-hemisphere liveness exchange
+  double *coop_slots = nullptr;
+  int *coop_flags = nullptr;
 };
 
 namespace {
@@ -506,9 +513,9 @@ MiK make_mik(Problem &P) {
 
 // ---- fused solves: one workgroup per hemisphere runs the whole Krylov loop -------
 //
-// The solves of devices or grids that cannot hold the register-resident
-// kernels' workgroups at once (more than 768 rings on 256 compute units), or
-// with GCS_MI_COOPERATIVE=0.
+// The solves of devices without cooperative launches or with
+// GCS_MI_COOPERATIVE=0, and the Pedersen solve of grids whose rings the
+// register-resident kernel's workgroups cannot hold at once.
 //
 // The same iterations as the reference's solvers (CG: :516-600, BiCGStab:
 // :1029-1131, with the ring preconditioner above), but every scalar stays on
@@ -948,6 +955,224 @@ __global__ void __launch_bounds__(kSolveThreads) k_mi_bicgstab(MiK c, double rel
     rho_prev = rho;
   }
   store_result(c, h, res, first);
+}
+
+// The Hall-tensor solve of grids with more rings than k_ring_bicgstab's
+// workgroups can hold at once (768 on 256 compute units): each hemisphere's
+// solve spread over kCoopBlocks workgroups (the same iterations as
+// k_mi_bicgstab, with grid-wide barriers where one workgroup's barrier
+// sufficed there). What bounds it is its ten barriers an iteration and, on
+// large grids, the vectors' traffic through L2. 2 x 800 x 256 points, 3,400 -
+// 3,900 iterations: 908 ms (k_mi_bicgstab: 9,221); 2 x 771 x 64: 403 ms
+// (3,219). Below that limit k_ring_bicgstab is the faster one: 2 x 770 x 64,
+// 42 against 384 ms; 2 x 128 x 256, 4.0 against 45. Dot products sum the
+// workgroups' partial sums in workgroup order from two alternating slot
+// banks (a bank is rewritten only after every workgroup passed the barrier
+// that follows its last read), so every workgroup of a hemisphere computes
+// the same sums and takes the same branches.
+constexpr int kCoopBlocks = 16;
+
+// Both hemispheres in one cooperative launch: workgroups [0, kCoopBlocks)
+// solve the north, [kCoopBlocks, 2 kCoopBlocks) the south, concurrently. The
+// grid barriers are shared, so every workgroup must pass the same sequence
+// of barriers whatever its hemisphere does: each iteration runs a fixed
+// schedule of ten barrier-carrying steps, and a hemisphere that has
+// converged, broken down or needs no true-residual check this iteration
+// skips the work of a step but not its barrier. No branch contains a
+// barrier, the loop bound and its exit test are grid-uniform (the exit reads
+// both hemispheres' flags after a barrier), so every workgroup leaves after
+// the same number of barriers, at the latest after maximum_iterations.
+// Per hemisphere the arithmetic is k_mi_bicgstab's.
+__global__ void __launch_bounds__(kSolveThreads) k_mi_bicgstab_pair(MiK c, double rel_tol,
+                                                                    int maxit, double *slots,
+                                                                    int *flags) {
+  namespace cg = cooperative_groups;
+  cg::grid_group grid = cg::this_grid();
+  __shared__ double red[kSolveThreads / 64];
+  const int h = blockIdx.x / kCoopBlocks, lb = blockIdx.x % kCoopBlocks;
+  const long n = c.n;
+  const long t0 = lb * (long)blockDim.x + threadIdx.x;
+  const long st = (long)kCoopBlocks * blockDim.x;
+  const bool pole_wave = lb == 0 && threadIdx.x < 64;
+  int bank = 0;
+  // sums of up to two values over this hemisphere's workgroups
+  auto gsum2 = [&](double v, double w, double &sv, double &sw) {
+    const double bv = block_sum(v, red);
+    const double bw = block_sum(w, red);
+    double *sl = slots + bank * (4 * kCoopBlocks) + h * (2 * kCoopBlocks);
+    if (threadIdx.x == 0) {
+      sl[lb] = bv;
+      sl[kCoopBlocks + lb] = bw;
+    }
+    bank ^= 1;
+    grid.sync();
+    sv = 0.0;
+    sw = 0.0;
+    for (int i = 0; i < kCoopBlocks; ++i) {
+      sv += sl[i];
+      sw += sl[kCoopBlocks + i];
+    }
+  };
+  auto gsum = [&](double v) {
+    double sv, sw;
+    gsum2(v, 0.0, sv, sw);
+    return sv;
+  };
+  const double dt = c.max_colat / (double)(c.nt - 1);
+  const double half = 0.5 * dt;
+  const double pe = sin(half) * c.pedersen / (incl2(half) * dt * dt);
+  const double ps = (double)c.np * pe;
+  double *x = c.vec(h, V_X), *r = c.vec(h, V_R), *p = c.vec(h, V_P), *ap = c.vec(h, V_AP),
+         *sh = c.vec(h, V_SH), *pp = c.vec(h, V_PP), *s = c.vec(h, V_S), *psv = c.vec(h, V_PS),
+         *as = c.vec(h, V_AS);
+  const double *rhs = c.vec(h, V_RHS);
+  const int lane = threadIdx.x & 63;
+  auto precondition = [&](bool work, const double *in, double *out) {
+    grid.sync();  // `in` complete
+    if (work) {
+      if (t0 == 0) out[0] = in[0] / c.vec(h, V_DIAG)[0];
+      for (long ring = t0 >> 6; ring < c.nt - 2; ring += st >> 6)
+        ring_apply(c, h, in, out, (int)ring, lane);
+    }
+    grid.sync();  // `out` complete
+  };
+  for (long ring = t0; ring < c.nt - 2; ring += st) ring_factor(c, h, (int)ring);
+  double a = 0.0, b = 0.0;
+  {
+    const double pole = pole_wave ? pole_row(c, h, true, x, pe) : 0.0;
+    for (long q = t0; q < n; q += st) {
+      r[q] = rhs[q] - (q == 0 ? pole : apply_at(c, h, true, x, q, nullptr, pe));
+      sh[q] = r[q];
+      p[q] = 0.0;
+      ap[q] = 0.0;
+      a += orig_term(c, r[q], q, ps, dt);
+      b += q == 0 ? 0.0 : orig_term(c, rhs[q], q, ps, dt);
+    }
+  }
+  double n0, b0;
+  gsum2(a, b, n0, b0);  // also orders the ring factors before their first use
+  double norm = sqrt(fmax(0.0, n0));
+  const double first = norm;
+  const double target = rel_tol * fmax(sqrt(fmax(0.0, b0)), 1.0);
+  SolveResult res{0, norm <= target, norm};
+  bool live = !res.ok;  // this hemisphere still iterates
+  double rho_prev = 1.0, alpha = 1.0, omega = 1.0;
+  bool other_live = true;
+  for (int it = 1; it <= maxit && (live || other_live); ++it) {
+    // 1: rho
+    a = 0.0;
+    if (live)
+      for (long q = t0; q < n; q += st) a += sh[q] * r[q];
+    const double rho = gsum(a);
+    if (live && (!isfinite(rho) || fabs(rho) <= DBL_MIN || !isfinite(omega) ||
+                 fabs(omega) <= DBL_MIN))
+      live = false;
+    // 2, 3: p and its preconditioned image
+    if (live) {
+      const double beta = (rho / rho_prev) * (alpha / omega);
+      for (long q = t0; q < n; q += st) p[q] = r[q] + beta * (p[q] - omega * ap[q]);
+    }
+    precondition(live, p, pp);
+    // 4: A pp and den
+    a = 0.0;
+    {
+      const double pole = (live && pole_wave) ? pole_row(c, h, true, pp, pe) : 0.0;
+      if (live)
+        for (long q = t0; q < n; q += st) {
+          ap[q] = q == 0 ? pole : apply_at(c, h, true, pp, q, nullptr, pe);
+          a += sh[q] * ap[q];
+        }
+    }
+    const double den = gsum(a);
+    // 5: s and its norm
+    a = 0.0;
+    if (live) {
+      alpha = rho / den;
+      for (long q = t0; q < n; q += st) {
+        s[q] = r[q] - alpha * ap[q];
+        a += orig_term(c, s[q], q, ps, dt);
+      }
+    }
+    const double snorm = sqrt(fmax(0.0, gsum(a)));
+    if (live && (!isfinite(den) || fabs(den) <= DBL_MIN)) live = false;
+    if (live && snorm <= target) {
+      res.last = snorm;
+      res.iters = it;
+      res.ok = true;
+      live = false;
+      for (long q = t0; q < n; q += st) x[q] += alpha * pp[q];
+    }
+    // 6, 7: preconditioned s
+    precondition(live, s, psv);
+    // 8: A ps and omega
+    a = 0.0;
+    b = 0.0;
+    {
+      const double pole = (live && pole_wave) ? pole_row(c, h, true, psv, pe) : 0.0;
+      if (live)
+        for (long q = t0; q < n; q += st) {
+          as[q] = q == 0 ? pole : apply_at(c, h, true, psv, q, nullptr, pe);
+          a += as[q] * as[q];
+          b += as[q] * s[q];
+        }
+    }
+    double wden, wnum;
+    gsum2(a, b, wden, wnum);
+    if (live) {
+      omega = wnum / wden;
+      if (!isfinite(wden) || wden <= DBL_MIN || !isfinite(omega) || fabs(omega) <= DBL_MIN)
+        live = false;
+    }
+    // 9: x, r and the recursive residual norm
+    a = 0.0;
+    if (live)
+      for (long q = t0; q < n; q += st) {
+        x[q] += alpha * pp[q] + omega * psv[q];
+        r[q] = s[q] - omega * as[q];
+        a += orig_term(c, r[q], q, ps, dt);
+      }
+    const double rn = gsum(a);
+    bool verify = false;
+    if (live) {
+      norm = sqrt(fmax(0.0, rn));
+      res.iters = it;
+      res.last = norm;
+      verify = norm <= target || it % 256 == 0;
+    }
+    // 10: true residual when checked; the exit flags of both hemispheres
+    a = 0.0;
+    if (verify) {
+      const double pole = pole_wave ? pole_row(c, h, true, x, pe) : 0.0;
+      for (long q = t0; q < n; q += st) {
+        r[q] = rhs[q] - (q == 0 ? pole : apply_at(c, h, true, x, q, nullptr, pe));
+        sh[q] = r[q];
+        a += orig_term(c, r[q], q, ps, dt);
+      }
+    }
+    const double tn = gsum(a);
+    if (verify) {
+      norm = sqrt(fmax(0.0, tn));
+      res.last = norm;
+      if (norm <= target) {
+        res.ok = true;
+        live = false;
+      } else {
+        for (long q = t0; q < n; q += st) {
+          p[q] = 0.0;
+          ap[q] = 0.0;
+        }
+        rho_prev = alpha = omega = 1.0;
+      }
+    } else if (live) {
+      rho_prev = rho;
+    }
+    // exchange liveness: written now, read after the next iteration's first
+    // barrier; one more round trip than needed only delays the exit
+    if (lb == 0 && threadIdx.x == 0) flags[(it & 1) * 2 + h] = live ? 1 : 0;
+    grid.sync();
+    other_live = flags[(it & 1) * 2 + (1 - h)] != 0;
+  }
+  if (lb == 0) store_result(c, h, res, first);
 }
 
 // ---- register-resident solves: one wavefront per colatitude ring ------------------
@@ -1954,21 +2179,27 @@ int solve(Problem &P, bool tensor) {
   if (m.net != nullptr && warm_start(P, c, tensor) != 0) return -1;
   double rel = m.cfg.relative_tolerance;
   int maxit = m.cfg.maximum_iterations;
+  auto cooperative = [&](const void *kernel, int groups, int threads, void **args) {
+    if (hipLaunchCooperativeKernel(kernel, dim3(groups), dim3(threads), args, 0, s) == hipSuccess)
+      return true;
+    (void)hipGetLastError();
+    return false;
+  };
   bool resident = comm.red != nullptr;
   if (resident) {
     if (tensor) k_ring_factor<<<dim3(m.nt - 2, 2), 64, 0, s>>>(c);
     void *args[] = {&c, &comm, &rel, &maxit};
-    if (hipLaunchCooperativeKernel((const void *)ring_kernel(points, tensor),
-                                   dim3(2 * m.ring_groups), dim3(kRingThreads), args, 0, s) !=
-        hipSuccess) {
-      (void)hipGetLastError();
-      resident = false;
-    }
+    resident = cooperative((const void *)ring_kernel(points, tensor), 2 * m.ring_groups,
+                           kRingThreads, args);
   }
   if (!resident) {
-    if (tensor)
+    void *args[] = {&c, &rel, &maxit, &m.coop_slots, &m.coop_flags};
+    const bool pair = tensor && m.coop_slots != nullptr &&
+                      cooperative((const void *)k_mi_bicgstab_pair, 2 * kCoopBlocks,
+                                  kSolveThreads, args);
+    if (!pair && tensor)
       k_mi_bicgstab<<<2, kSolveThreads, 0, s>>>(c, rel, maxit);
-    else
+    else if (!pair)
       k_mi_cg<<<2, kSolveThreads, 4 * (size_t)m.nt * sizeof(double), s>>>(c, rel, maxit);
     k_mi_vec<<<dim3(blocks_of((long)m.np * m.nt), 2), kT, 0, s>>>(c, OP_EXPAND, 0.0, m.active);
   }
@@ -2147,10 +2378,11 @@ int mi_create(Problem &P) {
   GCS_HIP(hipMalloc(&m.drift, 18L * L.ghost * L.NJ * L.NK * sizeof(double)));
   GCS_HIP(hipMalloc(&m.work, 2L * kVectors * m.n * sizeof(double)));
   {
-    // the register-resident solves need all their workgroups resident at
-    // once; GCS_MI_COOPERATIVE=0 selects the single-workgroup solves instead
-    // (for tools that cannot follow a cooperative launch, such as the kernel
-    // tracer of rocprofv3 7.2, which faults at exit after one)
+    // the register-resident solves and the one by grid-wide barriers need all
+    // their workgroups resident at once; GCS_MI_COOPERATIVE=0 selects the
+    // single-workgroup solves instead (for tools that cannot follow a
+    // cooperative launch, such as the kernel tracer of rocprofv3 7.2, which
+    // faults at exit after one)
     const char *env = std::getenv("GCS_MI_COOPERATIVE");
     const bool allowed = env == nullptr || std::strcmp(env, "0") != 0;
     const int points = (m.np + 63) / 64, groups = (m.nt - 2 + kRingOwn - 1) / kRingOwn;
@@ -2161,11 +2393,19 @@ int mi_create(Problem &P) {
         hipOccupancyMaxActiveBlocksPerMultiprocessor(
             &per_cu, (const void *)ring_kernel(points, m.hall > 0.0), kRingThreads, 0) ==
             hipSuccess &&
-        coop != 0 && (long)per_cu * cus >= 2L * groups) {
-      m.ring_groups = groups;
-      GCS_HIP(hipMalloc(&m.ring_words, (RingComm::red_words(groups) +
-                                        RingComm::halo_words(groups, points)) *
-                                           sizeof(ll_word)));
+        coop != 0) {
+      if ((long)per_cu * cus >= 2L * groups) {
+        m.ring_groups = groups;
+        GCS_HIP(hipMalloc(&m.ring_words, (RingComm::red_words(groups) +
+                                          RingComm::halo_words(groups, points)) *
+                                             sizeof(ll_word)));
+      } else if (m.hall > 0.0 &&
+                 hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                     &per_cu, k_mi_bicgstab_pair, kSolveThreads, 0) == hipSuccess &&
+                 per_cu * cus >= 2 * kCoopBlocks) {
+        GCS_HIP(hipMalloc(&m.coop_slots, 8 * kCoopBlocks * sizeof(double)));
+        GCS_HIP(hipMalloc(&m.coop_flags, 4 * sizeof(int)));
+      }
     }
     (void)hipGetLastError();
   }
@@ -2213,6 +2453,8 @@ void mi_destroy(Problem &P) {
   if (m->host_scal) (void)hipHostFree(m->host_scal);
   (void)hipFree(m->warm_scale);
   (void)hipFree(m->ring_words);
+  (void)hipFree(m->coop_slots);
+  (void)hipFree(m->coop_flags);
   delete m;
   P.mi = nullptr;
 }

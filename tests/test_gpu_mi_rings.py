@@ -50,3 +50,47 @@ def test_ring_solves_return_the_generated_potential(gpu, monkeypatch, nt, np_, h
     q = gpu.GpuProblem(cfg)
     single, _, _ = ws.solve_current(q, cur, np.zeros_like(pot), use_network=False)
     assert np.abs(single - got).max() <= 2 * TOL * scale
+
+
+# Colatitude points up to the most that one wavefront per ring can take (128
+# workgroups a hemisphere, two on 256 compute units), and one more.
+RING_LIMIT = 770
+
+
+@pytest.mark.parametrize("nt,np_", [(400, 9), (RING_LIMIT, 64), (RING_LIMIT + 1, 64)])
+@pytest.mark.parametrize("hall", [0.0, 5.0])
+def test_solves_of_many_rings(gpu, monkeypatch, nt, np_, hall):
+    """Reductions over more than 64 workgroups (67 and 128 a hemisphere), and
+    the Hall solve beyond the ring kernel's limit, which must still be spread
+    over the chip: several times faster an iteration than one workgroup per
+    hemisphere (by 8 and more when measured).
+
+    Tolerance: a residual of 1e-12 of the right-hand side bounds the error by
+    1e-12 times the ratio of the right-hand side to the potential, and that
+    grows with the longitude coupling of the ring next to the pole, 1 /
+    sin(theta)^2, as the square of the rings' number: TOL, which holds to 33
+    rings, times (nt / 33)^2."""
+    ws = importlib.import_module("gamera-cube_amd.warm_start")
+    cfg = gcs_config.earth_problem(16, 12, mi=True, hall_siemens=hall, mi_azimuth=np_,
+                                   mi_colatitude=nt)
+    cfg.mi.relative_tolerance = 1e-12
+    tol = TOL * (nt / 33) ** 2
+
+    def solve():
+        p = gpu.GpuProblem(cfg)
+        cur, pot = ws.make_pairs(p, seed=nt + np_, count=2, pedersen=cfg.mi.pedersen_siemens,
+                                 hall=hall)
+        got, its, ms = ws.solve_current(p, cur, np.zeros_like(pot), use_network=False)
+        scale = np.abs(pot).max()
+        err = np.abs(got - pot).max() / scale
+        print(f"  {nt} x {np_} hall {hall}: iterations {its}, {ms:.1f} ms, error {err:.1e}",
+              flush=True)
+        assert err <= tol
+        return got / scale, ms / max(its)
+
+    spread, spread_ms = solve()
+    monkeypatch.setenv("GCS_MI_COOPERATIVE", "0")
+    single, single_ms = solve()
+    assert np.abs(single - spread).max() <= 2 * tol
+    if hall > 0.0 and np_ == 64:
+        assert spread_ms < 0.5 * single_ms
