@@ -53,9 +53,10 @@ struct Bilinear {
   double wx, wy;
 };
 
-enum Slot {  // solver scalars per hemisphere
-  SL_RHS2, SL_FIRST, SL_TARGET, SL_RZ, SL_PAP, SL_NORM, SL_RHO, SL_DEN, SL_WNUM,
-  SL_WDEN, SL_ALPHA, SL_OMEGA, SL_RHOPREV, SL_POLE, SL_ITER, SL_OK, SL_COUNT = 16
+enum Slot {  // what a solve leaves per hemisphere
+  SL_ITER, SL_OK, SL_NORM, SL_FIRST,
+  SL_GAVE_UP,  // a workgroup of k_ring_cg or k_ring_bicgstab gave up a wait
+  SL_COUNT
 };
 
 }  // namespace
@@ -99,6 +100,7 @@ struct MiState {
   // not fit) and its workgroups per hemisphere
   unsigned long long *ring_words = nullptr;
   int ring_groups = 0;
+  int ring_spins = 0;  // polls after which its waits are given up
   // of the tensor solve by grid-wide barriers (null: not used): partial sums
   // and the per-hemisphere liveness exchange
   double *coop_slots = nullptr;
@@ -343,7 +345,8 @@ GCS_DEV TensorRow tensor_row(double sp, double hall, int i, double dt, double dp
 // Right-hand side (:428-448, weighted by sin theta), initial guess from the
 // previous potential (:449-464), and the diagonal (Pedersen, :322-344) or the
 // five-point tensor stencil (:777-833).
-// The exchange words of the register-resident solve are cleared here too.
+// The exchange words of the register-resident solve and its report of waits
+// given up are cleared here too.
 __global__ void k_mi_setup(MiK c, int tensor, double hall, unsigned long long *words,
                            long n_words) {
   const int h = blockIdx.y;
@@ -359,6 +362,7 @@ __global__ void k_mi_setup(MiK c, int tensor, double hall, unsigned long long *w
   const double *pot = c.potential + (long)h * c.nt * np;
   const double *fac = c.fac + (long)h * c.nt * np;
   if (q == 0) {
+    c.sl(h)[SL_GAVE_UP] = 0.0;
     rhs[0] = 0.0;
     double pole = 0.0;
     for (int j = 0; j < np; ++j) {
@@ -1201,9 +1205,12 @@ __global__ void __launch_bounds__(kSolveThreads) k_mi_bicgstab_pair(MiK c, doubl
 // The hemispheres are independent groups of workgroups. Every workgroup of a
 // hemisphere sums the same words in the same order and so takes the same
 // branches. All workgroups must be resident (a cooperative launch); a wait
-// ends after kSpinLimit polls at the latest, and a workgroup that gave up
-// leaves with the solve marked as failed, after which its neighbours' waits
-// end the same way.
+// ends after RingComm::spins polls at the latest, one at least (a loop that
+// may run none keeps what it loads live around it: 24 registers more, 3.95 ->
+// 4.58 ms on 2 x 128 x 256). A workgroup that gave one up says so in its
+// hemisphere's results (SL_GAVE_UP) and leaves, after which its neighbours'
+// waits end the same way; the host then has the system, which these kernels
+// leave as it was, solved without waits between workgroups.
 
 typedef unsigned long long ll_word;
 
@@ -1211,7 +1218,7 @@ constexpr int kRingWaves = 8;
 constexpr int kRingOwn = kRingWaves - 2;
 constexpr int kRingThreads = 64 * kRingWaves;
 constexpr int kRingSums = 7;         // most values of one reduction
-constexpr int kSpinLimit = 1 << 20;  // polls of a wait, about a second
+constexpr int kSpinLimit = 1 << 20;  // polls of a wait by default, about a second
 
 // Device buffers of the exchange, zeroed before each solve (the sequence
 // numbers of a solve start at 1): red [2 banks][2 hemispheres][groups]
@@ -1221,6 +1228,7 @@ constexpr int kSpinLimit = 1 << 20;  // polls of a wait, about a second
 struct RingComm {
   ll_word *red, *halo;
   int groups, points;
+  int spins;  // polls of a wait (one at least)
   static size_t red_words(int groups) { return 2UL * 2 * groups * kRingSums * 2; }
   static size_t halo_words(int groups, int points) {
     return 2UL * 2 * groups * 2 * points * 2 * 64;
@@ -1345,7 +1353,8 @@ struct RingWave {
   GCS_DEV void receive(double v[KP]) {
     if (!ghost) return;
     const ll_word *s = halo_slot(g, w == 0 ? 0 : 1);
-    for (int spin = 0; spin < kSpinLimit; ++spin) {
+    int spin = 0;
+    do {
       ll_word a[KP], b[KP];
       bool ok = true;
 #pragma unroll
@@ -1363,7 +1372,7 @@ struct RingWave {
           if (t < cnt) v[t] = ll_value(a[t], b[t]);
         return;
       }
-    }
+    } while (++spin < comm.spins);
     *gave_up = 1;
   }
 
@@ -1393,7 +1402,8 @@ struct RingWave {
       for (int q = lane; q < (groups + 63) / 64 * 64; q += 64) {
         const ll_word *slot = bank + (long)min(q, groups - 1) * (kRingSums * 2);
         int spin = 0;
-        for (; spin < kSpinLimit; ++spin) {
+        bool here = false;
+        do {
           ll_word a[NV], b[NV];
           bool ok = true;
 #pragma unroll
@@ -1404,14 +1414,14 @@ struct RingWave {
 #pragma unroll
           for (int n = 0; n < NV; ++n)
             ok = ok && (unsigned)a[n] == seq && (unsigned)b[n] == seq;
-          if (__all(ok)) {
+          here = __all(ok);
+          if (here) {
 #pragma unroll
             for (int n = 0; n < NV; ++n)
               if (q < groups) acc[n] += ll_value(a[n], b[n]);
-            break;
           }
-        }
-        got = got && spin < kSpinLimit;
+        } while (!here && ++spin < comm.spins);
+        got = got && here;
       }
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
@@ -1428,6 +1438,13 @@ struct RingWave {
 #pragma unroll
     for (int n = 0; n < NV; ++n) v[n] = total[n];
     dead = dead || total[kRingSums] != 0.0;
+  }
+
+  // At the end: whether a wait was given up, in the hemisphere's results (the
+  // same value from every workgroup that says so).
+  GCS_DEV void report(const MiK &c) const {
+    __syncthreads();
+    if (threadIdx.x == 0 && *gave_up != 0) c.sl(h)[SL_GAVE_UP] = 1.0;
   }
 
   // Put v into this wavefront's LDS row, for the neighbour rings.
@@ -1661,9 +1678,9 @@ __global__ void __launch_bounds__(kRingThreads) k_ring_cg(MiK c, RingComm comm, 
     r0 -= alpha * s0;
     restart = false;
   }
-  res.ok = res.ok && !s.dead;
   ring_store<KP>(s, c, x, x0);
   if (s.g == 0) store_result(c, s.h, res, first);
+  s.report(c);
 }
 
 // Factors of the ring preconditioner (ring_factor) that a lane applies.
@@ -1943,9 +1960,9 @@ __global__ void __launch_bounds__(kRingThreads) k_ring_bicgstab(MiK c, RingComm 
     rho_prev = rho;
     rho = v2[1];
   }
-  res.ok = res.ok && !s.dead;
   ring_store<KP>(s, c, x, x0);
   if (s.g == 0) store_result(c, s.h, res, first);
+  s.report(c);
 }
 
 // The kernels by points per lane, 1 .. kRingChunk.
@@ -2170,7 +2187,7 @@ int solve(Problem &P, bool tensor) {
   const auto t0 = std::chrono::steady_clock::now();
   const dim3 g2(blocks_of(m.n), 2);
   const int points = (m.np + 63) / 64;
-  RingComm comm{m.ring_words, nullptr, m.ring_groups, points};
+  RingComm comm{m.ring_words, nullptr, m.ring_groups, points, m.ring_spins};
   const long red = (long)RingComm::red_words(m.ring_groups);
   const long words =
       comm.red != nullptr ? red + (long)RingComm::halo_words(m.ring_groups, points) : 0;
@@ -2185,6 +2202,22 @@ int solve(Problem &P, bool tensor) {
     (void)hipGetLastError();
     return false;
   };
+  auto single_workgroups = [&]() {
+    if (tensor)
+      k_mi_bicgstab<<<2, kSolveThreads, 0, s>>>(c, rel, maxit);
+    else
+      k_mi_cg<<<2, kSolveThreads, 4 * (size_t)m.nt * sizeof(double), s>>>(c, rel, maxit);
+  };
+  auto expand = [&]() {
+    k_mi_vec<<<dim3(blocks_of((long)m.np * m.nt), 2), kT, 0, s>>>(c, OP_EXPAND, 0.0, m.active);
+  };
+  auto results = [&]() -> int {
+    GCS_HIP(hipGetLastError());
+    GCS_HIP(hipMemcpyAsync(m.host_scal, m.scal, 2 * SL_COUNT * sizeof(double),
+                           hipMemcpyDeviceToHost, s));
+    GCS_HIP(hipStreamSynchronize(s));
+    return 0;
+  };
   bool resident = comm.red != nullptr;
   if (resident) {
     if (tensor) k_ring_factor<<<dim3(m.nt - 2, 2), 64, 0, s>>>(c);
@@ -2197,16 +2230,17 @@ int solve(Problem &P, bool tensor) {
     const bool pair = tensor && m.coop_slots != nullptr &&
                       cooperative((const void *)k_mi_bicgstab_pair, 2 * kCoopBlocks,
                                   kSolveThreads, args);
-    if (!pair && tensor)
-      k_mi_bicgstab<<<2, kSolveThreads, 0, s>>>(c, rel, maxit);
-    else if (!pair)
-      k_mi_cg<<<2, kSolveThreads, 4 * (size_t)m.nt * sizeof(double), s>>>(c, rel, maxit);
-    k_mi_vec<<<dim3(blocks_of((long)m.np * m.nt), 2), kT, 0, s>>>(c, OP_EXPAND, 0.0, m.active);
+    if (!pair) single_workgroups();
+    expand();
   }
-  GCS_HIP(hipGetLastError());
-  GCS_HIP(hipMemcpyAsync(m.host_scal, m.scal, 2 * SL_COUNT * sizeof(double),
-                         hipMemcpyDeviceToHost, s));
-  GCS_HIP(hipStreamSynchronize(s));
+  if (results() != 0) return -1;
+  if (resident && (m.host_scal[SL_GAVE_UP] != 0.0 || m.host_scal[SL_COUNT + SL_GAVE_UP] != 0.0)) {
+    // a wait of the register-resident solve was given up (a workgroup did not
+    // run for about a second): the same system with no such waits
+    single_workgroups();
+    expand();
+    if (results() != 0) return -1;
+  }
   m.solve_ms = std::chrono::duration<double, std::milli>(
                    std::chrono::steady_clock::now() - t0).count();
   bool ok = true;
@@ -2395,6 +2429,10 @@ int mi_create(Problem &P) {
             hipSuccess &&
         coop != 0) {
       if ((long)per_cu * cus >= 2L * groups) {
+        // GCS_MI_SPIN_LIMIT is for tests of the solve after a wait that was
+        // given up
+        const char *spins = std::getenv("GCS_MI_SPIN_LIMIT");
+        m.ring_spins = spins != nullptr ? std::atoi(spins) : kSpinLimit;
         m.ring_groups = groups;
         GCS_HIP(hipMalloc(&m.ring_words, (RingComm::red_words(groups) +
                                           RingComm::halo_words(groups, points)) *

@@ -94,3 +94,34 @@ def test_solves_of_many_rings(gpu, monkeypatch, nt, np_, hall):
     assert np.abs(single - spread).max() <= 2 * tol
     if hall > 0.0 and np_ == 64:
         assert spread_ms < 0.5 * single_ms
+
+
+@pytest.mark.parametrize("hall", [0.0, 5.0])
+@pytest.mark.parametrize("polls", [1, 50])
+def test_solve_after_a_wait_that_was_given_up(gpu, monkeypatch, polls, hall):
+    """A wait between workgroups that runs out of its polls (GCS_MI_SPIN_LIMIT,
+    read when a problem is made) must not end the solve: one workgroup per
+    hemisphere solves the system. One poll never suffices for all six
+    workgroups of each of a hundred iterations, so there the bits are those of
+    that solve asked first; 50 may or may not."""
+    ws = importlib.import_module("gamera-cube_amd.warm_start")
+    cfg = gcs_config.earth_problem(16, 12, mi=True, hall_siemens=hall, mi_azimuth=65,
+                                   mi_colatitude=33)
+    cfg.mi.relative_tolerance = 1e-12
+    monkeypatch.setenv("GCS_MI_COOPERATIVE", "0")
+    p = gpu.GpuProblem(cfg)
+    cur, pot = ws.make_pairs(p, seed=3, count=2, pedersen=cfg.mi.pedersen_siemens, hall=hall)
+    guess = 0.5 * pot
+    single, its, _ = ws.solve_current(p, cur, guess, use_network=False)
+    monkeypatch.delenv("GCS_MI_COOPERATIVE")
+    monkeypatch.setenv("GCS_MI_SPIN_LIMIT", str(polls))
+    q = gpu.GpuProblem(cfg)
+    scale = np.abs(pot).max()
+    for _ in range(2):
+        got, got_its, _ = ws.solve_current(q, cur, guess, use_network=False)
+        if polls == 1:
+            assert got_its == its and np.array_equal(got, single)
+        assert np.abs(got - pot).max() <= TOL * scale
+    # and in a coupled run
+    q.advance(2)
+    assert q.mi_report()["ready"] and np.isfinite(q.mi_field(0)).all()
