@@ -169,22 +169,51 @@ void parallel_copy(void *dst, const void *src, size_t bytes, size_t block = 1UL 
 
 }  // namespace
 
+namespace {
+
+// One plane at a time through a pageable copy: slow, and needs no device or
+// pinned memory.
+int planes_to_arrays_direct(Problem &P, int first, int ncomp, int face, int faces,
+                            const size_t ext[3], HostArray *const out[]) {
+  const Layout &L = P.L;
+  std::vector<double> buf(L.face_stride);
+  for (int f = 0; f < faces; ++f) {
+    for (int c = 0; c < ncomp; ++c) {
+      GCS_HIP(hipMemcpy(buf.data(), P.plane(first + c) + (face + f) * L.face_stride,
+                        L.face_stride * sizeof(double), hipMemcpyDeviceToHost));
+      double *to = out[f]->data + c;
+      for (size_t i = 0; i < ext[0]; ++i)
+        for (size_t j = 0; j < ext[1]; ++j)
+          for (size_t k = 0; k < ext[2]; ++k, to += ncomp) *to = buf[(i * L.SJ + j) * L.SK + k];
+    }
+    out[f]->valid = true;
+  }
+  return 0;
+}
+
+}  // namespace
+
 // The planes are interleaved on the device and cross PCIe in two alternating
 // pinned chunks, each copied out by the host threads while the next one
 // arrives. What bounds it is PCIe and the host's memory (6 x 96^2 x 192, U, B
 // and face flux, 1.25 GB: 30 ms, 42 GB/s; a pageable copy per plane and one
-// host thread that scattered it took 228 ms).
+// host thread that scattered it took 228 ms). A device with no room for the
+// interleaved array, or a host without pinned memory, takes the direct way.
 int planes_to_arrays(Problem &P, int first, int ncomp, int face, int faces,
                      const size_t ext[3], HostArray *const out[]) {
   const size_t per = ext[0] * ext[1] * ext[2] * (size_t)ncomp, total = per * faces;
   for (int f = 0; f < faces; ++f)
     if (size_array(*out[f], per) != 0) return -1;
-  if (pack_planes(P, first, ncomp, face, faces, ext) != 0) return -1;
   const size_t chunk = std::min<size_t>(total, 1UL << 20);  // doubles
   double *buf = pinned(P, 2 * chunk);
-  if (buf == nullptr) return -1;
+  bool staged = buf != nullptr;
   for (hipEvent_t &e : P.copied)
-    if (e == nullptr) GCS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (staged && e == nullptr)
+      staged = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+  if (!staged || pack_planes(P, first, ncomp, face, faces, ext) != 0) {
+    (void)hipGetLastError();
+    return planes_to_arrays_direct(P, first, ncomp, face, faces, ext, out);
+  }
   const size_t chunks = (total + chunk - 1) / chunk;
   auto request = [&](size_t q) -> int {
     const size_t at = q * chunk, n = std::min(chunk, total - at);
