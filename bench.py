@@ -58,7 +58,7 @@ STAGE_MODEL = {
 # The FP64 kernel of each modelled stage (rocprofv3's names, templates kept).
 STAGE_KERNEL = {
     "face_flux_i": "k_face_flux_tiled<0, 8, 16>", "face_flux_j": "k_face_flux_tiled<1, 8, 16>",
-    "face_flux_k": "k_face_flux", "edge_emf_i": "k_edge_emf_tiled<0>",
+    "face_flux_k": "k_face_flux_rows", "edge_emf_i": "k_edge_emf_tiled<0>",
     "edge_emf_j": "k_edge_emf_tiled<1>", "edge_emf_k": "k_edge_emf",
     "update": "k_update<false>", "predict": "k_predict<false>",
 }

@@ -239,13 +239,17 @@ struct Problem {
   uint8_t *byte_plane(int q) const { return bytes + (long)q * L.total; }
 };
 
-// Stages of one step, in launch order (names for timing reports).
+// Stages of one step, in launch order (names for timing reports): one per
+// launch, but for the ghost recovery and the i-face velocities. The sweeps of
+// the face fluxes and edge EMFs are S_FACE_FLUX0 .. 2 and S_EDGE_EMF0 .. 2 in
+// FP64, S_FACE_FLUX and S_EDGE_EMF in the mixed form (three directions to a
+// launch), S_SWEEPS and S_SWEEPS_END on small grids.
 enum Stage {
-  S_CFL, S_DT, S_SYNC_PHI, S_HALO_CELLS, S_OUTFLOW, S_HALO_FACES,
-  S_EARTH_CELLS, S_EARTH_FACES, S_EARTH_RECOVER, S_PREDICT, S_FACE_FLUX0,
-  S_FACE_FLUX1, S_FACE_FLUX2, S_SYNC_FLUX, S_INNER_TRAP, S_FACE_VELOCITY,
-  S_EDGE_EMF0, S_EDGE_EMF1, S_EDGE_EMF2, S_EARTH_EMF, S_SYNC_EDGES, S_UPDATE,
-  S_FINAL_SYNC, S_SEAM_RECOVER, S_FIDELITY, S_CLOCK, S_END, S_MI, kStages
+  S_CFL, S_GHOST_FILL, S_EARTH_GHOSTS, S_EARTH_RECOVER, S_PREDICT, S_FACE_FLUX0,
+  S_FACE_FLUX1, S_FACE_FLUX2, S_FACE_FLUX, S_FINISH_FLUX, S_FACE_VELOCITY,
+  S_EDGE_EMF0, S_EDGE_EMF1, S_EDGE_EMF2, S_EDGE_EMF, S_SWEEPS, S_SWEEPS_END,
+  S_EARTH_EMF, S_SYNC_EDGES, S_UPDATE, S_FINISH_STEP, S_SEAM_RECOVER, S_END, S_MI,
+  kStages
 };
 const char *stage_name(int stage);
 // Record a stage boundary on the problem's stream when profiling.

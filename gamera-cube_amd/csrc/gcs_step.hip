@@ -2630,11 +2630,11 @@ int launch_recover_all(Problem &P, int phi_first, int b_first) {
 
 const char *stage_name(int stage) {
   static const char *names[kStages] = {
-      "cfl", "dt", "sync_phi", "halo_cells", "radial_outflow", "halo_faces",
-      "earth_cells", "earth_faces", "earth_recover", "predict", "face_flux_i",
-      "face_flux_j", "face_flux_k", "sync_flux", "inner_trap", "face_velocity",
-      "edge_emf_i", "edge_emf_j", "edge_emf_k", "earth_emf", "sync_edges",
-      "update", "final_sync", "seam_recover", "fidelity", "clock", "end", "mi_update"};
+      "cfl", "ghost_fill", "earth_ghosts", "earth_recover", "predict", "face_flux_i",
+      "face_flux_j", "face_flux_k", "face_flux", "finish_flux", "face_velocity",
+      "edge_emf_i", "edge_emf_j", "edge_emf_k", "edge_emf", "sweeps", "sweeps_end",
+      "earth_emf", "sync_edges", "update", "finish_step", "seam_recover", "end",
+      "mi_update"};
   return stage >= 0 && stage < kStages ? names[stage] : "?";
 }
 
@@ -2671,10 +2671,12 @@ static void launch_sweeps(Problem &P, const K &c) {
     g.blocks[q] = (g.real[q] + 7) / 8 * 8;
     blocks += g.blocks[q];
   }
+  mark_stage(P, S_SWEEPS);
   k_sweeps<<<blocks, kSweepThreads, 0, P.stream>>>(c, g);
   const unsigned flux = nblocks(P.n_seams, 128);
   const unsigned trap = P.bnd.inner_trap ? nblocks(6L * L.n * L.n, 128) : 0u;
   const unsigned edges = nblocks(6L * (L.nr + 1) * (L.n + 1) * L.n, 128);
+  mark_stage(P, S_SWEEPS_END);
   k_sweeps_end<<<flux + trap + edges, 128, 0, P.stream>>>(c, P.seams, P.n_seams, flux, trap);
 }
 
@@ -2703,8 +2705,8 @@ int enqueue_phase(Problem &P, Phase phase, bool driver, bool whole) {
   const StepBoundary &bd = P.bnd;
   // Fluxes and EMF sweeps in joint launches (launch_sweeps): whole steps of
   // small FP64 grids.
-  const bool joint = whole && !P.mixed && !P.plain && !P.profiling && P.opt.mhd &&
-                     n_active <= kJointCells;
+  const bool joint =
+      whole && !P.mixed && !P.plain && P.opt.mhd && n_active <= kJointCells;
 
   if (phase == PHASE_GHOSTS) {
     // cubedsphere_step.c:51-65
@@ -2732,16 +2734,14 @@ int enqueue_phase(Problem &P, Phase phase, bool driver, bool whole) {
     }
     g.seam_blocks = nblocks(g.n_seams, kGhostThreads);
     g.cell_blocks = nblocks(g.n_cells, kGhostThreads);
-    mark_stage(P, S_HALO_CELLS);
+    mark_stage(P, S_GHOST_FILL);
     k_ghost_fill<<<(g.partial != nullptr ? 1u : 0u) + g.seam_blocks + g.cell_blocks +
                        nblocks(g.n_faces, kGhostThreads),
                    kGhostThreads, 0, s>>>(c, g);
-    if (bd.outflow) {
-      mark_stage(P, S_OUTFLOW);
+    if (bd.outflow)
       k_radial_outflow<<<nblocks(6L * 2 * L.ghost * L.NJ * L.NK, T), T, 0, s>>>(c);
-    }
     if (bd.earth_cells) {
-      mark_stage(P, S_EARTH_CELLS);
+      mark_stage(P, S_EARTH_GHOSTS);
       EarthWork e;
       unsigned blocks = nblocks(6L * 2 * L.ghost * L.NJ * L.NK, T);
       for (int d = 0; d < 3; ++d) {
@@ -2751,13 +2751,13 @@ int enqueue_phase(Problem &P, Phase phase, bool driver, bool whole) {
         blocks += e.face_blocks[d];
       }
       k_earth_ghosts<<<blocks, T, 0, s>>>(c, w, e);
-      mark_stage(P, S_EARTH_RECOVER);
       // cubedsphere_earth_boundary.c:169 recovers every cell of both levels.
       // After a completed step the six face fluxes of an active cell are
       // those its B was last recovered from (the step ends with the seam
       // sync and a recovery), so only the non-active cells change; and
       // ghost-cell B is never read by the step (see halo_cell), so with
       // fidelity 0 only the first step's recovery of every cell runs.
+      if (!P.b_recovered || P.fidelity) mark_stage(P, S_EARTH_RECOVER);
       if (!P.b_recovered) {
         for (int lev : {c.cur, c.old})
           k_recover<<<nblocks(n_cells, T), T, 0, s>>>(c, plane_phi(lev, 0), plane_b(lev, 0), 1,
@@ -2780,7 +2780,7 @@ int enqueue_phase(Problem &P, Phase phase, bool driver, bool whole) {
     if (P.mixed) {
       // The FP32 kernels read half the bytes and are faster without tiles;
       // the three directions share a launch (blockIdx.y).
-      mark_stage(P, S_FACE_FLUX0);
+      mark_stage(P, S_FACE_FLUX);
       k_face_flux_fp32<<<dim3(nblocks(n_faces, 128), 3), 128, 0, s>>>(c);
     }
     for (int d = 0; d < (P.mixed ? 0 : 3); ++d) {
@@ -2800,7 +2800,7 @@ int enqueue_phase(Problem &P, Phase phase, bool driver, bool whole) {
       else
         k_face_flux<<<nblocks(n, 128), 128, 0, s>>>(c, d);
     }
-    mark_stage(P, S_SYNC_FLUX);
+    mark_stage(P, S_FINISH_FLUX);
     const unsigned trap_from = nblocks(P.n_seams, T);
     const unsigned blocks = trap_from + (bd.inner_trap ? nblocks(6L * L.n * L.n, T) : 0u);
     if (P.mixed)
@@ -2822,7 +2822,7 @@ int enqueue_phase(Problem &P, Phase phase, bool driver, bool whole) {
       long n = n_velocity[1];
       if (P.plain) n = std::max(n, n_velocity[0]);
       k_face_velocity_fp32<<<dim3(nblocks(n, T), 3 - first), T, 0, s>>>(c, first);
-      mark_stage(P, S_EDGE_EMF0);
+      mark_stage(P, S_EDGE_EMF);
       k_edge_emf_fp32<<<dim3(nblocks(n_edges, 128), 3), 128, 0, s>>>(c);
     } else {
       // FP64: the i-face velocities for the k-edges only; the j- and i-edges
@@ -2871,7 +2871,7 @@ int enqueue_phase(Problem &P, Phase phase, bool driver, bool whole) {
     n.old = c.cur;
     const unsigned sync_blocks = P.opt.mhd ? nblocks(P.n_seams, T) : 0u;
     const unsigned finish = sync_blocks + (P.fidelity ? nblocks(n_box, T) : 0u);
-    mark_stage(P, S_FINAL_SYNC);
+    mark_stage(P, S_FINISH_STEP);
     if (finish > 0 || driver)
       k_finish_step<<<std::max(finish, 1u), T, 0, s>>>(c, P.seams, P.opt.mhd ? P.n_seams : 0,
                                                        P.fidelity ? sync_blocks
