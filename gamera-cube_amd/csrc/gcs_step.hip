@@ -862,16 +862,12 @@ GCS_DEV bool recover_at(const K &c, long at, int phi_level_plane,
 // Recover every cell of a level (nonorthogonal_step.c:310-359); with
 // inner_copy the cells inside the wall take the first shell's value
 // (cubedsphere_earth_boundary.c:235-245).
-__global__ void k_recover(K c, int phi_plane, int b_plane, int inner_copy,
-                          int ghost_only) {
+__global__ void k_recover(K c, int phi_plane, int b_plane, int inner_copy) {
   const Layout &L = c.L;
   const int lo[3] = {0, 0, 0};
   const int hi[3] = {L.NI, L.NJ, L.NK};
   int f, i, j, k;
   if (!box(tid(), lo, hi, f, i, j, k)) return;
-  if (ghost_only && i >= L.ghost && i < L.ghost + L.nr && j >= L.ghost &&
-      j < L.ghost + L.n && k >= L.ghost && k < L.ghost + L.n)
-    return;
   const long at = L.at(f, i, j, k);
   double b[3];
   if (!recover_at(c, at, phi_plane, b)) {
@@ -2623,7 +2619,7 @@ int launch_recover_all(Problem &P, int phi_first, int b_first) {
   K c = make_k(P);
   const Layout &L = P.L;
   const long n = 6L * L.NI * L.NJ * L.NK;
-  k_recover<<<nblocks(n, 256), 256, 0, P.stream>>>(c, phi_first, b_first, 0, 0);
+  k_recover<<<nblocks(n, 256), 256, 0, P.stream>>>(c, phi_first, b_first, 0);
   GCS_HIP(hipGetLastError());
   return 0;
 }
@@ -2760,8 +2756,7 @@ int enqueue_phase(Problem &P, Phase phase, bool driver, bool whole) {
       if (!P.b_recovered || P.fidelity) mark_stage(P, S_EARTH_RECOVER);
       if (!P.b_recovered) {
         for (int lev : {c.cur, c.old})
-          k_recover<<<nblocks(n_cells, T), T, 0, s>>>(c, plane_phi(lev, 0), plane_b(lev, 0), 1,
-                                                      0);
+          k_recover<<<nblocks(n_cells, T), T, 0, s>>>(c, plane_phi(lev, 0), plane_b(lev, 0), 1);
       } else if (P.fidelity) {
         k_recover_ghosts<<<dim3(nblocks(n_cells - n_active, T), 2), T, 0, s>>>(c, 1);
       }
