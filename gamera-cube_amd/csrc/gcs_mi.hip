@@ -967,9 +967,9 @@ __global__ void __launch_bounds__(kSolveThreads) k_mi_bicgstab(MiK c, double rel
 // k_mi_bicgstab, with grid-wide barriers where one workgroup's barrier
 // sufficed there). What bounds it is its ten barriers an iteration and, on
 // large grids, the vectors' traffic through L2. 2 x 800 x 256 points, 3,400 -
-// 3,900 iterations: 908 ms (k_mi_bicgstab: 9,221); 2 x 771 x 64: 403 ms
+// 3,900 iterations: 900 ms (k_mi_bicgstab: 9,221); 2 x 771 x 64: 400 ms
 // (3,219). Below that limit k_ring_bicgstab is the faster one: 2 x 770 x 64,
-// 42 against 384 ms; 2 x 128 x 256, 4.0 against 45. Dot products sum the
+// 43 against 384 ms; 2 x 128 x 256, 4.0 against 45. Dot products sum the
 // workgroups' partial sums in workgroup order from two alternating slot
 // banks (a bank is rewritten only after every workgroup passed the barrier
 // that follows its last read), so every workgroup of a hemisphere computes
@@ -1181,26 +1181,34 @@ __global__ void __launch_bounds__(kSolveThreads) k_mi_bicgstab_pair(MiK c, doubl
 
 // ---- register-resident solves: one wavefront per colatitude ring ------------------
 //
-// The iterations of k_mi_cg and k_mi_bicgstab with every solver vector held
-// in registers: a wavefront owns one ring, a lane kRingPoints = ceil(np / 64)
+// The iterations of k_mi_cg and k_mi_bicgstab with the solver vectors held in
+// registers: a wavefront owns one ring, a lane kRingPoints = ceil(np / 64)
 // consecutive points of it, and a workgroup kRingOwn rings plus a ghost copy
 // of the ring on each side. Neighbour rings inside a workgroup meet in LDS.
 // A ghost wavefront runs the same vector updates as the ring's owner (so its
 // values are the owner's, bit for bit) and receives from it only the product
 // A p that it cannot form itself. Workgroups exchange two things, both as
-// self-validating words (32 bits of a double and a 32-bit sequence number
-// in one 64-bit atomic): the partial sums of the dot products, and those
+// words of the LL protocol of the collective libraries (32 bits of a double
+// and a 32-bit sequence number in one 64-bit store, so that a word that has
+// arrived says so itself): the partial sums of the dot products, and those
 // boundary rings, which are sent before a reduction and read after it, so
 // that their way is hidden behind the reduction's. A reduction is therefore
 // the only wait: one per CG iteration, two per BiCGStab iteration, where a
 // grid barrier per dot product and per vector took ten. What bounds an
 // iteration is the latency of these reductions and of the ring solve's two
-// wavefront-wide prefixes; nothing in it is limited by bandwidth or issue.
-// Measured on 2 x 128 x 256 points: BiCGStab 9.4 us an iteration and 4.6 ms a
-// solve (two grid barriers of cooperative groups per step of the method, all
-// vectors in memory: 115 us, 48 ms), CG 4.0 us and 4.0 ms (one workgroup per
-// hemisphere: 88 us, 83 ms); on 2 x 33 x 57, 7.5 us and 0.9 ms (75 us, 8.9
-// ms). Putting a hemisphere's workgroups on one XCD changed nothing (3 %).
+// wavefront-wide prefixes, as long as the vectors fit: a lane has 256
+// registers (512 threads a workgroup). CG's fit up to 512 points a ring
+// (255), BiCGStab's nine vectors and factors up to 256 (235); at 5, 6, 7 and
+// 8 points a lane 32, 86, 127 and 231 registers are spilled to scratch memory.
+// Measured, solves from zero on 2 x 128 rings (ms; in brackets BiCGStab with
+// grid-wide barriers, CG on one workgroup per hemisphere, vectors in memory):
+//   points a ring      256          320          384          448         512
+//   BiCGStab      4.0 (45)     4.7 (46)     5.8 (50)     8.4 (53)   12.6 (56)
+//   CG            3.6 (81)    4.6 (117)    6.1 (169)   10.0 (308)  14.9 (494)
+// that is 9.5 us a BiCGStab iteration at 256 points (100) and 28 at 512 (135),
+// 3.9 us (87) and 5.2 (171) of CG; on 2 x 33 x 57, 7.7 us and 0.85 ms, 3.3 us
+// and 0.63 ms. Putting a hemisphere's workgroups on one XCD changed nothing
+// (3 %).
 //
 // The hemispheres are independent groups of workgroups. Every workgroup of a
 // hemisphere sums the same words in the same order and so takes the same

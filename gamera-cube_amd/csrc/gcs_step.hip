@@ -449,7 +449,7 @@ GCS_DEV void halo_face(const K &c, const HaloFace *e, int n, int both, long t) {
 // take active cells' U and B, the averages change active faces only, and the
 // times and ratio that the dt rule sets are read from the next launch on.
 // On small grids a launch costs its latency, several us, whatever it does
-// (16 x 12^2: a step's 33 launches took 236 us, its 12 take 105; see
+// (16 x 12^2: a step's 33 launches took 236 us, its 11 take 104; see
 // enqueue_phase).
 struct GhostWork {
   const SeamPair *seams;
@@ -2644,9 +2644,11 @@ void mark_stage(Problem &P, int stage) {
 
 // Launch the FP64 sweeps of a small grid, fluxes and EMFs, in two launches
 // (k_sweeps, k_sweeps_end). The line lies where the separate launches, each
-// with its own registers and LDS, catch up (us a step, separate / joint, graph
-// launches): 14 k cells 149 / 95, 166 k 322 / 273, 393 k 509 / 449, 911 k 989
-// / 960, 1.33 M 1286 / 1295.
+// with its own registers and LDS, catch up, launched one by one and as graphs
+// alike (us a step, separate / joint, without ghost upkeep):
+//   cells         14 k       166 k       393 k       911 k        1.33 M
+//   one by one    143 / 89   316 / 267   502 / 443   984 / 956   1281 / 1290
+//   graph         147 / 94   320 / 271   508 / 449   988 / 962   1288 / 1295
 constexpr long kJointCells = 1000000;
 
 static void launch_sweeps(Problem &P, const K &c) {
@@ -2678,8 +2680,8 @@ static void launch_sweeps(Problem &P, const K &c) {
 
 // Kernels that need nothing of each other share a launch: on small grids a
 // step is the sum of its launches' latencies, 5-13 us each (16 x 12^2 cells a
-// face, default options: 33 launches 236 us a step, 12 launches 105; 48 x
-// 24^2: 462, 331).
+// face, default options: 33 launches 236 us a step, 11 launches 104; 48 x
+// 24^2: 462, 329).
 int enqueue_phase(Problem &P, Phase phase, bool driver, bool whole) {
   K c = make_k(P);
   const Layout &L = P.L;

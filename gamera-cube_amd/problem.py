@@ -119,7 +119,11 @@ class Problem:
                 "steps": int(out[3])}
 
     def field(self, face, field_id):
-        """Zero-copy numpy view of one face's array (host memory)."""
+        """Zero-copy numpy view of one face's array (host memory), for use
+        until the next step. The GPU library keeps the memory of the state's
+        arrays: the first request for a field after a step writes the new
+        state into the view (on small grids into those of all six faces), so
+        copy what a later frame is compared with."""
         ptr = ctypes.POINTER(ctypes.c_double)()
         count = ctypes.c_size_t()
         if self._api["field"](self._handle, face, field_id, ctypes.byref(ptr),

@@ -51,7 +51,11 @@ int gcs_problem_step_explicit(gcs_problem *problem, double predictor_ratio,
 void gcs_problem_clock(gcs_problem *problem, double out[4]);
 
 /* Host copy of field `field` (GCS_FIELD_*) of cube face `face`, in the
- * reference's array-of-structs layout; valid until the next step. */
+ * reference's array-of-structs layout; valid until the next step. The
+ * memory of the state's arrays (ids below GCS_FIELD_VERTEX) stays where it is
+ * and is written again by the first request for the field after a step,
+ * for all six faces at once where they are small: copy what is to be
+ * compared with a later frame. */
 int gcs_problem_field(gcs_problem *problem, int face, int field,
                       double **data, size_t *count);
 int gcs_problem_edge_valid(gcs_problem *problem, int face, int direction,
